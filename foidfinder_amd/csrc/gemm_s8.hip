@@ -12,7 +12,7 @@
 // rows through LDS for 16-byte stores. K slices sit in LDS with their 16-byte chunks XOR-swizzled by row bits
 // (conflict-free 16-byte fragment reads). The variant (the engine autotunes it per GEMM and batch size):
 //
-//  * 1, gemm_s8_kernel<128, 128>: 128 x 128 tiles, 4 waves, register-staged double buffering (small M).
+//  * 1, gemm_s8_pair_kernel: 128 x 128 tiles, 8 waves in two K groups, a 4-slot ring per group (small M).
 //  * 2, gemm_s8_ring_kernel: 256 x 128 tiles, 4 waves, a 3-slot ring of K-64 slices filled by buffer loads straight
 //    into LDS, two workgroups per CU.
 //  * 3, gemm_s8_wide_kernel: 256 x 256 tiles, 8 waves (2 per SIMD), one workgroup per CU, a 2-slot ring of K-128
@@ -47,8 +47,6 @@ struct GemmArgs {
   float q_scale;
 };
 
-constexpr int BK = 64;
-
 constexpr uint32_t RSRC_WORD3 = 0x00020000;  // buffer descriptor word 3: raw dword access (gfx9 family)
 
 // Raw buffer loads and stores through a descriptor over [base, base + nbytes): an access past the range reads zeros
@@ -76,13 +74,6 @@ __device__ __forceinline__ void buf_store_h8(half8_t v, void* base, int nbytes, 
   const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, nbytes, RSRC_WORD3);
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(int4_t, v), r, voff, 0, 0);
 }
-
-// LDS rows of 64 bytes (4 chunks of 16 B); chunk index XOR-swizzled with bits 2-3 of the row. gfx950 serves a
-// 16-byte-per-lane LDS read 16 lanes at a time from 64 four-byte banks (256 B), so the 16 rows read by 16 consecutive
-// lanes must land in 16 distinct 16-byte slots of a 256-byte window: rows r..r+3 fill one window's 4 slots each, and
-// the XOR with (r >> 2) & 3 spreads r, r+4, r+8, r+12 over the 4 chunk positions (measured: zero bank conflicts,
-// where XOR with bits 1-2 doubles every read).
-__device__ __forceinline__ int swz(int row, int chunk) { return row * BK + ((chunk ^ ((row >> 2) & 3)) << 4); }
 
 // silu(g) = g / (1 + e^-g) from the hardware transcendental units: e^-g = v_exp_f32(-g log2 e) and the quotient as
 // g * v_rcp_f32(1 + e^-g), each about 1 ulp, so silu(g) * value lands within one fp16 ulp of the correctly rounded
@@ -129,10 +120,28 @@ constexpr int stage_bytes() {
 // in that order, 1 KB each.
 constexpr int META_BYTES = 3 * 1024;
 
-template <int EPI, int NI, int MI>
+// The residual segments of rows 0-31 of a wave's tile, as the RESIDUAL epilogue's store phase adds them.
+template <int NI>
+__device__ __forceinline__ void load_residual_rows(half8_t (&x)[NI * 2], int m_base, int n_base, int lane,
+                                                   const GemmArgs& args) {
+  constexpr int LANES_PER_ROW = NI * 4, ROWS_PER_PASS = 64 / LANES_PER_ROW;
+  const int ld = args.N, n = n_base + (lane % LANES_PER_ROW) * 8;
+  const half_t* base = static_cast<const half_t*>(args.out) + static_cast<int64_t>(m_base) * ld;
+  const int bytes = buf_bytes(static_cast<int64_t>(args.M - m_base) * ld * 2);
+#pragma unroll
+  for (int p = 0; p < 32 / ROWS_PER_PASS; ++p) {
+    const int r = p * ROWS_PER_PASS + lane / LANES_PER_ROW;
+    x[p] = buf_load_h8(base, bytes, n < ld ? static_cast<uint32_t>(r * ld + n) * 2 : OOB_OFFSET);
+  }
+}
+
+// LDS_META: `meta` holds the tile's metadata (the wave's tile starts at row row0 and column col0 of it), otherwise
+// scales and biases come from global memory. PRE: `pre` holds the first 32 rows' residual segments
+// (load_residual_rows).
+template <int EPI, int NI, int MI, bool LDS_META = false, bool PRE = false>
 __device__ __forceinline__ void store_epilogue(const int16_t_v (&acc)[NI][MI], int m_base, int n_base, int lane,
                                                const GemmArgs& args, uint8_t* stage, const uint8_t* meta = nullptr,
-                                               int row0 = 0, int col0 = 0) {
+                                               int row0 = 0, int col0 = 0, const half8_t* pre = nullptr) {
   const int M = args.M, N = args.N;
   const int fr = lane & 31, fk = lane >> 5;
   if constexpr (EPI == FF_EPI_I32) {  // debug output: raw accumulators, stored from registers
@@ -167,22 +176,27 @@ __device__ __forceinline__ void store_epilogue(const int16_t_v (&acc)[NI][MI], i
     half_t* o16 = static_cast<half_t*>(args.out) + static_cast<int64_t>(m_base) * out_ld;
     const int o_bytes = buf_bytes(static_cast<int64_t>(M - m_base) * out_ld * 2);
     // Scale and bias of the wave's 32 NI columns, loaded once per lane column group (i, q); past N they read zeros
-    // (those columns are never stored).
+    // (those columns are never stored). A single row block takes them from LDS where it uses them instead: held, they
+    // are 32 NI registers.
     float4_t cs[NI][4], bi[NI][4];
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t off = static_cast<uint32_t>(32 * i + 8 * q + 4 * fk) * 4;
-        if (meta) {
-          cs[i][q] = *reinterpret_cast<const float4_t*>(meta + col0 * 4 + off);
-          bi[i][q] = *reinterpret_cast<const float4_t*>(meta + 1024 + col0 * 4 + off);
-        } else {
-          const int nb = buf_bytes(static_cast<int64_t>(N - n_base) * 4);
-          cs[i][q] = buf_load_f4(args.col_scale + n_base, nb, off);
-          bi[i][q] = buf_load_f4(args.bias + n_base, nb, off);
-        }
+    auto load_cols = [&](int i, int q) __attribute__((always_inline)) {
+      const uint32_t off = static_cast<uint32_t>(32 * i + 8 * q + 4 * fk) * 4;
+      if constexpr (LDS_META) {
+        cs[i][q] = *reinterpret_cast<const float4_t*>(meta + col0 * 4 + off);
+        bi[i][q] = *reinterpret_cast<const float4_t*>(meta + 1024 + col0 * 4 + off);
+      } else {
+        const int nb = buf_bytes(static_cast<int64_t>(N - n_base) * 4);
+        cs[i][q] = buf_load_f4(args.col_scale + n_base, nb, off);
+        bi[i][q] = buf_load_f4(args.bias + n_base, nb, off);
       }
+    };
+    constexpr bool COLS_LATE = MI == 1 && LDS_META;
+    if constexpr (!COLS_LATE) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) load_cols(i, q);
+    }
     // Per-row inputs are software-pipelined: the row scale of block j + 1 is loaded as soon as block j's results are
     // computed, and the residual rows (or RoPE table rows) of block j + 1 as soon as block j is stored, so their
     // latency hides behind the other phase. The staging area needs no barrier: one wave's LDS operations execute in
@@ -203,7 +217,7 @@ __device__ __forceinline__ void store_epilogue(const int16_t_v (&acc)[NI][MI], i
     };
     auto load_row = [&](int j) __attribute__((always_inline)) {
       // rows past M read 0 (computed, never stored)
-      if (meta)
+      if constexpr (LDS_META)
         rs = *reinterpret_cast<const float*>(meta + 2048 + (row0 + 32 * j + fr) * 4);
       else
         rs = buf_load_f1(args.row_scale + m_base, buf_bytes(static_cast<int64_t>(M - m_base) * 4),
@@ -241,7 +255,14 @@ __device__ __forceinline__ void store_epilogue(const int16_t_v (&acc)[NI][MI], i
       }
     };
     load_row(0);
-    load_residual(0);
+    if constexpr (EPI == FF_EPI_RESIDUAL) {
+      if constexpr (PRE) {
+#pragma unroll
+        for (int p = 0; p < 32 / ROWS_PER_PASS; ++p) xres[p] = pre[p];
+      } else {
+        load_residual(0);
+      }
+    }
     load_rope(0);
 #pragma unroll
     for (int j = 0; j < MI; ++j) {
@@ -250,6 +271,7 @@ __device__ __forceinline__ void store_epilogue(const int16_t_v (&acc)[NI][MI], i
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           const int c = 32 * i + 8 * q + 4 * fk;  // column within the wave's tile
+          if constexpr (COLS_LATE) load_cols(i, q);
           float y[4];
 #pragma unroll
           for (int t = 0; t < 4; ++t)
@@ -336,9 +358,12 @@ typedef __attribute__((address_space(3))) void lds_void;
 constexpr int R_BM = 256, R_BN = 128;
 constexpr int R_GROUP_M = 8;                 // m-tiles per tile group
 
-// LDS row layout of a K slice of RK bytes (64: 4 chunks of 16 B, 32: 2 chunks). A 16-byte-per-lane read pass covers
-// 16 rows and 64 banks: with 64-byte rows the chunk XOR bits 2-3 of the row spreads rows r, r+4, r+8, r+12; with
-// 32-byte rows (8 rows per 256 B) the chunk XOR bit 3 of the row separates r from r+8.
+// LDS row layout of a K slice of RK bytes (64: 4 chunks of 16 B, 32: 2 chunks). gfx950 serves a 16-byte-per-lane LDS
+// read 16 lanes at a time from 64 four-byte banks (256 B), so the 16 rows read by 16 consecutive lanes must land in 16
+// distinct 16-byte slots of a 256-byte window. With 64-byte rows, r..r+3 fill one window's 4 slots each, and the XOR
+// with (r >> 2) & 3 spreads r, r+4, r+8, r+12 over the 4 chunk positions (measured: zero bank conflicts, where XOR
+// with bits 1-2 doubles every read); with 32-byte rows (8 rows per 256 B) the chunk XOR bit 3 of the row separates r
+// from r+8.
 template <int RK>
 __device__ __forceinline__ int rswz(int row, int chunk) {
   if constexpr (RK == 64)
@@ -1090,7 +1115,7 @@ __global__ __launch_bounds__(512, 1) void gemm_s8_persist_kernel(const GemmArgs 
     int el = lane;
     asm volatile("" : "+v"(el));
     const uint8_t* md = META ? smem + META_OFF + (r & 1) * META_BYTES : nullptr;
-    store_epilogue<EPI, NI, MI>(acc, m0 + wm * WM, n0 + wn * WN, el, args, stage, md, wm * WM, wn * WN);
+    store_epilogue<EPI, NI, MI, META>(acc, m0 + wm * WM, n0 + wn * WN, el, args, stage, md, wm * WM, wn * WN);
     // Staging in the ring slot: every wave must be done with it before the next slice loads into it. With their own
     // staging areas the waves go on (the next tile's first slice barrier joins them), except for one-slice tiles,
     // whose next metadata load could overwrite the buffer a slower wave still reads.
@@ -1139,124 +1164,207 @@ static int launch_persist(const GemmArgs& args, int epi, hipStream_t st) {
   return check_launch("gemm_s8");
 }
 
-// ---------------- variant 1: 128 x 128 tiles, register-staged double buffering ----------------
+// ---------------- variant 1: 128 x 128 tiles, K split over two groups of 4 waves ----------------
+//
+// For the sizes between variant 6's 64 x 64 blocks (whose operand traffic per product is too high) and the 256-wide
+// tiles (too few of them): EVA02-L's qkv and fc1 at one image are 216 and 396 tiles here, 60 and 110 of 256 x 256. The
+// eight waves are two K groups of 2 x 2 waves, each wave a 64 x 64 sub-tile; group g multiplies the 64-byte K chunks
+// g, g + 2, ... from its own ring of S 16 KB slots (128 A rows + 128 W rows) filled by buffer->LDS loads, so two waves
+// per SIMD work on one tile and a tile takes half the steps. One barrier per step: a slot's loads are waited for with
+// a counter (S - 2 newer slots stay in flight), and past the last chunk the loads read through an empty descriptor
+// (zeros, whose products add nothing), so every step is the same. The groups then swap halves of their int32 partial
+// tiles through LDS and each wave finishes 32 rows x 64 columns; its residual rows load under the swap, and the tile's
+// scales and biases sit in LDS since before its first slice.
+// A step loads 32 KB per CU in ~0.32 us (45 B/clk of the ~55 B/clk load path), which bounds the loop. Per launch, M =
+// 1025, weights rotating over four copies: N = 3072, K = 1024 10.8 us (256 x 128 tiles 12.1, 64 x 64 blocks 13.8);
+// N = 2304, K = 768 9.1 (11.1, 10.4); N = 1024, K = 4736 at M = 3075 28.7 (31.0, 38.3). Two tiles per CU with 2-slot
+// rings ran 20.8 us at M = 2050, N = 3072, behind the 256-wide tiles (15.1), so there is no such form.
+constexpr int PR_SLOT = (128 + 128) * 64, PR_RING = 4;
 
-template <int BM, int BN, int EPI>
-__global__ __launch_bounds__(256) void gemm_s8_kernel(const GemmArgs args) {
-  constexpr int WM = BM / 2, WN = BN / 2;     // wave sub-tile
-  constexpr int MI = WM / 32, NI = WN / 32;   // 32x32 MFMA blocks per wave
-  constexpr int A_LD = BM * (BK / 16) / 256;  // 16-byte chunks per thread per slice
-  constexpr int W_LD = BN * (BK / 16) / 256;
-  constexpr int STAGE = (BM + BN) * BK;
-  constexpr int SMEM = 2 * STAGE > 4 * stage_bytes<FF_EPI_QKV_ROPE, NI>() ? 2 * STAGE : 4 * stage_bytes<FF_EPI_QKV_ROPE, NI>();
-  __shared__ __attribute__((aligned(16))) int8_t smem[SMEM];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int M = args.M, N = args.N, K = args.K;
-  const int tiles_n = (N + BN - 1) / BN;
-  const int tile = xcd_remap(blockIdx.x, gridDim.x);
-  const int m0 = (tile / tiles_n) * BM, n0 = (tile % tiles_n) * BN;
-  const int KT = K / BK;
-
-  int4_t ra[A_LD], rw[W_LD];
-  auto gload = [&](int kt) {
-    const int kb = kt * BK;
-#pragma unroll
-    for (int p = 0; p < A_LD; ++p) {
-      const int q = tid + 256 * p, r = q >> 2, c = q & 3;
-      const int m = min(m0 + r, M - 1);
-      ra[p] = *reinterpret_cast<const int4_t*>(args.A + static_cast<int64_t>(m) * K + kb + c * 16);
-    }
-#pragma unroll
-    for (int p = 0; p < W_LD; ++p) {
-      const int q = tid + 256 * p, r = q >> 2, c = q & 3;
-      const int n = min(n0 + r, N - 1);
-      rw[p] = *reinterpret_cast<const int4_t*>(args.W + static_cast<int64_t>(n) * K + kb + c * 16);
-    }
-  };
-  auto swrite = [&](int buf) {
-    int8_t* sa = smem + buf * STAGE;
-    int8_t* sw = sa + BM * BK;
-#pragma unroll
-    for (int p = 0; p < A_LD; ++p) {
-      const int q = tid + 256 * p;
-      *reinterpret_cast<int4_t*>(sa + swz(q >> 2, q & 3)) = ra[p];
-    }
-#pragma unroll
-    for (int p = 0; p < W_LD; ++p) {
-      const int q = tid + 256 * p;
-      *reinterpret_cast<int4_t*>(sw + swz(q >> 2, q & 3)) = rw[p];
-    }
-  };
-
-  int16_t_v acc[NI][MI];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < MI; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-
-  const int fr = lane & 31, fk = lane >> 5;  // fragment row, k half
-  auto compute = [&](int buf) {
-    const int8_t* sa = smem + buf * STAGE;
-    const int8_t* sw = sa + BM * BK;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      int4_t xw[NI], ya[MI];
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-        xw[i] = *reinterpret_cast<const int4_t*>(sw + swz(wn * WN + i * 32 + fr, 2 * kk + fk));
-#pragma unroll
-      for (int j = 0; j < MI; ++j)
-        ya[j] = *reinterpret_cast<const int4_t*>(sa + swz(wm * WM + j * 32 + fr, 2 * kk + fk));
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int j = 0; j < MI; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xw[i], ya[j], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  gload(0);
-  swrite(0);
-  __syncthreads();
-  for (int kt = 0; kt < KT; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < KT) gload(kt + 1);
-    compute(cur);
-    if (kt + 1 < KT) swrite(cur ^ 1);
-    __syncthreads();
-  }
-  store_epilogue<EPI, NI, MI>(acc, m0 + wm * WM, n0 + wn * WN, lane, args,
-                              reinterpret_cast<uint8_t*>(smem) + wave * stage_bytes<EPI, NI>());
+// The metadata of the tile at (m0, n0) into LDS, laid out as store_epilogue reads it (1 KB each: column scales,
+// biases, row scales), one buffer->LDS load by each of waves 0-2; entries past N or M read as zeros.
+__device__ __forceinline__ void load_meta(const GemmArgs& args, int m0, int n0, int wave, int lane, uint8_t* meta) {
+  const uint32_t off = static_cast<uint32_t>(lane) * 16;
+  const int cols = buf_bytes(static_cast<int64_t>(args.N - n0) * 4);
+  if (wave == 0)
+    buffer_to_lds(args.col_scale + n0, cols, meta, off);
+  else if (wave == 1)
+    buffer_to_lds(args.bias + n0, cols, meta + 1024, off);
+  else if (wave == 2)
+    buffer_to_lds(args.row_scale + m0, buf_bytes(static_cast<int64_t>(args.M - m0) * 4), meta + 2048, off);
 }
 
-template <int BM, int BN>
-static int launch_staged(const GemmArgs& a, int epi, hipStream_t st) {
-  const int64_t tiles = static_cast<int64_t>((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+// A barrier for LDS traffic only: unlike __syncthreads it leaves global loads in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512, 2) void gemm_s8_pair_kernel(const GemmArgs args) {
+  constexpr bool META = EPI != FF_EPI_I32;
+  constexpr int S = PR_RING, BUFS = 2 * S * PR_SLOT;
+  static_assert(8 * stage_bytes<EPI, 2>() <= BUFS, "staging must fit in the ring");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[BUFS + (META ? META_BYTES : 0)];
+  uint8_t* meta = META ? smem + BUFS : nullptr;
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave >> 2, w4 = wave & 3, wm = w4 >> 1, wn = w4 & 1;
+  const int fr = lane & 31, fk = lane >> 5;
+  const int M = args.M, N = args.N, K = args.K, nch = K / 64, steps = (nch + 1) / 2;
+  const int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int per_group = R_GROUP_M * tiles_n;
+  const int g = t / per_group, in_g = t % per_group;
+  const int gm = min(R_GROUP_M, tiles_m - g * R_GROUP_M);
+  const int m0 = (g * R_GROUP_M + in_g % gm) * 128, n0 = (in_g / gm) * 128;
+
+  // Waves 0, 1 of a group load the slot's A rows (8 KB), waves 2, 3 its W rows: load p of a wave fills rows
+  // 64 (w4 & 1) + 16 p .. + 15; lane l writes physical chunk l % 4 of row l / 4, so it fetches the one rswz puts there.
+  const bool is_a = w4 < 2;
+  const int8_t* gbase = is_a ? args.A + static_cast<int64_t>(m0) * K : args.W + static_cast<int64_t>(n0) * K;
+  const int gbytes = buf_bytes(static_cast<int64_t>(is_a ? M - m0 : N - n0) * K);
+  uint8_t* ring = smem + grp * S * PR_SLOT;
+  uint32_t voff[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int row = 64 * (w4 & 1) + 16 * p + (lane >> 2);
+    voff[p] = static_cast<uint32_t>(row * K + (((lane & 3) ^ ((row >> 2) & 3)) << 4));
+  }
+  auto issue = [&](int i) __attribute__((always_inline)) {
+    const int c = 2 * i + grp;
+    uint8_t* dst = ring + (i % S) * PR_SLOT + w4 * 4096;
+    const int nb = c < nch ? gbytes - c * 64 : 0;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) buffer_to_lds(gbase + c * 64, nb, dst + p * 1024, voff[p]);
+  };
+
+  if constexpr (META) load_meta(args, m0, n0, wave, lane, meta);
+  int16_t_v acc[2][2] = {};
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i) issue(i);
+  for (int i = 0; i < steps; ++i) {
+    // slot i has landed once only the S - 2 newer slots' loads are outstanding; this wave's reads of slot i - 1 are done
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S - 2) * 4) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint8_t* sa = ring + (i % S) * PR_SLOT;
+    const uint8_t* sw = sa + 128 * 64;
+    int4_t xw[2][2], ya[2][2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        xw[kk][x] = *reinterpret_cast<const int4_t*>(sw + rswz<64>(wn * 64 + 32 * x + fr, 2 * kk + fk));
+        ya[kk][x] = *reinterpret_cast<const int4_t*>(sa + rswz<64>(wm * 64 + 32 * x + fr, 2 * kk + fk));
+      }
+    }
+    issue(i + S - 1);  // into the slot of step i - 1, which every wave finished reading before the barrier
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[x][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(xw[kk][x], ya[kk][j], acc[x][j], 0, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the ring takes no more loads
+  lds_barrier();
+  // Wave (grp, w4) finishes row block j = grp of its 64 x 64 and hands block 1 - grp to its partner in the other group.
+  const int fm = m0 + wm * 64 + 32 * grp, fn = n0 + wn * 64;
+  half8_t res[4];
+  if constexpr (EPI == FF_EPI_RESIDUAL) load_residual_rows<2>(res, fm, fn, lane, args);
+  int16_t_v sum[2][1];
+  uint8_t* out_area = smem + (2 * w4 + grp) * 8192 + lane * 16;
+  const uint8_t* in_area = smem + (2 * w4 + 1 - grp) * 8192 + lane * 16;
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int16_t_v give = grp ? acc[x][0] : acc[x][1];
+    sum[x][0] = grp ? acc[x][1] : acc[x][0];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<int4_t*>(out_area + x * 4096 + q * 1024) =
+          int4_t{give[4 * q], give[4 * q + 1], give[4 * q + 2], give[4 * q + 3]};
+  }
+  lds_barrier();
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int4_t v = *reinterpret_cast<const int4_t*>(in_area + x * 4096 + q * 1024);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[x][0][4 * q + e] += v[e];
+    }
+  lds_barrier();  // every partial is read: the ring becomes the epilogue's staging area
+  store_epilogue<EPI, 2, 1, META, true>(sum, fm, fn, lane, args, smem + wave * stage_bytes<EPI, 2>(), meta,
+                                        wm * 64 + 32 * grp, wn * 64, res);
+}
+
+static int launch_pair(const GemmArgs& a, int epi, hipStream_t st) {
+  const int64_t tiles = static_cast<int64_t>((a.M + 127) / 128) * ((a.N + 127) / 128);
   if (tiles > 0x7fffffff) return fail(FF_EINVAL, "gemm_s8: too many tiles");
   const dim3 grid(static_cast<unsigned>(tiles));
   switch (epi) {
-    case FF_EPI_QKV_ROPE: gemm_s8_kernel<BM, BN, FF_EPI_QKV_ROPE><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_RESIDUAL: gemm_s8_kernel<BM, BN, FF_EPI_RESIDUAL><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_GELU_F16: gemm_s8_kernel<BM, BN, FF_EPI_GELU_F16><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_SWIGLU: gemm_s8_kernel<BM, BN, FF_EPI_SWIGLU><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_BIAS_F16: gemm_s8_kernel<BM, BN, FF_EPI_BIAS_F16><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_I32: gemm_s8_kernel<BM, BN, FF_EPI_I32><<<grid, 256, 0, st>>>(a); break;
+    case FF_EPI_QKV_ROPE: gemm_s8_pair_kernel<FF_EPI_QKV_ROPE><<<grid, 512, 0, st>>>(a); break;
+    case FF_EPI_RESIDUAL: gemm_s8_pair_kernel<FF_EPI_RESIDUAL><<<grid, 512, 0, st>>>(a); break;
+    case FF_EPI_GELU_F16: gemm_s8_pair_kernel<FF_EPI_GELU_F16><<<grid, 512, 0, st>>>(a); break;
+    case FF_EPI_SWIGLU: gemm_s8_pair_kernel<FF_EPI_SWIGLU><<<grid, 512, 0, st>>>(a); break;
+    case FF_EPI_BIAS_F16: gemm_s8_pair_kernel<FF_EPI_BIAS_F16><<<grid, 512, 0, st>>>(a); break;
+    case FF_EPI_I32: gemm_s8_pair_kernel<FF_EPI_I32><<<grid, 512, 0, st>>>(a); break;
     default: return fail(FF_EINVAL, "gemm_s8: bad epilogue");
   }
   return check_launch("gemm_s8");
 }
 
-// 1: 128 x 128 register-staged; 2: 256 x 128 buffer->LDS ring (3 slots of K 64), two workgroups per CU;
-// 3: 256 x 256, 8 waves, one workgroup per CU (2 slots of K 128, or 4 slots of K 64 when K % 128 != 0);
-// 4: variant 3 as a persistent grid, the ring streaming across tiles (4 slots of K 64, not persistent, when
-// K % 128 != 0); 5: variant 3 on 256 x 128 tiles of 64 x 64 per wave, 3 slots of K 128; 6: 64 x 64 blocks with K
-// split over 4 waves. These are the variants the engine's autotune picks at the served shapes (1, 5 and 6
-// for small M, 2, 3 and 5 for mid-sized M and the narrower GEMMs, 4 for large M).
+// The engine's autotune picks among these; a call without a choice takes pick_variant's.
 constexpr int kVariants = 6;
+
+// Estimated time of a variant in us on 256 CUs: a launch, its rounds of tiles over the CUs (each a chain of K slices)
+// and the chip-wide throughput of all tiles. The constants are a non-negative least-squares fit to 2100 timed launches
+// (16 products of the taggers and linears, K 768-4736, N 768-5632, M 1-32800, all epilogues), within 5-9 % rms each.
+struct VariantCost {
+  int bm, bn;         // tile
+  int per_round;      // tiles that run at once
+  double launch;      // us per launch
+  double round;       // us per round
+  double round_k;     // us per round and 1000 K
+  double tile;        // us per 256 tiles
+  double tile_k;      // us per 256 tiles and 1000 K
+};
+constexpr VariantCost kCost[kVariants] = {
+    {128, 128, 256, 2.0, 3.5, 2.6, 0.65, 2.5},  {256, 128, 256, 5.2, 0.4, 6.1, 2.4, 2.3},
+    {256, 256, 256, 2.1, 6.0, 7.5, 3.9, 4.75},  {256, 256, 256, 5.0, 2.7, 8.1, 3.6, 5.75},
+    {256, 128, 256, 1.7, 4.3, 4.4, 2.1, 2.8},   {64, 64, 512, 4.0, 0.0, 1.05, 0.245, 1.72},
+};
+
+// The variant of the lowest estimate. Against the fastest variant of each timed product the pick is 0.5 % slower on
+// average and 23 % at worst; the rule it replaces (variant 6 below M = 4096, 3 below 16384, then 4) was 14 % and 138 %:
+// qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. Every variant's results are the same
+// bits.
+static int pick_variant(int64_t M, int64_t N, int64_t K) {
+  auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const double k = static_cast<double>(K) * 1e-3;
+  int best = 1;
+  double best_t = 0.0;
+  for (int v = 1; v <= kVariants; ++v) {
+    const VariantCost& c = kCost[v - 1];
+    const bool persist = v == 4 && K % 128 == 0;
+    const int64_t rows = persist && M > 256 ? M / 256 * 256 : M;  // the rest in 32 x 32 blocks of the same launch
+    const int64_t tiles = cdiv(rows, c.bm) * cdiv(N, c.bn);
+    const double rounds = static_cast<double>(cdiv(tiles, c.per_round)), fill = static_cast<double>(tiles) / 256.0;
+    double t = c.launch + rounds * (c.round + c.round_k * k) + fill * (c.tile + c.tile_k * k);
+    if (rows < M) {
+      const int64_t blocks = cdiv(M - rows, 32) * cdiv(N, 32);
+      t += static_cast<double>(cdiv(blocks, tiles < 256 ? tiles : 256)) * (1.8 + 0.6 * k);
+    }
+    if (v == 1 || t < best_t) {
+      best = v;
+      best_t = t;
+    }
+  }
+  return best;
+}
 
 }  // namespace ff
 
@@ -1308,11 +1416,9 @@ extern "C" int ff_gemm_s8(const int8_t* A, const int8_t* W, int64_t M, int64_t N
   a.rope_len = static_cast<int>(rope_len);
   a.q_scale = q_scale;
   hipStream_t st = as_stream(stream);
-  // The default follows the autotune's usual picks: K-split 64 x 64 blocks while they fill the GPU, 256 x 256 tiles
-  // for mid-size M, the persistent grid from a few tiles per CU on.
-  if (variant == 0) variant = M < 4096 ? 6 : (M < 16384 ? 3 : 4);
+  if (variant == 0) variant = pick_variant(M, N, K);
   switch (variant) {
-    case 1: return launch_staged<128, 128>(a, epi, st);
+    case 1: return launch_pair(a, epi, st);
     case 2: return launch_ring<64, 3>(a, epi, st);
     case 3: return a.K % 128 == 0 ? launch_wide<128, 2>(a, epi, st) : launch_wide<64, 4>(a, epi, st);
     case 4: return a.K % 128 == 0 ? launch_persist(a, epi, st) : launch_wide<64, 4>(a, epi, st);

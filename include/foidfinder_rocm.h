@@ -56,11 +56,10 @@ int ff_rot_q8_h128(const void* x, int64_t T, int64_t C, int64_t c_real, const fl
  * y[m,n] = ((float)(sum_k A[m,k] W[n,k]) * row_scale[m]) * col_scale[n] + bias[n], then the epilogue `epi`.
  * A int8 [M,K], W int8 [N,K] (K contiguous); K % 64 == 0, N % 16 == 0, K <= 2^22, N <= 2^21. rope_cos/rope_sin
  * fp32 [rope_len, 32], 0 < rope_len < 2^24, are needed by FF_EPI_QKV_ROPE only. `variant` selects the tile shape:
- * 1 = 128x128 register-staged, 2 = 256x128 buffer->LDS ring (two workgroups per CU), 3 = 256x256 with 8 waves,
+ * 1 = 128x128 with K over two wave groups, 2 = 256x128 buffer->LDS ring (two workgroups per CU), 3 = 256x256, 8 waves,
  * 4 = variant 3 on a persistent grid (the rows past the last whole 256-row tile as split-K blocks in the same
  * launch), 5 = variant 3 on 256x128 tiles (narrow products at small M), 6 = 64x64 blocks with K split over
- * 4 waves (small M); 0 = a default by M (6 below 4096 rows, 3 below 16384, else 4). All give identical
- * results.
+ * 4 waves (small M); 0 = the fastest by an estimate from M, N and K. All give identical results.
  * Replaces op `gemm_s8(A, W, row_scale, col_scale, bias, out!, epi, stages, rope_cos?, rope_sin?, q_scale)`,
  * foidfinder/backends/cuda/csrc/kernels.cu:187-217, whose `stages` is the same kind of autotuned knob. */
 int ff_gemm_s8(const int8_t* A, const int8_t* W, int64_t M, int64_t N, int64_t K, const float* row_scale,

@@ -245,6 +245,36 @@ def test_w8a8_linear_chain_bit_exact(dev, variant):
     assert bad.size == 0, f"{len(bad)} outputs differ, first at {bad[:4].tolist()}"
 
 
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("epi", [OG.EPI_BIAS_F16, OG.EPI_RESIDUAL, OG.EPI_QKV_ROPE])
+@pytest.mark.parametrize(("M", "N", "K"), [(1, 192, 64), (127, 192, 128), (129, 384, 192), (33, 192, 576),
+                                           (2200, 1536, 64)])
+def test_gemm_s8_k_group_tiles_bit_exact(dev, rng, M, N, K, epi, variant):
+    """The 128 x 128 tiles with K split over two wave groups (and the default pick) where they can go wrong: one K chunk
+    (the second group has none), odd and short chunk counts (below the ring's depth), rows and columns that end inside a
+    tile, more tiles than CUs; the row scales start 4 bytes past a 16-byte boundary (they load 16 bytes a lane). The
+    integer sums are exact and the epilogue's roundings are fixed, so the results are the oracle's bits."""
+    from foidfinder_amd import kernels as Kn
+
+    a, w, rs, cs, bias = gemm_inputs(rng, M, N, K)
+    rope = (rng.uniform(-1, 1, (40, 32)).astype(np.float32), rng.uniform(-1, 1, (40, 32)).astype(np.float32))
+    kw = {}
+    out = torch.empty(M, N, dtype=torch.float16, device=dev)
+    if epi == OG.EPI_RESIDUAL:
+        kw["residual"] = rng.standard_normal((M, N)).astype(np.float16)
+        out = to_gpu(kw["residual"], dev)
+    if epi == OG.EPI_QKV_ROPE:
+        kw.update(rope_cos=rope[0], rope_sin=rope[1], q_scale=OM.Q_SCALE)
+    rs_off = to_gpu(np.concatenate([np.zeros(1, np.float32), rs]), dev)[1:]
+    assert rs_off.data_ptr() % 16 == 4
+    cos, sin = (to_gpu(t, dev) for t in rope) if epi == OG.EPI_QKV_ROPE else (None, None)
+    Kn.gemm_s8(to_gpu(a, dev), to_gpu(w, dev), rs_off, to_gpu(cs, dev), to_gpu(bias, dev), out, epi, variant, cos, sin,
+               kw.get("q_scale", 1.0))
+    got, want = out.cpu().numpy(), OG.gemm_s8(a, w, rs, cs, bias, epi, **kw)
+    bad = np.argwhere(got.view(np.uint16) != want.view(np.uint16))
+    assert bad.size == 0, f"{len(bad)} mismatches, first at {bad[:4].tolist()}"
+
+
 @pytest.mark.parametrize("variant", GEMM_VARIANTS)
 @pytest.mark.parametrize("rope_len", [1, 5, 8, 65, 200])
 def test_gemm_s8_qkv_short_rope_tables(dev, rng, rope_len, variant):
