@@ -18,7 +18,8 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 INCLUDE = PKG.parent / "include"
 LIB = PKG / "libfoidfinder_rocm.so"
-SOURCES = ["capi.hip", "rotq8.hip", "gemm_s8.hip", "attention.hip", "resample.hip", "pool.hip"]
+SOURCES = ["capi.hip", "rotq8.hip", "gemm_s8.hip", "attention.hip", "resample.hip", "pool.hip", "tree_pool.hip",
+           "head.hip"]
 ARCH = "gfx950"
 
 FLAGS = [

@@ -1,0 +1,496 @@
+// Haruka's tree pool (foidfinder/backends/mlx/haruka.py:101-136) as a chain of a few launches. With keys and values
+// never formed (logits = xn . u, u = Wk_h^T q; pooled = w^T xn, then Wv_h), the two attention levels each take:
+//
+//  * pool_weights: logits xn u^T on MFMA and from them the slot-sigmoid weights, transposed, in one kernel;
+//  * (the pooling product w^T xn, a library GEMM)
+//  * pool_values: the value projection of the pooled tokens plus the value bias times each query's mass;
+//
+// and between and after them: pool_queries (parent norm, leaf queries), pool_keys (the leaf queries' u), pool_tree (leaf
+// norm times the mass gate) and pool_leaf (each leaf's own projection). At 16 images these kernels take the place of some
+// 40 launches of 4-13 us, most of them a few hundred KB of element-wise work.
+#include <algorithm>
+
+#include "common.h"
+
+namespace ff {
+
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr uint32_t RSRC_WORD3 = 0x00020000;  // buffer descriptor word 3: raw dword access (gfx9 family)
+
+__device__ __forceinline__ void to_lds(const void* base, int nbytes, void* lds_dst, uint32_t voff) {
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nbytes, RSRC_WORD3);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds_dst, 16, voff, 0, 0, 0);
+}
+
+constexpr int PW_TOK = 64;  // tokens per workgroup of pool_weights
+
+// Grid (token blocks of 64, batch), 8 waves. Logits of the block's tokens against all GM = G M query columns: u [GM, D]
+// and xn stream through two LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
+// conflict-free fragment reads) filled by buffer->LDS loads; rows past GM or the sequence read as zeros. Wave w takes
+// the 32 tokens of half w & 1 and the 32-query tiles w / 2, w / 2 + 4, ... (queries as MFMA rows, tokens as columns). The
+// fp32 logits go to LDS as [GM][64 + 1]; a thread then turns the M logits of a (token, head) pair into weights in place:
+// softmax over the queries times sigmoid(logit + bias), from the hardware exp2 and reciprocal (each about 1 ulp). Tokens
+// past the sequence get weight 0. partial[b, block, j] is column j's sum over the block's tokens, a_t[b, j, n] the weight
+// in fp16 (rows of ldt; a row's pad column may be written with 0).
+// GMAX bounds GM: at 288 (Haruka's 16 heads x 18 leaves) 75 KB of LDS let two workgroups share a CU.
+template <int M, int GMAX>
+__global__ __launch_bounds__(512, GMAX <= 288 ? 4 : 2) void pool_weights_kernel(
+    const half_t* __restrict__ xn, const half_t* __restrict__ u, int64_t u_stride, const float* __restrict__ c,
+    int64_t c_stride, const float* __restrict__ bias, int N, int G, int D, int ldt, half_t* __restrict__ a_t,
+    float* __restrict__ partial) {
+  constexpr int CT = (GMAX + 127) / 128;          // 32-query tiles per wave
+  constexpr int ROWS = 128 * CT + PW_TOK;         // staged rows: queries, then tokens
+  constexpr int SLOT = ROWS * 64;
+  constexpr int LDT = PW_TOK + 1;
+  constexpr int BYTES = 2 * SLOT > GMAX * LDT * 4 ? 2 * SLOT : GMAX * LDT * 4;
+  constexpr float LOG2E = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[BYTES];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int GM = G * M, b = blockIdx.y, n0 = blockIdx.x * PW_TOK;
+  const int ntok = min(PW_TOK, N - n0);
+  const half_t* ub = u + b * u_stride;
+  const half_t* xb = xn + (static_cast<int64_t>(b) * N + n0) * D;
+  const int u_bytes = GM * D * 2, x_bytes = ntok * D * 2;
+
+  auto issue = [&](int kc, int slot) __attribute__((always_inline)) {
+    uint8_t* dst = lds + slot * SLOT;
+#pragma unroll
+    for (int p = 0; p < CT; ++p) {
+      const int q = wave + 8 * p, row = 16 * q + (lane >> 2);
+      to_lds(ub, u_bytes, dst + q * 1024, static_cast<uint32_t>(row * D * 2 + kc * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)));
+    }
+    if (wave < PW_TOK / 16) {
+      const int row = 16 * wave + (lane >> 2);
+      to_lds(xb, x_bytes, dst + 128 * CT * 64 + wave * 1024,
+             static_cast<uint32_t>(row * D * 2 + kc * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)));
+    }
+  };
+  auto frag = [&](const uint8_t* base, int row, int chunk) __attribute__((always_inline)) {
+    return *reinterpret_cast<const half8_t*>(base + row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4));
+  };
+  const int rt = wave & 1, cg = wave >> 1, fr = lane & 31, fh = lane >> 5;
+  float16_t acc[CT] = {};
+  const int chunks = D / 32;
+  issue(0, 0);
+  for (int kc = 0; kc < chunks; ++kc) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // slot kc has landed; every wave has read slot kc - 1
+    asm volatile("" ::: "memory");
+    if (kc + 1 < chunks) issue(kc + 1, (kc + 1) & 1);
+    const uint8_t* su = lds + (kc & 1) * SLOT;
+    const uint8_t* sx = su + 128 * CT * 64;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const half8_t xf = frag(sx, 32 * rt + fr, 2 * ks + fh);
+#pragma unroll
+      for (int i = 0; i < CT; ++i) {
+        if (32 * (cg + 4 * i) >= GM) continue;  // wave-uniform
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(su, 32 * (cg + 4 * i) + fr, 2 * ks + fh), xf, acc[i], 0, 0, 0);
+      }
+    }
+  }
+  __syncthreads();  // the slots are read: the logits take their place
+  float* tile = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int i = 0; i < CT; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int j = 32 * (cg + 4 * i) + 8 * (r >> 2) + 4 * fh + (r & 3);
+      if (j < GM) tile[j * LDT + 32 * rt + fr] = acc[i][r];
+    }
+  const float* cb = c + b * c_stride;
+  __syncthreads();
+  for (int p = threadIdx.x; p < PW_TOK * G; p += 512) {  // a wave's 64 lanes are the block's tokens, its head is uniform
+    const int t = p % PW_TOK, h = __builtin_amdgcn_readfirstlane(p / PW_TOK);
+    float l[M], w[M], mx = -INFINITY, s = 0.f;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      l[m] = tile[(h * M + m) * LDT + t] + cb[h * M + m];
+      mx = fmaxf(mx, l[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      w[m] = __builtin_amdgcn_exp2f((l[m] - mx) * LOG2E);
+      s += w[m];
+    }
+    const float inv = __builtin_amdgcn_rcpf(s);
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float gate = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(__builtin_fmaf(-l[m], LOG2E, -bias[m] * LOG2E)));
+      tile[(h * M + m) * LDT + t] = t < ntok ? w[m] * inv * gate : 0.f;
+    }
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < GM; j += 512) {
+    float s = 0.f;
+#pragma unroll 8
+    for (int t = 0; t < PW_TOK; ++t) s += tile[j * LDT + t];
+    partial[(static_cast<int64_t>(b) * gridDim.x + blockIdx.x) * GM + j] = s;
+  }
+  // two query rows per wave and pass, two tokens (4 bytes) per lane; ldt is even, so a pair past an odd end is pad
+  const int t2 = 2 * (lane & 31);
+  if (t2 < ntok)
+    for (int j = 2 * wave + (lane >> 5); j < GM; j += 16)
+      *reinterpret_cast<half2_t*>(a_t + (static_cast<int64_t>(b) * GM + j) * ldt + n0 + t2) =
+          half2_t{static_cast<half_t>(tile[j * LDT + t2]), static_cast<half_t>(tile[j * LDT + t2 + 1])};
+}
+
+// One 16 x 16 product tile over K (K % 32 == 0, columns contiguous) by 4 waves: wave w takes the 32-column steps w,
+// w + 4, ...; lane l's pointers are at its row (l % 16) and column 8 (l / 16). The waves' sums meet in LDS; every lane of
+// wave 0 returns D[a row 4 (l / 16) + i][b row l % 16].
+__device__ __forceinline__ float4_t tile16(const half_t* a, const half_t* b, int K, float4_t (&part)[4][64]) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float4_t acc = {};
+  const int steps = K / 32;
+#pragma unroll 6
+  for (int s = wave; s < steps; s += 4)
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const half8_t*>(a + 32 * s),
+                                                 *reinterpret_cast<const half8_t*>(b + 32 * s), acc, 0, 0, 0);
+  part[wave][lane] = acc;
+  __syncthreads();
+  return part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+}
+
+// z[b, m, h hd + e] = sum_d pooled[b, h M + m, d] wv[h hd + e, d] + mass[b, h, m] bv[h hd + e], the mass summed from the
+// weights' partial sums. Grid (hd / 16, ceil(B M / 16), G).
+__global__ __launch_bounds__(256) void pool_values_kernel(const half_t* __restrict__ pooled, const half_t* __restrict__ wv,
+                                                          const float* __restrict__ bv, const float* __restrict__ partial,
+                                                          int nblk, int B, int G, int M, int hd, half_t* __restrict__ z) {
+  __shared__ float4_t part[4][64];
+  __shared__ float mass[16];
+  const int lane = threadIdx.x & 63, D = G * hd, R = B * M;
+  const int e0 = 16 * blockIdx.x, r0 = 16 * blockIdx.y, h = blockIdx.z;
+  {
+    const int r = min(r0 + static_cast<int>(threadIdx.x >> 4), R - 1);
+    const float* p = partial + (static_cast<int64_t>(r / M) * nblk * G + h) * M + r % M;
+    float s = 0.f;
+    for (int k = threadIdx.x & 15; k < nblk; k += 16) s += p[static_cast<int64_t>(k) * G * M];
+    s = s + dpp<DPP_XOR15>(s);
+    s = s + dpp<DPP_XOR7>(s);
+    s = s + dpp<DPP_XOR3>(s);
+    s = s + dpp<DPP_XOR1>(s);
+    if ((threadIdx.x & 15) == 0) mass[threadIdx.x >> 4] = s;
+  }
+  const int r = min(r0 + (lane & 15), R - 1);
+  const half_t* pa = wv + static_cast<int64_t>(h * hd + e0 + (lane & 15)) * D + 8 * (lane >> 4);
+  const half_t* pb = pooled + (static_cast<int64_t>(r / M) * G * M + h * M + r % M) * D + 8 * (lane >> 4);
+  const float4_t v = tile16(pa, pb, D, part);
+  if (threadIdx.x >= 64 || r0 + (lane & 15) >= R) return;
+  const int e = h * hd + e0 + 4 * (lane >> 4);
+  half4_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = static_cast<half_t>(__builtin_fmaf(mass[lane & 15], bv[e + i], v[i]));
+  *reinterpret_cast<half4_t*>(z + static_cast<int64_t>(r0 + (lane & 15)) * D + e) = o;
+}
+
+// LayerNorm of a row held two columns per lane and step, c = 2 (lane + 64 k), D <= 128 PER: v = (v - mean) rstd g + b.
+template <int PER>
+__device__ __forceinline__ void norm_row(float (&v)[PER][2], int D, const half_t* g, const half_t* b, float eps) {
+  const int lane = threadIdx.x & 63;
+  float s = 0.f, q = 0.f;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) s += v[k][0] + v[k][1];  // columns past D hold zeros
+  const float mean = wave_sum(s) / static_cast<float>(D);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float d = 2 * (lane + 64 * k) < D ? v[k][e] - mean : 0.f;
+      q = __builtin_fmaf(d, d, q);
+    }
+  const float rstd = 1.f / sqrtf(wave_sum(q) / static_cast<float>(D) + eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = 2 * (lane + 64 * k);
+    if (c < D) {
+      const half2_t gk = *reinterpret_cast<const half2_t*>(g + c), bk = *reinterpret_cast<const half2_t*>(b + c);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        v[k][e] = (v[k][e] - mean) * rstd * static_cast<float>(gk[e]) + static_cast<float>(bk[e]);
+    }
+  }
+}
+template <int PER>
+__device__ __forceinline__ void load_row2(float (&v)[PER][2], const half_t* row, int D, bool add) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = 2 * (lane + 64 * k);
+    const half2_t x = c < D ? *reinterpret_cast<const half2_t*>(row + c) : half2_t{};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[k][e] = (add ? v[k][e] : 0.f) + static_cast<float>(x[e]);
+  }
+}
+template <int PER>
+__device__ __forceinline__ void store_row2(const float (&v)[PER][2], half_t* row, int D) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = 2 * (lane + 64 * k);
+    if (c < D) *reinterpret_cast<half2_t*>(row + c) = half2_t{static_cast<half_t>(v[k][0]), static_cast<half_t>(v[k][1])};
+  }
+}
+
+struct Norm {
+  const half_t *g, *b;
+};
+
+// One wave per (batch, leaf q): its parent is coarse query m = q C / Q. parent[b, m] = LN(z[b, m]; trunk), qleaf[b, q] =
+// LN(parent + child[q]; childn), cq[b, h Q + q] = sum over head h's columns of qleaf bk (the keys' bias term).
+template <int PER>
+__global__ __launch_bounds__(64) void pool_queries_kernel(const half_t* __restrict__ z, Norm trunk,
+                                                          const half_t* __restrict__ child, Norm childn,
+                                                          const float* __restrict__ bk, float eps, int C, int Q, int G,
+                                                          int D, half_t* __restrict__ parent, half_t* __restrict__ qleaf,
+                                                          float* __restrict__ cq) {
+  __shared__ float prod[128 * PER];
+  const int q = blockIdx.x, b = blockIdx.y, lane = threadIdx.x, m = q / (Q / C), hd = D / G;
+  float v[PER][2];
+  load_row2(v, z + (static_cast<int64_t>(b) * C + m) * D, D, false);
+  norm_row(v, D, trunk.g, trunk.b, eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[k][e] = static_cast<float>(static_cast<half_t>(v[k][e]));  // as the stored parent
+  if (q % (Q / C) == 0) store_row2(v, parent + (static_cast<int64_t>(b) * C + m) * D, D);
+  load_row2(v, child + static_cast<int64_t>(q) * D, D, true);
+  norm_row(v, D, childn.g, childn.b, eps);
+  store_row2(v, qleaf + (static_cast<int64_t>(b) * Q + q) * D, D);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = 2 * (lane + 64 * k);
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      if (c < D) prod[c + e] = static_cast<float>(static_cast<half_t>(v[k][e])) * bk[c + e];
+  }
+  __syncthreads();
+  for (int h = lane; h < G; h += 64) {
+    float s = 0.f;
+    for (int e = 0; e < hd; ++e) s += prod[h * hd + e];
+    cq[(static_cast<int64_t>(b) * G + h) * Q + q] = s;
+  }
+}
+
+// u[b, h Q + q, d] = sum_e qleaf[b, q, h hd + e] kT[h, d, e]: one wave per 16 (batch, query) rows x 64 columns d of a head,
+// K = hd in steps of 16 (v_mfma_f32_16x16x16_f16: lane l holds 4 columns 4 (l / 16) .. of row l % 16). Grid
+// (ceil(D / 256), ceil(B Q / 16), G), wave w the w-th 64 columns.
+__global__ __launch_bounds__(256) void pool_keys_kernel(const half_t* __restrict__ qleaf, const half_t* __restrict__ kT,
+                                                        int B, int Q, int G, int hd, half_t* __restrict__ u) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, D = G * hd, R = B * Q;
+  const int d0 = 256 * blockIdx.x + 64 * wave, r0 = 16 * blockIdx.y, h = blockIdx.z, i16 = lane & 15, kq = lane >> 4;
+  if (d0 >= D) return;
+  const int r = min(r0 + i16, R - 1);
+  const half_t* pq = qleaf + static_cast<int64_t>(r) * D + h * hd + 4 * kq;
+  float4_t acc[4] = {};
+  for (int k = 0; k < hd; k += 16) {
+    const half4_t x = *reinterpret_cast<const half4_t*>(pq + k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = min(d0 + 16 * i + i16, D - 1);
+      const half4_t w = *reinterpret_cast<const half4_t*>(kT + (static_cast<int64_t>(h) * D + d) * hd + 4 * kq + k);
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x16f16(w, x, acc[i], 0, 0, 0);
+    }
+  }
+  if (r0 + i16 >= R) return;
+  half_t* o = u + (static_cast<int64_t>(r / Q) * G * Q + h * Q + r % Q) * D + d0 + 4 * kq;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (d0 + 16 * i >= D) break;
+    half4_t v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = static_cast<half_t>(acc[i][e]);
+    *reinterpret_cast<half4_t*>(o + 16 * i) = v;
+  }
+}
+
+// One wave per (batch, leaf): tree[q, b] = LN(parent[b, q C / Q] + zc[b, q]; leafn) * mass / (mass + 4), mass the leaf's
+// weight sum averaged over the heads.
+template <int PER>
+__global__ __launch_bounds__(64) void pool_tree_kernel(const half_t* __restrict__ parent, const half_t* __restrict__ zc,
+                                                       Norm leafn, const float* __restrict__ partial, int nblk, float eps,
+                                                       int C, int Q, int G, int D, half_t* __restrict__ tree) {
+  const int q = blockIdx.x, b = blockIdx.y, B = gridDim.y, lane = threadIdx.x;
+  float s = 0.f;
+  for (int i = lane; i < nblk * G; i += 64) s += partial[(static_cast<int64_t>(b) * nblk * G + i) * Q + q];
+  const float mass = wave_sum(s) / static_cast<float>(G);
+  float v[PER][2];
+  load_row2(v, parent + (static_cast<int64_t>(b) * C + q / (Q / C)) * D, D, false);
+  load_row2(v, zc + (static_cast<int64_t>(b) * Q + q) * D, D, true);
+  norm_row(v, D, leafn.g, leafn.b, eps);
+  const float gate = mass / (mass + 4.f);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[k][e] = v[k][e] * gate;
+  store_row2(v, tree + (static_cast<int64_t>(q) * B + b) * D, D);
+}
+
+// leaf[b, q F + f] = sum_d tree[q, b, d] wl[q, f, d] + bl[q, f]. Grid (F / 16, ceil(B / 16), Q).
+__global__ __launch_bounds__(256) void pool_leaf_kernel(const half_t* __restrict__ tree, const half_t* __restrict__ wl,
+                                                        const half_t* __restrict__ bl, int B, int Q, int F, int D,
+                                                        half_t* __restrict__ leaf) {
+  __shared__ float4_t part[4][64];
+  const int lane = threadIdx.x & 63, f0 = 16 * blockIdx.x, b0 = 16 * blockIdx.y, q = blockIdx.z;
+  const int b = min(b0 + (lane & 15), B - 1);
+  const float4_t v = tile16(wl + (static_cast<int64_t>(q) * F + f0 + (lane & 15)) * D + 8 * (lane >> 4),
+                            tree + (static_cast<int64_t>(q) * B + b) * D + 8 * (lane >> 4), D, part);
+  if (threadIdx.x >= 64 || b0 + (lane & 15) >= B) return;
+  const int f = q * F + f0 + 4 * (lane >> 4);
+  half4_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] = static_cast<half_t>(v[i] + static_cast<float>(bl[f + i]));
+  *reinterpret_cast<half4_t*>(leaf + static_cast<int64_t>(b) * Q * F + f) = o;
+}
+
+}  // namespace ff
+
+using namespace ff;
+
+static bool al(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
+
+// The shapes all of the pool's kernels share: D = G hd columns in whole 32-column steps and 16-column head tiles.
+static const char* pool_shape(int64_t B, int64_t G, int64_t D) {
+  if (B < 0 || B > 65535) return "need 0 <= B <= 65535";
+  if (G <= 0 || G > 64 || D <= 0 || D > 2048 || D % 128 != 0 || D % G != 0 || (D / G) % 16 != 0)
+    return "need 0 < G <= 64 heads of a multiple of 16 columns, D % 128 == 0, D <= 2048";
+  return nullptr;
+}
+#define FF_POOL_CHECK(name, ...)                                                        \
+  if (const char* m = pool_shape(__VA_ARGS__)) return fail(FF_EINVAL, std::string(name ": ") + m)
+
+extern "C" int64_t ff_pool_weights_blocks(int64_t N) { return N > 0 ? (N + PW_TOK - 1) / PW_TOK : 0; }
+
+extern "C" int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, const float* c, int64_t c_stride,
+                               const float* bias, int64_t B, int64_t N, int64_t G, int64_t M, int64_t D, int64_t ldt,
+                               void* a_t, float* partial, void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_weights", B, G, D);
+  if (N <= 0 || N > (1 << 24)) return fail(FF_EINVAL, "pool_weights: bad N");
+  if (M != 6 && M != 18) return fail(FF_EINVAL, "pool_weights: M must be 6 or 18 (the tree pool's query counts)");
+  if (G * M > 512) return fail(FF_EINVAL, "pool_weights: G*M above 512");
+  if ((u_stride != 0 && u_stride < G * M * D) || u_stride % 8 != 0 || (c_stride != 0 && c_stride < G * M))
+    return fail(FF_EINVAL, "pool_weights: u_stride must be 0 or >= G*M*D, c_stride 0 or >= G*M");
+  if (ldt < N || ldt % 2 != 0) return fail(FF_EINVAL, "pool_weights: need ldt >= N, even");
+  if (B == 0) return FF_OK;
+  if (!xn || !u || !c || !bias || !a_t || !partial) return fail(FF_EINVAL, "pool_weights: null pointer");
+  if (!al(xn, 16) || !al(u, 16) || !al(a_t, 4)) return fail(FF_EINVAL, "pool_weights: misaligned pointer");
+  const dim3 grid(static_cast<unsigned>(ff_pool_weights_blocks(N)), static_cast<unsigned>(B));
+  const hipStream_t st = as_stream(stream);
+  const auto *px = static_cast<const half_t*>(xn), *pu = static_cast<const half_t*>(u);
+  auto* pa = static_cast<half_t*>(a_t);
+  const int Ni = static_cast<int>(N), Gi = static_cast<int>(G), Di = static_cast<int>(D), li = static_cast<int>(ldt);
+#define FF_PW(MM, GMAX) \
+  pool_weights_kernel<MM, GMAX><<<grid, 512, 0, st>>>(px, pu, u_stride, c, c_stride, bias, Ni, Gi, Di, li, pa, partial)
+  if (M == 6 && G * M <= 96)
+    FF_PW(6, 96);
+  else if (M == 6)
+    FF_PW(6, 512);
+  else if (G * M <= 288)
+    FF_PW(18, 288);
+  else
+    FF_PW(18, 512);
+#undef FF_PW
+  return check_launch("pool_weights");
+}
+
+extern "C" int ff_pool_values(const void* pooled, const void* wv, const float* bv, const float* partial, int64_t nblk,
+                              int64_t B, int64_t G, int64_t M, int64_t D, void* z, void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_values", B, G, D);
+  if (M <= 0 || M > 64 || nblk <= 0 || nblk > (1 << 24)) return fail(FF_EINVAL, "pool_values: bad M or nblk");
+  if (B == 0) return FF_OK;
+  if (!pooled || !wv || !bv || !partial || !z) return fail(FF_EINVAL, "pool_values: null pointer");
+  if (!al(pooled, 16) || !al(wv, 16) || !al(z, 8)) return fail(FF_EINVAL, "pool_values: misaligned pointer");
+  const int hd = static_cast<int>(D / G);
+  const int64_t rows = (B * M + 15) / 16;
+  if (rows > 65535) return fail(FF_EINVAL, "pool_values: B*M too large");
+  const dim3 grid(static_cast<unsigned>(hd / 16), static_cast<unsigned>(rows), static_cast<unsigned>(G));
+  pool_values_kernel<<<grid, 256, 0, as_stream(stream)>>>(
+      static_cast<const half_t*>(pooled), static_cast<const half_t*>(wv), bv, partial, static_cast<int>(nblk),
+      static_cast<int>(B), static_cast<int>(G), static_cast<int>(M), hd, static_cast<half_t*>(z));
+  return check_launch("pool_values");
+}
+
+extern "C" int ff_pool_queries(const void* z, const void* trunk_g, const void* trunk_b, const void* child,
+                               const void* child_g, const void* child_b, const float* bk, float eps, int64_t B, int64_t C,
+                               int64_t Q, int64_t G, int64_t D, void* parent, void* qleaf, float* cq, void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_queries", B, G, D);
+  if (C <= 0 || Q <= 0 || Q > 65535 || Q % C != 0) return fail(FF_EINVAL, "pool_queries: need C | Q");
+  if (!(eps > 0.f)) return fail(FF_EINVAL, "pool_queries: eps must be > 0");
+  if (B == 0) return FF_OK;
+  if (!z || !trunk_g || !trunk_b || !child || !child_g || !child_b || !bk || !parent || !qleaf || !cq)
+    return fail(FF_EINVAL, "pool_queries: null pointer");
+  for (const void* p : {z, trunk_g, trunk_b, child, child_g, child_b, const_cast<const void*>(parent),
+                        const_cast<const void*>(qleaf)})
+    if (!al(p, 4)) return fail(FF_EINVAL, "pool_queries: misaligned pointer");
+  const dim3 grid(static_cast<unsigned>(Q), static_cast<unsigned>(B));
+  const Norm t{static_cast<const half_t*>(trunk_g), static_cast<const half_t*>(trunk_b)};
+  const Norm n{static_cast<const half_t*>(child_g), static_cast<const half_t*>(child_b)};
+  const auto *pz = static_cast<const half_t*>(z), *pc = static_cast<const half_t*>(child);
+  auto *pp = static_cast<half_t*>(parent), *pq = static_cast<half_t*>(qleaf);
+  const int Ci = static_cast<int>(C), Qi = static_cast<int>(Q), Gi = static_cast<int>(G), Di = static_cast<int>(D);
+  if (D <= 768)
+    pool_queries_kernel<6><<<grid, 64, 0, as_stream(stream)>>>(pz, t, pc, n, bk, eps, Ci, Qi, Gi, Di, pp, pq, cq);
+  else
+    pool_queries_kernel<16><<<grid, 64, 0, as_stream(stream)>>>(pz, t, pc, n, bk, eps, Ci, Qi, Gi, Di, pp, pq, cq);
+  return check_launch("pool_queries");
+}
+
+extern "C" int ff_pool_keys(const void* qleaf, const void* kT, int64_t B, int64_t Q, int64_t G, int64_t D, void* u,
+                            void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_keys", B, G, D);
+  if (Q <= 0 || Q > 65535) return fail(FF_EINVAL, "pool_keys: bad Q");
+  if (B == 0) return FF_OK;
+  if (!qleaf || !kT || !u) return fail(FF_EINVAL, "pool_keys: null pointer");
+  if (!al(qleaf, 8) || !al(kT, 8) || !al(u, 8)) return fail(FF_EINVAL, "pool_keys: misaligned pointer");
+  const int64_t rows = (B * Q + 15) / 16;
+  if (rows > 65535) return fail(FF_EINVAL, "pool_keys: B*Q too large");
+  const dim3 grid(static_cast<unsigned>((D + 255) / 256), static_cast<unsigned>(rows), static_cast<unsigned>(G));
+  pool_keys_kernel<<<grid, 256, 0, as_stream(stream)>>>(static_cast<const half_t*>(qleaf), static_cast<const half_t*>(kT),
+                                                        static_cast<int>(B), static_cast<int>(Q), static_cast<int>(G),
+                                                        static_cast<int>(D / G), static_cast<half_t*>(u));
+  return check_launch("pool_keys");
+}
+
+extern "C" int ff_pool_tree(const void* parent, const void* zc, const void* g, const void* b, const float* partial,
+                            int64_t nblk, float eps, int64_t B, int64_t C, int64_t Q, int64_t G, int64_t D, void* tree,
+                            void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_tree", B, G, D);
+  if (C <= 0 || Q <= 0 || Q > 65535 || Q % C != 0) return fail(FF_EINVAL, "pool_tree: need C | Q");
+  if (nblk <= 0 || nblk > (1 << 24)) return fail(FF_EINVAL, "pool_tree: bad nblk");
+  if (!(eps > 0.f)) return fail(FF_EINVAL, "pool_tree: eps must be > 0");
+  if (B == 0) return FF_OK;
+  if (!parent || !zc || !g || !b || !partial || !tree) return fail(FF_EINVAL, "pool_tree: null pointer");
+  for (const void* p : {parent, zc, g, b, const_cast<const void*>(tree)})
+    if (!al(p, 4)) return fail(FF_EINVAL, "pool_tree: misaligned pointer");
+  const dim3 grid(static_cast<unsigned>(Q), static_cast<unsigned>(B));
+  const Norm n{static_cast<const half_t*>(g), static_cast<const half_t*>(b)};
+  const auto *pp = static_cast<const half_t*>(parent), *pz = static_cast<const half_t*>(zc);
+  auto* pt = static_cast<half_t*>(tree);
+  const int nb = static_cast<int>(nblk), Ci = static_cast<int>(C), Qi = static_cast<int>(Q), Gi = static_cast<int>(G),
+            Di = static_cast<int>(D);
+  if (D <= 768)
+    pool_tree_kernel<6><<<grid, 64, 0, as_stream(stream)>>>(pp, pz, n, partial, nb, eps, Ci, Qi, Gi, Di, pt);
+  else
+    pool_tree_kernel<16><<<grid, 64, 0, as_stream(stream)>>>(pp, pz, n, partial, nb, eps, Ci, Qi, Gi, Di, pt);
+  return check_launch("pool_tree");
+}
+
+extern "C" int ff_pool_leaf(const void* tree, const void* wl, const void* bl, int64_t B, int64_t Q, int64_t F, int64_t D,
+                            void* leaf, void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_leaf", B, 1, D);
+  if (Q <= 0 || Q > 65535 || F <= 0 || F % 16 != 0 || F > 65536) return fail(FF_EINVAL, "pool_leaf: need F % 16 == 0");
+  if (B == 0) return FF_OK;
+  if (!tree || !wl || !bl || !leaf) return fail(FF_EINVAL, "pool_leaf: null pointer");
+  if (!al(tree, 16) || !al(wl, 16) || !al(leaf, 8)) return fail(FF_EINVAL, "pool_leaf: misaligned pointer");
+  const dim3 grid(static_cast<unsigned>(F / 16), static_cast<unsigned>((B + 15) / 16), static_cast<unsigned>(Q));
+  pool_leaf_kernel<<<grid, 256, 0, as_stream(stream)>>>(static_cast<const half_t*>(tree), static_cast<const half_t*>(wl),
+                                                        static_cast<const half_t*>(bl), static_cast<int>(B),
+                                                        static_cast<int>(Q), static_cast<int>(F), static_cast<int>(D),
+                                                        static_cast<half_t*>(leaf));
+  return check_launch("pool_leaf");
+}

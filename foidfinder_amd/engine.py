@@ -25,7 +25,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 
-from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, kernels, lib, pad_norm
+from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, lib, pad_norm
 
 Q_SCALE = 0.125 * math.log2(math.e)  # softmax scale x log2(e), folded into q by the QKV epilogue (engine.py:26)
 FORMAT = "foidfinder-eva02-int8-v1"
@@ -417,6 +417,10 @@ class Eva02Int8(Int8Engine):
             self._gemm(buf["h8"], lw["fc2"], rs, EPI_RESIDUAL, v["fc2"], x)
             if trace is not None:
                 trace[f"x{i}"] = x.clone()
+        if head_fits(B, self.head_w):
+            out = torch.empty(B, self.head_w.size(0), device=x.device, dtype=torch.float32)
+            k.head(xv[:, 0], self.head_w, self.head_b, out, *self.norm, eps)
+            return out
         cls = F.layer_norm(xv[:, 0].float(), (d,), *self.norm, eps).half()
         return F.linear(cls, self.head_w, self.head_b).float()
 

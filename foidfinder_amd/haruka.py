@@ -31,7 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from .engine import Int8Engine, eva02_rope_tables, rotate_quantize
-from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, kernels, pad_norm, slot_weights_blocks
+from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, pad_norm, pool_weights_blocks, slot_weights_blocks
 
 ARCHITECTURE = "haruka-eva02-tree"  # foidfinder/haruka.py:14
 QUANTIZED = ("qkv", "proj", "fc1", "fc2")  # the backbone linears that run as W8A8
@@ -247,16 +247,26 @@ class HarukaInt8(Int8Engine):
         kv_w, kv_b = t["pool.kv.weight"].double(), t["pool.kv.bias"].double()
         wk, bk = kv_w[:d].reshape(Hp, hd, d), kv_b[:d].reshape(Hp, hd)
         qc = t["pool.q_coarse"].double().reshape(C, Hp, hd)
-        self.coarse_uT = half(torch.einsum("hed,mhe->dhm", wk, qc).reshape(d, Hp * C))  # column h*C + m
+        coarse_u = half(torch.einsum("hed,mhe->hmd", wk, qc).reshape(Hp * C, d))  # row h*C + m
         self.coarse_c = torch.einsum("he,mhe->hm", bk, qc).reshape(Hp * C).float().contiguous()
         self.pool_kT = half(wk.transpose(1, 2))  # [Hp, d, hd]: Wk_h^T
         self.pool_bk = bk.float().contiguous()
-        self.pool_vT = half(kv_w[d:].reshape(Hp, hd, d).transpose(1, 2))  # [Hp, d, hd]: Wv_h^T
         self.pool_bv = kv_b[d:].reshape(Hp, hd).float().contiguous()
         self.q_coarse_bias = t["pool.q_coarse_bias"].float().reshape(cfg.coarse).contiguous()
         self.q_child = half(t["pool.q_child"].reshape(cfg.leaves, d))
         self.q_child_bias = t["pool.q_child_bias"].float().reshape(cfg.leaves).contiguous()
-        self.leaf_w = half(t["pool.leaf.weight"].reshape(cfg.leaves, d, cfg.leaf_dim))
+        leaf_w = half(t["pool.leaf.weight"].reshape(cfg.leaves, d, cfg.leaf_dim))
+        # The pool's own kernels take heads and leaves of whole 16-column tiles (Haruka: 48 and 64); other shapes run
+        # on library products, with those products' weight layouts.
+        self.fused_pool = hd % 16 == 0 and cfg.leaf_dim % 16 == 0 and d <= 2048 and Hp * cfg.leaves <= 512
+        if self.fused_pool:
+            self.coarse_u = coarse_u
+            self.pool_v = half(kv_w[d:])  # [d, d]: Wv
+            self.leaf_wT = leaf_w.transpose(1, 2).contiguous()  # [Q, leaf_dim, d]
+        else:
+            self.coarse_uT = coarse_u.t().contiguous()  # column h*C + m
+            self.pool_vT = half(kv_w[d:].reshape(Hp, hd, d).transpose(1, 2))  # [Hp, d, hd]: Wv_h^T
+            self.leaf_w = leaf_w
         self.leaf_b = half(t["pool.leaf.bias"].reshape(cfg.leaves, cfg.leaf_dim))
         self.head = (half(t["head.weight"]), half(t["head.bias"]))
         cos, sin = eva02_rope_tables(cfg.grid, cfg.rope_ref)  # mlx/haruka.py:22-33
@@ -302,11 +312,53 @@ class HarukaInt8(Int8Engine):
 
         Same algebra as the reference with the key/value projection moved onto the queries' side (see __init__):
         logits = xn @ [Wk_h^T q] + q . bk_h, pooled = (w^T xn) Wv_h^T + bv_h sum(w), so the [B, N, 2d] key/value
-        tensor is never formed. The two LayerNorms (backbone, then pool) are one kernel (ff_layer_norm2), and the
-        weights w (softmax over queries x sigmoid gate), their transpose for the pooling product and their sums over
-        the tokens are another (ff_slot_weights)."""
+        tensor is never formed. The two LayerNorms (backbone, then pool) are one kernel (ff_layer_norm2), the rest of
+        the pool runs in _pool_leaves, and the tags' product streams the head's weights (ff_head, up to 64 images)."""
         cfg, k = self.cfg, self.k
-        B, N, d = x.shape
+        xn = torch.empty_like(x)
+        k.layer_norm2(x, *self.norm, *self.pool["norm"], cfg.eps, xn)
+        leaf = self._pool_leaves(xn) if self.fused_pool else self._pool_leaves_library(xn)
+        w, b = self.head
+        if head_fits(leaf.size(0), w):
+            out = torch.empty(leaf.size(0), cfg.tags, device=x.device, dtype=torch.float32)
+            k.head(leaf, w, b, out)
+            return out
+        return F.linear(leaf, w, b).float()
+
+    def _pool_leaves(self, xn: torch.Tensor) -> torch.Tensor:
+        """Normed tokens [B, N, d] -> leaf features [B, Q * leaf_dim] fp16, on the pool's own kernels: twelve launches
+        a call, where the library products with their element-wise steps take some forty."""
+        cfg, k = self.cfg, self.k
+        B, N, d = xn.shape
+        Hp, C, Q = cfg.pool_heads, cfg.coarse, cfg.leaves
+
+        def new(*shape, dtype=torch.half):
+            return torch.empty(*shape, device=xn.device, dtype=dtype)
+
+        def attend(u, c, bias, M):
+            a_t = new(B, Hp * M, (N + 7) // 8 * 8)  # whole 16-byte rows; the product reads the first N columns
+            partial = new(B, pool_weights_blocks(N), Hp * M, dtype=torch.float32)
+            k.pool_weights(xn, u, c, bias, Hp, a_t, partial)
+            z = new(B, M, d)
+            k.pool_values(torch.bmm(a_t[:, :, :N], xn), self.pool_v, self.pool_bv.view(-1), partial, Hp, z)
+            return z, partial
+
+        z, _ = attend(self.coarse_u, self.coarse_c, self.q_coarse_bias, C)
+        parent, qleaf, cq = torch.empty_like(z), new(B, Q, d), new(B, Hp * Q, dtype=torch.float32)
+        k.pool_queries(z, *self.pool["trunk_norm"], self.q_child, *self.pool["child_q_norm"], self.pool_bk.view(-1), Hp,
+                       cfg.eps, parent, qleaf, cq)
+        u = new(B, Hp * Q, d)
+        k.pool_keys(qleaf, self.pool_kT, u)
+        zc, partial = attend(u, cq, self.q_child_bias, Q)
+        tree, leaf = new(Q, B, d), new(B, Q * cfg.leaf_dim)
+        k.pool_tree(parent, zc, *self.pool["leaf_norm"], partial, Hp, cfg.eps, tree)
+        k.pool_leaf(tree, self.leaf_wT, self.leaf_b, leaf)
+        return leaf
+
+    def _pool_leaves_library(self, xn: torch.Tensor) -> torch.Tensor:
+        """_pool_leaves on library products, for heads or leaves that are not whole 16-column tiles."""
+        cfg, k = self.cfg, self.k
+        B, N, d = xn.shape
         Hp, C, Q = cfg.pool_heads, cfg.coarse, cfg.leaves
         hd = d // Hp
 
@@ -314,14 +366,12 @@ class HarukaInt8(Int8Engine):
             w, b = self.pool[name]
             return F.layer_norm(t, (d,), w, b, cfg.eps)
 
-        xn = torch.empty_like(x)
-        k.layer_norm2(x, *self.norm, *self.pool["norm"], cfg.eps, xn)
         nblk = slot_weights_blocks(N)
 
         def attend(logits, c, bias, M):
             """logits fp16 [B, N, Hp*M] (column h*M + m) + c -> (mass [B, Hp, M] fp32, pooled [B, M, d] fp16)."""
-            a_t = torch.empty(B, Hp * M, N, device=x.device, dtype=torch.half)
-            partial = torch.empty(B, nblk, Hp * M, device=x.device, dtype=torch.float32)
+            a_t = torch.empty(B, Hp * M, N, device=xn.device, dtype=torch.half)
+            partial = torch.empty(B, nblk, Hp * M, device=xn.device, dtype=torch.float32)
             k.slot_weights(logits, c, bias, Hp, a_t, partial)
             mass = partial.sum(1).view(B, Hp, M)
             pooled = torch.bmm(a_t, xn).view(B, Hp, M, d).transpose(0, 1).reshape(Hp, B * M, d)
@@ -341,7 +391,7 @@ class HarukaInt8(Int8Engine):
         mass = mass.mean(1)[..., None]  # [B, Q, 1]: patch mass per leaf, averaged over heads
         z_tree = z_tree * (mass / (mass + 4.0)).half()
         leaf = torch.bmm(z_tree.transpose(0, 1).contiguous(), self.leaf_w).transpose(0, 1) + self.leaf_b
-        return F.linear(leaf.reshape(B, Q * cfg.leaf_dim), *self.head).float()
+        return leaf.reshape(B, Q * cfg.leaf_dim)
 
     def _forward(self, img: torch.Tensor, buf: dict[str, torch.Tensor], trace: dict | None = None) -> torch.Tensor:
         """One forward into the preallocated buffers; `trace` (eager debugging only) collects the stem output and,

@@ -38,6 +38,14 @@ SIGNATURES = {
     "ff_layer_norm2": ([_vp, _i64, _i64, _vp, _vp, _vp, _vp, _f32, _vp, _vp], _int),
     "ff_slot_weights_blocks": ([_i64], _i64),
     "ff_slot_weights": ([_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp], _int),
+    "ff_pool_weights_blocks": ([_i64], _i64),
+    "ff_pool_weights": ([_vp, _vp, _i64, _vp, _i64, _vp, *[_i64] * 6, _vp, _vp, _vp], _int),
+    "ff_pool_values": ([_vp, _vp, _vp, _vp, *[_i64] * 5, _vp, _vp], _int),
+    "ff_pool_queries": ([*[_vp] * 7, _f32, *[_i64] * 5, _vp, _vp, _vp, _vp], _int),
+    "ff_pool_keys": ([_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp], _int),
+    "ff_pool_tree": ([*[_vp] * 5, _i64, _f32, *[_i64] * 5, _vp, _vp], _int),
+    "ff_pool_leaf": ([_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp], _int),
+    "ff_head": ([_vp, _i64, _vp, _vp, _f32, _vp, _vp, _i64, _i64, _i64, _vp, _vp], _int),
 }
 ABI_VERSION = 3
 
@@ -251,6 +259,136 @@ def slot_weights(logits: torch.Tensor, c: torch.Tensor, bias: torch.Tensor, head
                                      _ptr(a_t), _ptr(partial), _stream(logits)))
 
 
+def pool_weights_blocks(N: int) -> int:
+    return lib().ff_pool_weights_blocks(N)
+
+
+def _half(shape: tuple, *ts: torch.Tensor) -> None:
+    for t in ts:
+        _require(t.dtype == torch.float16 and tuple(t.shape) == tuple(shape), f"need fp16 {tuple(shape)}")
+
+
+def _float(numel: int, *ts: torch.Tensor) -> None:
+    for t in ts:
+        _require(t.dtype == torch.float32 and t.numel() == numel, f"need fp32 of {numel} elements")
+
+
+def pool_weights(xn: torch.Tensor, u: torch.Tensor, c: torch.Tensor, bias: torch.Tensor, heads: int, a_t: torch.Tensor,
+                 partial: torch.Tensor) -> None:
+    """Tree-pool weights from the tokens and the queries' u (include/foidfinder_rocm.h, ff_pool_weights): xn fp16
+    [B, N, D], u fp16 [heads*M, D] (shared) or [B, heads*M, D], c fp32 [heads*M] or [B, heads*M], bias fp32 [M] -> a_t
+    fp16 [B, heads*M, ldt], partial fp32 [B, blocks, heads*M]."""
+    _on_gpu(xn, u, c, bias, a_t, partial)
+    B, N, D = xn.shape
+    M = bias.numel()
+    GM = heads * M
+    _require(xn.dtype == torch.float16 and u.dtype == torch.float16 and tuple(u.shape[-2:]) == (GM, D)
+             and (u.dim() == 2 or u.dim() == 3 and u.size(0) == B), "u must be fp16 [heads*M, D] or [B, heads*M, D]")
+    _require(c.dtype == bias.dtype == torch.float32 and c.numel() in (GM, B * GM), "c must be fp32 [heads*M] or [B, heads*M]")
+    _half((B, GM, a_t.size(-1)), a_t)
+    _float(B * pool_weights_blocks(N) * GM, partial)
+    with torch.cuda.device(xn.device):
+        _check(lib().ff_pool_weights(_ptr(xn), _ptr(u), 0 if u.dim() == 2 else GM * D, _ptr(c), 0 if c.numel() == GM else GM,
+                                     _ptr(bias), B, N, heads, M, D, a_t.size(-1), _ptr(a_t), _ptr(partial), _stream(xn)))
+
+
+def pool_values(pooled: torch.Tensor, wv: torch.Tensor, bv: torch.Tensor, partial: torch.Tensor, heads: int,
+                z: torch.Tensor) -> None:
+    """z fp16 [B, M, D] from pooled fp16 [B, heads*M, D], wv fp16 [D, D], bv fp32 [D] and the weights' partial sums."""
+    _on_gpu(pooled, wv, bv, partial, z)
+    B, M, D = z.shape
+    _half((B, M, D), z)
+    _half((B, heads * M, D), pooled)
+    _half((D, D), wv)
+    _float(D, bv)
+    _float(B * partial.size(1) * heads * M, partial)
+    with torch.cuda.device(z.device):
+        _check(lib().ff_pool_values(_ptr(pooled), _ptr(wv), _ptr(bv), _ptr(partial), partial.size(1), B, heads, M, D,
+                                    _ptr(z), _stream(z)))
+
+
+def pool_queries(z: torch.Tensor, trunk_g: torch.Tensor, trunk_b: torch.Tensor, child: torch.Tensor,
+                 child_g: torch.Tensor, child_b: torch.Tensor, bk: torch.Tensor, heads: int, eps: float,
+                 parent: torch.Tensor, qleaf: torch.Tensor, cq: torch.Tensor) -> None:
+    """z fp16 [B, C, D] -> parent fp16 [B, C, D], qleaf fp16 [B, Q, D], cq fp32 [B, heads*Q] (ff_pool_queries)."""
+    _on_gpu(z, trunk_g, trunk_b, child, child_g, child_b, bk, parent, qleaf, cq)
+    B, C, D = z.shape
+    Q = child.size(0)
+    _half((B, C, D), z, parent)
+    _half((B, Q, D), qleaf)
+    _half((Q, D), child)
+    _half((D,), trunk_g, trunk_b, child_g, child_b)
+    _float(D, bk)
+    _float(B * heads * Q, cq)
+    with torch.cuda.device(z.device):
+        _check(lib().ff_pool_queries(_ptr(z), _ptr(trunk_g), _ptr(trunk_b), _ptr(child), _ptr(child_g), _ptr(child_b),
+                                     _ptr(bk), eps, B, C, Q, heads, D, _ptr(parent), _ptr(qleaf), _ptr(cq), _stream(z)))
+
+
+def pool_keys(qleaf: torch.Tensor, kT: torch.Tensor, u: torch.Tensor) -> None:
+    """u fp16 [B, heads*Q, D] from qleaf fp16 [B, Q, D] and kT fp16 [heads, D, D / heads] (ff_pool_keys)."""
+    _on_gpu(qleaf, kT, u)
+    B, Q, D = qleaf.shape
+    heads = kT.size(0)
+    _half((B, Q, D), qleaf)
+    _half((heads, D, D // heads), kT)
+    _half((B, heads * Q, D), u)
+    with torch.cuda.device(u.device):
+        _check(lib().ff_pool_keys(_ptr(qleaf), _ptr(kT), B, Q, heads, D, _ptr(u), _stream(u)))
+
+
+def pool_tree(parent: torch.Tensor, zc: torch.Tensor, g: torch.Tensor, b: torch.Tensor, partial: torch.Tensor,
+              heads: int, eps: float, tree: torch.Tensor) -> None:
+    """tree fp16 [Q, B, D] from parent fp16 [B, C, D], zc fp16 [B, Q, D] and the weights' partial sums (ff_pool_tree)."""
+    _on_gpu(parent, zc, g, b, partial, tree)
+    B, Q, D = zc.shape
+    _half((B, parent.size(1), D), parent)
+    _half((B, Q, D), zc)
+    _half((D,), g, b)
+    _half((Q, B, D), tree)
+    _float(B * partial.size(1) * heads * Q, partial)
+    with torch.cuda.device(zc.device):
+        _check(lib().ff_pool_tree(_ptr(parent), _ptr(zc), _ptr(g), _ptr(b), _ptr(partial), partial.size(1), eps, B,
+                                  parent.size(1), Q, heads, D, _ptr(tree), _stream(zc)))
+
+
+def pool_leaf(tree: torch.Tensor, wl: torch.Tensor, bl: torch.Tensor, leaf: torch.Tensor) -> None:
+    """leaf fp16 [B, Q*F] from tree fp16 [Q, B, D], wl fp16 [Q, F, D], bl fp16 [Q, F] (ff_pool_leaf)."""
+    _on_gpu(tree, wl, bl, leaf)
+    Q, B, D = tree.shape
+    F = wl.size(1)
+    _half((Q, B, D), tree)
+    _half((Q, F, D), wl)
+    _half((Q, F), bl)
+    _half((B, Q * F), leaf)
+    with torch.cuda.device(tree.device):
+        _check(lib().ff_pool_leaf(_ptr(tree), _ptr(wl), _ptr(bl), B, Q, F, D, _ptr(leaf), _stream(tree)))
+
+
+def head_fits(rows: int, W: torch.Tensor) -> bool:
+    """Whether `head` takes this many rows of x with W [N, K] (others go to the library's GEMM)."""
+    return rows <= 64 and W.size(1) % 32 == 0 and W.size(1) <= 1280
+
+
+def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor, gamma: torch.Tensor | None = None,
+         beta: torch.Tensor | None = None, eps: float = 1e-6) -> None:
+    """Tag head: out fp32 [B, N] = LN(x) W^T + bias, x fp16 [B, K] with contiguous rows (any row stride that is a
+    multiple of 8), W fp16 [N, K], bias fp16 [N]; the norm (fp32 gamma, beta [K]) only if given (ff_head)."""
+    _on_gpu(W, bias, out, gamma, beta)
+    B, K = x.shape
+    N = W.size(0)
+    _require(x.device == W.device and x.dtype == torch.float16 and x.stride(1) == 1, "x must be fp16 rows on W's device")
+    _half((N, K), W)
+    _half((N,), bias)
+    _require(out.dtype == torch.float32 and tuple(out.shape) == (B, N), "out must be fp32 [B, N]")
+    if gamma is not None:
+        _require(beta is not None, "gamma and beta go together")
+        _float(K, gamma, beta)
+    with torch.cuda.device(W.device):
+        _check(lib().ff_head(_ptr(x), max(x.stride(0), K), _ptr(gamma), _ptr(beta), eps, _ptr(W), _ptr(bias), B, N, K,
+                             _ptr(out), _stream(W)))
+
+
 # ---- torch.ops.foidfinder_rocm registration (schemas as kernels.cu:268-273, plus eps / the fused norm) ----
 
 _LIB = torch.library.Library("foidfinder_rocm", "DEF")
@@ -270,6 +408,19 @@ _LIB.impl("attention", attention, "CUDA")
 # Haruka's tree pool (no reference CUDA op; out-param ops in the same style)
 _LIB.define("layer_norm2(Tensor x, Tensor g1, Tensor b1, Tensor g2, Tensor b2, float eps, Tensor(a!) out) -> ()")
 _LIB.define("slot_weights(Tensor logits, Tensor c, Tensor bias, int heads, Tensor(a!) a_t, Tensor(b!) partial) -> ()")
+_LIB.define("pool_weights(Tensor xn, Tensor u, Tensor c, Tensor bias, int heads, Tensor(a!) a_t, Tensor(b!) partial) "
+            "-> ()")
+_LIB.define("pool_values(Tensor pooled, Tensor wv, Tensor bv, Tensor partial, int heads, Tensor(a!) z) -> ()")
+_LIB.define("pool_queries(Tensor z, Tensor trunk_g, Tensor trunk_b, Tensor child, Tensor child_g, Tensor child_b, "
+            "Tensor bk, int heads, float eps, Tensor(a!) parent, Tensor(b!) qleaf, Tensor(c!) cq) -> ()")
+_LIB.define("pool_keys(Tensor qleaf, Tensor kT, Tensor(a!) u) -> ()")
+_LIB.define("pool_tree(Tensor parent, Tensor zc, Tensor g, Tensor b, Tensor partial, int heads, float eps, "
+            "Tensor(a!) tree) -> ()")
+_LIB.define("pool_leaf(Tensor tree, Tensor wl, Tensor bl, Tensor(a!) leaf) -> ()")
+_LIB.define("head(Tensor x, Tensor W, Tensor bias, Tensor(a!) out, Tensor? gamma=None, Tensor? beta=None, "
+            "float eps=1e-06) -> ()")
+for _fn in (pool_weights, pool_values, pool_queries, pool_keys, pool_tree, pool_leaf, head):
+    _LIB.impl(_fn.__name__, _fn, "CUDA")
 _LIB.impl("layer_norm2", layer_norm2, "CUDA")
 _LIB.impl("slot_weights", slot_weights, "CUDA")
 

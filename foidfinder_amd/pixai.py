@@ -19,7 +19,7 @@ import torch
 import torch.nn.functional as F
 
 from .engine import Int8Engine, rotate_quantize
-from .kernels import EPI_GELU_F16, EPI_QKV_ROPE, EPI_RESIDUAL, kernels
+from .kernels import EPI_GELU_F16, EPI_QKV_ROPE, EPI_RESIDUAL, head_fits, kernels
 
 FORMAT = "foidfinder-pixai-int8-v1"  # the reference's converted-checkpoint format name (engine.py:46)
 # Quantized block linears -> Hadamard block size of their input rotation (engine.py:45).
@@ -272,7 +272,12 @@ class PixAIInt8(Int8Engine):
         p = torch.softmax(scores, dim=-1)  # over the last dim (torch's softmax over an inner dim is far slower)
         o = (p.unsqueeze(-1) * kv[1]).sum(2).reshape(B, d).half()  # [B, H, 64] -> [B, d]
         o = F.linear(o, *self.pool_proj)
-        return F.linear(o, *self.head).float()
+        w, b = self.head
+        if head_fits(B, w):
+            out = torch.empty(B, w.size(0), device=x.device, dtype=torch.float32)
+            self.k.head(o, w, b, out)
+            return out
+        return F.linear(o, w, b).float()
 
     def _forward(self, img: torch.Tensor, buf: dict[str, torch.Tensor], trace: dict | None = None) -> torch.Tensor:
         """One forward into the preallocated buffers (engine.py:142-161). `trace` (eager debugging) collects the stem

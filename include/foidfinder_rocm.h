@@ -106,6 +106,41 @@ int64_t ff_slot_weights_blocks(int64_t N);
 int ff_slot_weights(const void* logits, const float* c, int64_t c_stride, const float* bias, int64_t B, int64_t N,
                     int64_t G, int64_t M, void* a_t, float* partial, void* stream);
 
+/* The rest of Haruka's tree pool (foidfinder/backends/mlx/haruka.py:101-136) in a few launches: G heads of hd = D / G
+ * columns (hd % 16 == 0, D % 128 == 0, D <= 2048, G <= 64), C coarse queries, Q leaf queries (C | Q), all activations
+ * and weights fp16, sums, biases and masses fp32.
+ *
+ * ff_pool_weights: ff_slot_weights with the logits' product in it: l[m] = xn[b, n] . u[b, h*M + m] + c[...], u fp16
+ * [B, G*M, D] (u_stride elements between batches, 0: shared), M = 6 or 18, G*M <= 512. a_t fp16 [B, G*M, ldt] (ldt >= N,
+ * even; pad columns undefined), partial fp32 [B, ff_pool_weights_blocks(N), G*M]. */
+int64_t ff_pool_weights_blocks(int64_t N);
+int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, const float* c, int64_t c_stride,
+                    const float* bias, int64_t B, int64_t N, int64_t G, int64_t M, int64_t D, int64_t ldt, void* a_t,
+                    float* partial, void* stream);
+/* z[b, m, h*hd + e] = pooled[b, h*M + m] . wv[h*hd + e] + bv[h*hd + e] * sum_k partial[b, k, h*M + m]; pooled
+ * [B, G*M, D], wv [D, D], z [B, M, D]. */
+int ff_pool_values(const void* pooled, const void* wv, const float* bv, const float* partial, int64_t nblk, int64_t B,
+                   int64_t G, int64_t M, int64_t D, void* z, void* stream);
+/* parent [B, C, D] = LN(z; trunk), qleaf [B, Q, D] = LN(parent[q*C/Q] + child[q]; child_g, child_b), cq fp32 [B, G*Q]:
+ * cq[b, h*Q + q] = qleaf[b, q] . bk over head h's columns. */
+int ff_pool_queries(const void* z, const void* trunk_g, const void* trunk_b, const void* child, const void* child_g,
+                    const void* child_b, const float* bk, float eps, int64_t B, int64_t C, int64_t Q, int64_t G,
+                    int64_t D, void* parent, void* qleaf, float* cq, void* stream);
+/* u[b, h*Q + q, d] = sum_e qleaf[b, q, h*hd + e] kT[h, d, e]; kT [G, D, hd], u [B, G*Q, D]. */
+int ff_pool_keys(const void* qleaf, const void* kT, int64_t B, int64_t Q, int64_t G, int64_t D, void* u, void* stream);
+/* tree [Q, B, D]: LN(parent[b, q*C/Q] + zc[b, q]; g, b) * mass / (mass + 4), mass = the mean over the heads of
+ * sum_k partial[b, k, h*Q + q]. */
+int ff_pool_tree(const void* parent, const void* zc, const void* g, const void* b, const float* partial, int64_t nblk,
+                 float eps, int64_t B, int64_t C, int64_t Q, int64_t G, int64_t D, void* tree, void* stream);
+/* leaf[b, q*F + f] = tree[q, b] . wl[q, f] + bl[q, f]; wl [Q, F, D], F % 16 == 0, leaf [B, Q*F]. */
+int ff_pool_leaf(const void* tree, const void* wl, const void* bl, int64_t B, int64_t Q, int64_t F, int64_t D,
+                 void* leaf, void* stream);
+
+/* Tag head: out fp32 [B, N] = LN(x) W^T + bias (the norm only with gamma and beta, fp32 [K]); x fp16, B <= 64 rows
+ * x_stride elements apart (% 8 == 0), W fp16 [N, K], bias fp16 [N], K % 32 == 0, K <= 1280. */
+int ff_head(const void* x, int64_t x_stride, const float* gamma, const float* beta, float eps, const void* W,
+            const void* bias, int64_t B, int64_t N, int64_t K, float* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
