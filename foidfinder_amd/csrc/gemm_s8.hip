@@ -1338,15 +1338,17 @@ constexpr VariantCost kCost[kVariants] = {
     {256, 128, 256, 1.7, 4.3, 4.4, 2.1, 2.8},   {64, 64, 512, 4.0, 0.0, 1.05, 0.245, 1.72},
 };
 
-// The variant of the lowest estimate. Against the fastest variant of each timed product the pick is 0.5 % slower on
-// average and 23 % at worst; the rule it replaces (variant 6 below M = 4096, 3 below 16384, then 4) was 14 % and 138 %:
-// qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. Every variant's results are the same
-// bits.
+// A variant by M alone (6 below 4096 rows, 3 below 16384, then 4), unless another's estimate is lower by more than the
+// fit's error. Against the fastest variant of each timed product the pick is 1 % slower on average; by M alone it was
+// 14 %, and 138 % at worst: qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. (The lowest
+// estimate as it stands took variant 2 for Haruka's qkv at 16 images, 3 % slower than 4 there.) Every variant's results
+// are the same bits.
 static int pick_variant(int64_t M, int64_t N, int64_t K) {
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const double k = static_cast<double>(K) * 1e-3;
-  int best = 1;
-  double best_t = 0.0;
+  const int by_rows = M < 4096 ? 6 : (M < 16384 ? 3 : 4);
+  int best = by_rows;
+  double best_t = 0.0, rows_t = 0.0;
   for (int v = 1; v <= kVariants; ++v) {
     const VariantCost& c = kCost[v - 1];
     const bool persist = v == 4 && K % 128 == 0;
@@ -1358,12 +1360,13 @@ static int pick_variant(int64_t M, int64_t N, int64_t K) {
       const int64_t blocks = cdiv(M - rows, 32) * cdiv(N, 32);
       t += static_cast<double>(cdiv(blocks, tiles < 256 ? tiles : 256)) * (1.8 + 0.6 * k);
     }
+    if (v == by_rows) rows_t = t;
     if (v == 1 || t < best_t) {
       best = v;
       best_t = t;
     }
   }
-  return best;
+  return best_t < 0.94 * rows_t ? best : by_rows;
 }
 
 }  // namespace ff
