@@ -7,7 +7,7 @@ reference's PixAI preprocessing (foidfinder/backends/cuda/preprocess.py:16-32), 
 `preprocess_haruka` (Haruka): the model card's preprocessing (foidfinder/backends/mlx/haruka.py:63-72, the
 reference's tests/test_haruka.py:19-34): composited onto white, Pillow bicubic resize so the longer side is `size`,
 pasted centered on a white canvas, raw uint8 pixels NHWC (the normalization is folded into the patch weights). The
-resize runs on the GPU (`ff_resample_u8`, two separable passes with Pillow's fixed-point taps computed here) and is
+resize runs on the GPU (`ff_resample_u8`, two separable passes with Pillow's fixed-point taps, computed there too) and is
 bit-exact with Pillow 13's `Image.resize(BICUBIC)` (the version the reference pins), as the reference's Metal resize
 is (foidfinder/backends/mlx/kernels.py:75-186).
 """
@@ -84,10 +84,19 @@ def bicubic_taps(in_size: int, out_size: int) -> tuple[np.ndarray, np.ndarray]:
     return kk, np.stack([first, count], axis=1).astype(np.int32)
 
 
+def taps_window(in_size: int, out_size: int, index: int) -> tuple[int, int]:
+    """(first input index, one past the last) of an output index's taps: bicubic_taps' bounds, for one index."""
+    scale = in_size / out_size
+    support = 2.0 * max(scale, 1.0)
+    center = (index + 0.5) * scale
+    return max(math.trunc(center - support + 0.5), 0), min(math.trunc(center + support + 0.5), in_size)
+
+
 def letterbox_gpu(rgb: np.ndarray, size: int, out: torch.Tensor) -> None:
     """uint8 [H, W, 3] -> out uint8 [size, size, 3] on the GPU: bicubic resize so the longer side is size (the other
-    side int(side * ratio), at least 1), centered on white; two passes of ff_resample_u8."""
-    from ...kernels import resample_u8
+    side int(side * ratio), at least 1), centered on white. Only the image goes to the GPU: the taps are computed there
+    (ff_bicubic_taps) for two passes of ff_resample_u8."""
+    from ... import kernels as K
 
     h, w = rgb.shape[:2]
     dev = out.device
@@ -98,22 +107,22 @@ def letterbox_gpu(rgb: np.ndarray, size: int, out: torch.Tensor) -> None:
     r = min(size / w, size / h)
     nw, nh = max(1, int(w * r)), max(1, int(h * r))
     top, left = (size - nh) // 2, (size - nw) // 2
-    kh, bh = bicubic_taps(w, nw)
-    kv, bv = bicubic_taps(h, nh)
-
-    def dev_t(a):
-        return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
-
-    if vertical_first(w, h, nw, nh):
+    down_first = vertical_first(w, h, nw, nh)
+    # horizontal first: only the source rows that the vertical pass reads
+    row0, end = (0, h) if down_first else (taps_window(h, nh, 0)[0], taps_window(h, nh, nh - 1)[1])
+    ks_w, ks_h = (2 * math.ceil(2.0 * max(n / m, 1.0)) + 1 for n, m in ((w, nw), (h, nh)))
+    buf = torch.empty(nw * (ks_w + 2) + nh * (ks_h + 2), dtype=torch.int32, device=dev)
+    kk_w, b_w, kk_h, b_h = buf.split([nw * ks_w, nw * 2, nh * ks_h, nh * 2])
+    kk_w, b_w, kk_h, b_h = kk_w.view(nw, ks_w), b_w.view(nw, 2), kk_h.view(nh, ks_h), b_h.view(nh, 2)
+    K.bicubic_taps((w, nw, 0), (h, nh, row0), kk_w, b_w, kk_h, b_h)
+    if down_first:
         tmp = torch.empty(nh, w, 3, dtype=torch.uint8, device=dev)
-        resample_u8(src, 1, dev_t(kv), dev_t(bv), 0, tmp, (0, 0, nh, w))
-        resample_u8(tmp, 0, dev_t(kh), dev_t(bh), 0, out, (top, left, nh, nw))
+        K.resample_u8(src, 1, kk_h, b_h, 0, tmp, (0, 0, nh, w))
+        K.resample_u8(tmp, 0, kk_w, b_w, 0, out, (top, left, nh, nw))
         return
-    row0 = int(bv[0, 0])  # only the source rows the vertical pass reads
-    rows = int(bv[-1, 0] + bv[-1, 1]) - row0
-    tmp = torch.empty(rows, nw, 3, dtype=torch.uint8, device=dev)
-    resample_u8(src, 0, dev_t(kh), dev_t(bh), row0, tmp, (0, 0, rows, nw))
-    resample_u8(tmp, 1, dev_t(kv), dev_t(bv - np.array([row0, 0], np.int32)), 0, out, (top, left, nh, nw))
+    tmp = torch.empty(end - row0, nw, 3, dtype=torch.uint8, device=dev)
+    K.resample_u8(src, 0, kk_w, b_w, row0, tmp, (0, 0, end - row0, nw))
+    K.resample_u8(tmp, 1, kk_h, b_h, 0, out, (top, left, nh, nw))
 
 
 @torch.no_grad()

@@ -35,6 +35,7 @@ SIGNATURES = {
     "ff_attention": ([_vp, _vp, _i64, _i64, _i64, _vp], _int),
     "ff_resample_u8": ([_vp, _i64, _i64, _int, _vp, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
                        _int),
+    "ff_bicubic_taps": ([*[_i64] * 3, _vp, _vp, *[_i64] * 4, _vp, _vp, _i64, _vp], _int),
     "ff_layer_norm2": ([_vp, _i64, _i64, _vp, _vp, _vp, _vp, _f32, _vp, _vp], _int),
     "ff_slot_weights_blocks": ([_i64], _i64),
     "ff_slot_weights": ([_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp], _int),
@@ -222,6 +223,20 @@ def resample_u8(src: torch.Tensor, axis: int, kk: torch.Tensor, bounds: torch.Te
     with torch.cuda.device(src.device):
         _check(lib().ff_resample_u8(_ptr(src), src.size(0), src.size(1), axis, _ptr(kk), _ptr(bounds), kk.size(1),
                                     row0, _ptr(out), out.size(0), out.size(1), top, left, h, w, _stream(src)))
+
+
+def bicubic_taps(width: tuple[int, int, int], height: tuple[int, int, int], kk_w: torch.Tensor, bounds_w: torch.Tensor,
+                 kk_h: torch.Tensor, bounds_h: torch.Tensor) -> None:
+    """Pillow's bicubic taps of both axes (include/foidfinder_rocm.h, ff_bicubic_taps): `width` and `height` are (input
+    size, output size, shift); kk int32 [output size, ksize], bounds int32 [output size, 2]."""
+    _on_gpu(kk_w, bounds_w, kk_h, bounds_h)
+    for (_, n, _), kk, bounds in ((width, kk_w, bounds_w), (height, kk_h, bounds_h)):
+        _require(kk.dtype == bounds.dtype == torch.int32 and kk.dim() == 2 and kk.size(0) == n
+                 and tuple(bounds.shape) == (n, 2), "kk int32 [n, ksize], bounds int32 [n, 2]")
+    with torch.cuda.device(kk_w.device):
+        _check(lib().ff_bicubic_taps(width[0], width[1], kk_w.size(1), _ptr(kk_w), _ptr(bounds_w), width[2],
+                                     height[0], height[1], kk_h.size(1), _ptr(kk_h), _ptr(bounds_h), height[2],
+                                     _stream(kk_w)))
 
 
 def layer_norm2(x: torch.Tensor, g1: torch.Tensor, b1: torch.Tensor, g2: torch.Tensor, b2: torch.Tensor, eps: float,

@@ -88,6 +88,13 @@ int ff_resample_u8(const uint8_t* src, int64_t src_h, int64_t src_w, int axis, c
                    const int32_t* bounds, int64_t ksize, int64_t row0, uint8_t* out, int64_t out_h, int64_t out_w,
                    int64_t top, int64_t left, int64_t h, int64_t w, void* stream);
 
+/* The bicubic taps of both axes for ff_resample_u8 (Pillow's precompute_coeffs and normalize_coeffs_8bpc with a = -0.5,
+ * the same float64 operations): in_w -> out_w into kk_w int32 [out_w, ksize_w] and bounds_w int32 [out_w, 2] (first input
+ * index minus shift_w, tap count), and the same for the height; ksize = 2 * ceil(2 * max(in / out, 1)) + 1. */
+int ff_bicubic_taps(int64_t in_w, int64_t out_w, int64_t ksize_w, int32_t* kk_w, int32_t* bounds_w, int64_t shift_w,
+                    int64_t in_h, int64_t out_h, int64_t ksize_h, int32_t* kk_h, int32_t* bounds_h, int64_t shift_h,
+                    void* stream);
+
 /* Two LayerNorms in a row over fp16 rows of C (C % 64 == 0, C <= 2048): y = LN(x; g1, b1) rounded to fp16, then
  * out = LN(y; g2, b2) in fp16; fp16 gamma/beta [C], epsilon eps for both. Haruka's final backbone norm followed by its
  * pool's norm (foidfinder/backends/mlx/haruka.py:101, :122); no counterpart in the reference's CUDA backend. */

@@ -274,6 +274,16 @@ def test_bicubic_taps_match_the_oracle():
         assert (np.abs(kk.sum(1).astype(np.int64) - (1 << 22)) <= kk.shape[1]).all()
 
 
+def test_taps_window_is_the_taps_bounds():
+    from foidfinder_amd.backends.rocm.preprocess import bicubic_taps, taps_window
+
+    r = np.random.default_rng(5)
+    for n_in, n_out in [(1, 1), (1, 448), (448, 448), (5000, 1), *(map(int, r.integers(1, 3000, 2)) for _ in range(200))]:
+        _, b = bicubic_taps(n_in, n_out)
+        for i in {0, n_out // 2, n_out - 1}:
+            assert taps_window(n_in, n_out, i) == (b[i, 0], b[i].sum())
+
+
 def test_bicubic_taps_match_the_pillow_known_answers():
     """The reference's own Pillow tap tables (web/src/engine/engine.test.ts:8-34), kept as a fixture."""
     from pathlib import Path

@@ -217,6 +217,23 @@ RESIZE_CASES = [(850, 1200), (448, 900), (3, 5000), (5000, 3), (100, 37), (448, 
                 (900, 449), (9, 900), (9, 910), (10, 1001), (448, 448)]
 
 
+@pytest.mark.parametrize(("width", "height"), [((1200, 448), (900, 336)), ((3, 1), (5000, 448)), ((37, 165), (1, 448)),
+                                               ((65535, 448), (448, 448)), ((1001, 63), (64, 4)), ((7, 3), (449, 448))])
+def test_gpu_bicubic_taps_are_the_host_taps(dev, width, height):
+    """ff_bicubic_taps against the numpy taps, bit for bit (the same float64 operations): enlarging and shrinking, an axis
+    of one output and one of 65535 inputs, output counts around a workgroup's 64, and a shifted first index."""
+    from foidfinder_amd import kernels as K
+    from foidfinder_amd.backends.rocm.preprocess import bicubic_taps
+
+    want = [bicubic_taps(*width), bicubic_taps(*height)]
+    got = [torch.full(a.shape, 99, dtype=torch.int32, device=dev) for pair in want for a in pair]
+    shift = int(want[1][1][0, 0])
+    K.bicubic_taps((*width, 0), (*height, shift), *got)
+    want[1][1][:, 0] -= shift
+    for g, a in zip(got, (a for pair in want for a in pair)):
+        assert np.array_equal(g.cpu().numpy(), a)
+
+
 @pytest.mark.parametrize(("w", "h"), RESIZE_CASES)
 def test_gpu_letterbox_is_bit_exact_with_pillow(dev, w, h):
     """The Haruka letterbox on the GPU (ff_resample_u8, two passes) against the oracle's letterbox in the pass order of
