@@ -59,83 +59,83 @@ __global__ __launch_bounds__(256) void layer_norm2_kernel(const half_t* __restri
     if (64 * k + lane < C) orow[64 * k + lane] = static_cast<half_t>(v[k]);
 }
 
-// The same two norms for C % 256 == 0 (Haruka's 768): lane l holds the 4 contiguous columns 4 (l + 64 k), so each
-// load and store moves 8 bytes per lane, and each wave streams rows (row = wave id + k * waves in the grid) with the
-// four affine vectors kept in registers. Same arithmetic as layer_norm2_kernel; only the order of the sums differs.
+// The same two norms for C = 256 CH (Haruka's 768): a row per 32-lane half-wave, lane l the 8 columns 8 (l + 32 k) .. of
+// each 256, so a load or store moves 16 bytes per lane, the reductions need no step across the halves, and each serves
+// two rows. Half-waves stream rows with the four affine vectors in registers and the next row's loads in flight. Same
+// arithmetic as layer_norm2_kernel; only the order of the sums differs.
 template <int CH>
-__global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __restrict__ x, int64_t T, int C,
+__global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __restrict__ x, int64_t T,
                                                               const half_t* __restrict__ g1,
                                                               const half_t* __restrict__ b1,
                                                               const half_t* __restrict__ g2,
                                                               const half_t* __restrict__ b2, float eps,
                                                               half_t* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int64_t waves = static_cast<int64_t>(gridDim.x) * 4;
-  const int nch = C / 256;  // chunks per lane (<= CH)
-  half4_t ga[CH], ba[CH], gb[CH], bb[CH];
-#pragma unroll
-  for (int k = 0; k < CH; ++k)
-    if (k < nch) {
-      const int c = 4 * (lane + 64 * k);
-      ga[k] = *reinterpret_cast<const half4_t*>(g1 + c);
-      ba[k] = *reinterpret_cast<const half4_t*>(b1 + c);
-      gb[k] = *reinterpret_cast<const half4_t*>(g2 + c);
-      bb[k] = *reinterpret_cast<const half4_t*>(b2 + c);
-    }
-  const float inv_c = 1.f / static_cast<float>(C);
-  // the next row's loads are issued before the current row's reductions, so a wave always has a row in flight
-  half4_t nxt[CH];
+  constexpr int C = 256 * CH;
+  const int lane = threadIdx.x & 31;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * 8;
+  half8_t ga[CH], ba[CH], gb[CH], bb[CH], nxt[CH];
   auto load = [&](int64_t r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < CH; ++k)
-      nxt[k] = k < nch ? *reinterpret_cast<const half4_t*>(x + r * C + 4 * (lane + 64 * k)) : half4_t{};
+    for (int k = 0; k < CH; ++k) nxt[k] = *reinterpret_cast<const half8_t*>(x + r * C + 8 * (lane + 32 * k));
   };
-  int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  int64_t row = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
   if (row < T) load(row);
-  for (; row < T; row += waves) {
-    float v[CH][4];
+#pragma unroll
+  for (int k = 0; k < CH; ++k) {
+    const int c = 8 * (lane + 32 * k);
+    ga[k] = *reinterpret_cast<const half8_t*>(g1 + c);
+    ba[k] = *reinterpret_cast<const half8_t*>(b1 + c);
+    gb[k] = *reinterpret_cast<const half8_t*>(g2 + c);
+    bb[k] = *reinterpret_cast<const half8_t*>(b2 + c);
+  }
+  constexpr float inv_c = 1.f / static_cast<float>(C);
+  auto half_sum = [](float v) __attribute__((always_inline)) {
+    v = v + swz_xor16(v);
+    v = v + dpp<DPP_XOR15>(v);
+    v = v + dpp<DPP_XOR7>(v);
+    v = v + dpp<DPP_XOR3>(v);
+    return v + dpp<DPP_XOR1>(v);
+  };
+  for (; row < T; row += stride) {  // the halves of a wave may end apart: every cross-lane step stays inside a half
+    float v[CH][8];
 #pragma unroll
     for (int k = 0; k < CH; ++k)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) v[k][t] = static_cast<float>(nxt[k][t]);
-    if (row + waves < T) load(row + waves);
-    auto norm = [&](const half4_t (&g)[CH], const half4_t (&b)[CH], bool round_fp16) __attribute__((always_inline)) {
+      for (int t = 0; t < 8; ++t) v[k][t] = static_cast<float>(nxt[k][t]);
+    if (row + stride < T) load(row + stride);
+    auto norm = [&](const half8_t (&g)[CH], const half8_t (&b)[CH], bool round_fp16) __attribute__((always_inline)) {
       float s = 0.f;
 #pragma unroll
       for (int k = 0; k < CH; ++k)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) s += v[k][t];
-      s = wave_sum(s);
-      const float mean = s * inv_c;
+        for (int t = 0; t < 8; ++t) s += v[k][t];
+      const float mean = half_sum(s) * inv_c;
       float q = 0.f;
 #pragma unroll
       for (int k = 0; k < CH; ++k)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const float d = k < nch ? v[k][t] - mean : 0.f;
-          q += d * d;
+        for (int t = 0; t < 8; ++t) {
+          v[k][t] = v[k][t] - mean;
+          q = __builtin_fmaf(v[k][t], v[k][t], q);
         }
-      q = wave_sum(q);
-      const float rstd = 1.f / sqrtf(q * inv_c + eps);
+      const float rstd = 1.f / sqrtf(half_sum(q) * inv_c + eps);
 #pragma unroll
       for (int k = 0; k < CH; ++k)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const float y = (v[k][t] - mean) * rstd * static_cast<float>(g[k][t]) + static_cast<float>(b[k][t]);
+        for (int t = 0; t < 8; ++t) {
+          const float y = __builtin_fmaf(v[k][t] * rstd, static_cast<float>(g[k][t]), static_cast<float>(b[k][t]));
           v[k][t] = round_fp16 ? static_cast<float>(static_cast<half_t>(y)) : y;
         }
     };
     norm(ga, ba, true);
     norm(gb, bb, false);
-    half_t* orow = out + row * C;
 #pragma unroll
-    for (int k = 0; k < CH; ++k)
-      if (k < nch) {
-        half4_t h;
+    for (int k = 0; k < CH; ++k) {
+      half8_t h;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) h[t] = static_cast<half_t>(v[k][t]);
-        *reinterpret_cast<half4_t*>(orow + 4 * (lane + 64 * k)) = h;
-      }
+      for (int t = 0; t < 8; ++t) h[t] = static_cast<half_t>(v[k][t]);
+      *reinterpret_cast<half8_t*>(out + row * C + 8 * (lane + 32 * k)) = h;
+    }
   }
 }
 
@@ -244,13 +244,17 @@ extern "C" int ff_layer_norm2(const void* x, int64_t T, int64_t C, const void* g
   const auto *pg2 = static_cast<const half_t*>(g2), *pb2 = static_cast<const half_t*>(b2);
   auto* po = static_cast<half_t*>(out);
   const int Ci = static_cast<int>(C);
-  const auto aligned8 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
-  const bool vec = C % 256 == 0 && C <= 1024 && aligned8(x) && aligned8(g1) && aligned8(b1) && aligned8(g2) &&
-                   aligned8(b2) && aligned8(out);
+  const auto aligned16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool vec = C % 256 == 0 && C <= 1024 && aligned16(x) && aligned16(g1) && aligned16(b1) && aligned16(g2) &&
+                   aligned16(b2) && aligned16(out);
   if (vec) {
-    // a few waves per SIMD stream the rows, so the affine vectors are loaded once per wave
-    const dim3 vgrid(static_cast<unsigned>(std::min<int64_t>((T + 3) / 4, 2048)));
-    layer_norm2_vec_kernel<4><<<vgrid, 256, 0, st>>>(px, T, Ci, pg1, pb1, pg2, pb2, eps, po);
+    const dim3 vgrid(static_cast<unsigned>(std::min<int64_t>((T + 7) / 8, 1024)));  // rows past that are streamed
+    switch (C / 256) {
+      case 1: layer_norm2_vec_kernel<1><<<vgrid, 256, 0, st>>>(px, T, pg1, pb1, pg2, pb2, eps, po); break;
+      case 2: layer_norm2_vec_kernel<2><<<vgrid, 256, 0, st>>>(px, T, pg1, pb1, pg2, pb2, eps, po); break;
+      case 3: layer_norm2_vec_kernel<3><<<vgrid, 256, 0, st>>>(px, T, pg1, pb1, pg2, pb2, eps, po); break;
+      default: layer_norm2_vec_kernel<4><<<vgrid, 256, 0, st>>>(px, T, pg1, pb1, pg2, pb2, eps, po); break;
+    }
   } else if (C <= 768) {
     layer_norm2_kernel<12><<<grid, 256, 0, st>>>(px, T, Ci, pg1, pb1, pg2, pb2, eps, po);
   } else {

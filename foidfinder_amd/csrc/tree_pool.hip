@@ -24,83 +24,99 @@ __device__ __forceinline__ void to_lds(const void* base, int nbytes, void* lds_d
 
 constexpr int PW_TOK = 64;  // tokens per workgroup of pool_weights
 
-// Grid (token blocks of 64, batch), 8 waves. Logits of the block's tokens against all GM = G M query columns: u [GM, D]
-// and xn stream through two LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
-// conflict-free fragment reads) filled by buffer->LDS loads; rows past GM or the sequence read as zeros. Wave w takes
-// the 32 tokens of half w & 1 and the 32-query tiles w / 2, w / 2 + 4, ... (queries as MFMA rows, tokens as columns). The
-// fp32 logits go to LDS as [GM][64 + 1]; a thread then turns the M logits of a (token, head) pair into weights in place:
-// softmax over the queries times sigmoid(logit + bias), from the hardware exp2 and reciprocal (each about 1 ulp). Tokens
-// past the sequence get weight 0. partial[b, block, j] is column j's sum over the block's tokens, a_t[b, j, n] the weight
-// in fp16 (rows of ldt; a row's pad column may be written with 0).
-// GMAX bounds GM: at 288 (Haruka's 16 heads x 18 leaves) 75 KB of LDS let two workgroups share a CU.
-template <int M, int GMAX>
-__global__ __launch_bounds__(512, GMAX <= 288 ? 4 : 2) void pool_weights_kernel(
+// A workgroup per (batch, block of 64 tokens). Logits of the block's tokens against all GM = G M query columns: u [GM, D] and xn
+// stream through three LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
+// conflict-free fragment reads) filled by buffer->LDS loads, two slots ahead; rows past GM or the sequence read as
+// zeros. A wave takes one 32-query tile (MFMA rows) and NT of the block's two 32-token tiles (MFMA columns): nine waves
+// of two at Haruka's 288 leaf columns, six of one at its 96 coarse columns. The fp32 logits go to LDS as [GM][64 + 1]; a
+// thread then turns the M logits of a (token, head) pair into weights in place: softmax over the queries times
+// sigmoid(logit + bias), from the hardware exp2 and reciprocal (each about 1 ulp). Tokens past the sequence get weight 0.
+// partial[b, block, j] is column j's sum over the block's tokens, a_t[b, j, n] the weight in fp16 (rows of ldt; a row's
+// pad column may be written with 0). GMAX bounds GM: at 288, 75 KB of LDS let two workgroups share a CU.
+template <int GMAX, int NT>
+constexpr int pw_waves() {
+  return GMAX / 32 * (PW_TOK / 32 / NT);
+}
+template <int M, int GMAX, int NT>
+__global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kernel(
     const half_t* __restrict__ xn, const half_t* __restrict__ u, int64_t u_stride, const float* __restrict__ c,
     int64_t c_stride, const float* __restrict__ bias, int N, int G, int D, int ldt, half_t* __restrict__ a_t,
     float* __restrict__ partial) {
-  constexpr int CT = (GMAX + 127) / 128;          // 32-query tiles per wave
-  constexpr int ROWS = 128 * CT + PW_TOK;         // staged rows: queries, then tokens
-  constexpr int SLOT = ROWS * 64;
+  constexpr int WV = pw_waves<GMAX, NT>(), THREADS = 64 * WV;
+  constexpr int LOADS = (GMAX + PW_TOK) / 16;     // 1 KB loads per slot: 16 rows each, queries, then tokens
+  constexpr int PER = (LOADS + WV - 1) / WV;      // per wave, the last only in waves below LOADS % WV (0: all)
+  constexpr int SLOT = LOADS * 1024, SLOTS = 3;
   constexpr int LDT = PW_TOK + 1;
-  constexpr int BYTES = 2 * SLOT > GMAX * LDT * 4 ? 2 * SLOT : GMAX * LDT * 4;
+  constexpr int BYTES = SLOTS * SLOT > GMAX * LDT * 4 ? SLOTS * SLOT : GMAX * LDT * 4;
   constexpr float LOG2E = 1.4426950408889634f;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[BYTES];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int GM = G * M, b = blockIdx.y, n0 = blockIdx.x * PW_TOK;
+  // 1-D grid over (batch, token block), remapped so that a batch's blocks share one XCD's L2 for its u
+  const int blocks = (N + PW_TOK - 1) / PW_TOK, t = xcd_remap(blockIdx.x, gridDim.x);
+  const int GM = G * M, b = t / blocks, blk = t % blocks, n0 = blk * PW_TOK;
   const int ntok = min(PW_TOK, N - n0);
   const half_t* ub = u + b * u_stride;
   const half_t* xb = xn + (static_cast<int64_t>(b) * N + n0) * D;
   const int u_bytes = GM * D * 2, x_bytes = ntok * D * 2;
+  const bool full = wave + WV * (PER - 1) < LOADS;  // this wave issues PER loads per slot, else PER - 1
 
-  auto issue = [&](int kc, int slot) __attribute__((always_inline)) {
-    uint8_t* dst = lds + slot * SLOT;
+  auto issue = [&](int kc) __attribute__((always_inline)) {
+    uint8_t* dst = lds + kc % SLOTS * SLOT;
 #pragma unroll
-    for (int p = 0; p < CT; ++p) {
-      const int q = wave + 8 * p, row = 16 * q + (lane >> 2);
-      to_lds(ub, u_bytes, dst + q * 1024, static_cast<uint32_t>(row * D * 2 + kc * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)));
-    }
-    if (wave < PW_TOK / 16) {
-      const int row = 16 * wave + (lane >> 2);
-      to_lds(xb, x_bytes, dst + 128 * CT * 64 + wave * 1024,
+    for (int p = 0; p < PER; ++p) {
+      const int q = wave + WV * p;  // wave-uniform
+      if (p == PER - 1 && !full) break;
+      const bool tok = q >= GMAX / 16;
+      const int row = 16 * q + (lane >> 2) - (tok ? GMAX : 0);
+      to_lds(tok ? xb : ub, tok ? x_bytes : u_bytes, dst + q * 1024,
              static_cast<uint32_t>(row * D * 2 + kc * 64 + (((lane & 3) ^ ((row >> 2) & 3)) << 4)));
     }
   };
   auto frag = [&](const uint8_t* base, int row, int chunk) __attribute__((always_inline)) {
     return *reinterpret_cast<const half8_t*>(base + row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4));
   };
-  const int rt = wave & 1, cg = wave >> 1, fr = lane & 31, fh = lane >> 5;
-  float16_t acc[CT] = {};
-  const int chunks = D / 32;
-  issue(0, 0);
+  const int qt = NT == 2 ? wave : wave >> 1, t0 = NT == 2 ? 0 : wave & 1, fr = lane & 31, fh = lane >> 5;
+  float16_t acc[NT] = {};
+  const int chunks = D / 32;  // at least four (D % 128 == 0)
+  issue(0);
+  issue(1);
   for (int kc = 0; kc < chunks; ++kc) {
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();  // slot kc has landed; every wave has read slot kc - 1
+    // slot kc has landed once only slot kc + 1's loads are outstanding
+    if (kc + 1 == chunks)
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else if (full)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER - 1) : "memory");
+    __builtin_amdgcn_s_barrier();  // and every wave has read slot kc - 1, which slot kc + 2 takes over
     asm volatile("" ::: "memory");
-    if (kc + 1 < chunks) issue(kc + 1, (kc + 1) & 1);
-    const uint8_t* su = lds + (kc & 1) * SLOT;
-    const uint8_t* sx = su + 128 * CT * 64;
+    const uint8_t* su = lds + kc % SLOTS * SLOT;
+    const uint8_t* sx = su + GMAX * 64;
+    half8_t uf[2], xf[2][NT];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      const half8_t xf = frag(sx, 32 * rt + fr, 2 * ks + fh);
+      uf[ks] = frag(su, 32 * qt + fr, 2 * ks + fh);
 #pragma unroll
-      for (int i = 0; i < CT; ++i) {
-        if (32 * (cg + 4 * i) >= GM) continue;  // wave-uniform
-        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag(su, 32 * (cg + 4 * i) + fr, 2 * ks + fh), xf, acc[i], 0, 0, 0);
-      }
+      for (int i = 0; i < NT; ++i) xf[ks][i] = frag(sx, 32 * (t0 + i) + fr, 2 * ks + fh);
     }
+    if (kc + 2 < chunks) issue(kc + 2);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(uf[ks], xf[ks][i], acc[i], 0, 0, 0);
   }
   __syncthreads();  // the slots are read: the logits take their place
   float* tile = reinterpret_cast<float*>(lds);
 #pragma unroll
-  for (int i = 0; i < CT; ++i)
+  for (int i = 0; i < NT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int j = 32 * (cg + 4 * i) + 8 * (r >> 2) + 4 * fh + (r & 3);
-      if (j < GM) tile[j * LDT + 32 * rt + fr] = acc[i][r];
+      const int j = 32 * qt + 8 * (r >> 2) + 4 * fh + (r & 3);
+      if (j < GM) tile[j * LDT + 32 * (t0 + i) + fr] = acc[i][r];
     }
   const float* cb = c + b * c_stride;
   __syncthreads();
-  for (int p = threadIdx.x; p < PW_TOK * G; p += 512) {  // a wave's 64 lanes are the block's tokens, its head is uniform
+  for (int p = threadIdx.x; p < PW_TOK * G; p += THREADS) {  // a wave's 64 lanes are the block's tokens, its head is uniform
     const int t = p % PW_TOK, h = __builtin_amdgcn_readfirstlane(p / PW_TOK);
     float l[M], w[M], mx = -INFINITY, s = 0.f;
 #pragma unroll
@@ -121,16 +137,16 @@ __global__ __launch_bounds__(512, GMAX <= 288 ? 4 : 2) void pool_weights_kernel(
     }
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < GM; j += 512) {
+  for (int j = threadIdx.x; j < GM; j += THREADS) {
     float s = 0.f;
 #pragma unroll 8
     for (int t = 0; t < PW_TOK; ++t) s += tile[j * LDT + t];
-    partial[(static_cast<int64_t>(b) * gridDim.x + blockIdx.x) * GM + j] = s;
+    partial[(static_cast<int64_t>(b) * blocks + blk) * GM + j] = s;
   }
   // two query rows per wave and pass, two tokens (4 bytes) per lane; ldt is even, so a pair past an odd end is pad
   const int t2 = 2 * (lane & 31);
   if (t2 < ntok)
-    for (int j = 2 * wave + (lane >> 5); j < GM; j += 16)
+    for (int j = 2 * wave + (lane >> 5); j < GM; j += 2 * WV)
       *reinterpret_cast<half2_t*>(a_t + (static_cast<int64_t>(b) * GM + j) * ldt + n0 + t2) =
           half2_t{static_cast<half_t>(tile[j * LDT + t2]), static_cast<half_t>(tile[j * LDT + t2 + 1])};
 }
@@ -183,13 +199,29 @@ __global__ __launch_bounds__(256) void pool_values_kernel(const half_t* __restri
   *reinterpret_cast<half4_t*>(z + static_cast<int64_t>(r0 + (lane & 15)) * D + e) = o;
 }
 
-// LayerNorm of a row held two columns per lane and step, c = 2 (lane + 64 k), D <= 128 PER: v = (v - mean) rstd g + b.
+struct Norm {
+  const half_t *g, *b;
+};
+
+// Rows held two columns per lane and step, c = 2 (lane + 64 k), D <= 128 PER. The kernels load everything a row needs
+// (operands, affine vectors) before their first reduction, so one round trip covers all of it.
 template <int PER>
-__device__ __forceinline__ void norm_row(float (&v)[PER][2], int D, const half_t* g, const half_t* b, float eps) {
+__device__ __forceinline__ void load_pairs(half2_t (&x)[PER], const half_t* row, int D) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int c = 2 * (lane + 64 * k);
+    x[k] = c < D ? *reinterpret_cast<const half2_t*>(row + c) : half2_t{};
+  }
+}
+// LayerNorm: v = (v - mean) rstd g + b. Columns past D hold zeros.
+template <int PER>
+__device__ __forceinline__ void norm_row(float (&v)[PER][2], int D, const half2_t (&g)[PER], const half2_t (&b)[PER],
+                                         float eps) {
   const int lane = threadIdx.x & 63;
   float s = 0.f, q = 0.f;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) s += v[k][0] + v[k][1];  // columns past D hold zeros
+  for (int k = 0; k < PER; ++k) s += v[k][0] + v[k][1];
   const float mean = wave_sum(s) / static_cast<float>(D);
 #pragma unroll
   for (int k = 0; k < PER; ++k)
@@ -201,24 +233,11 @@ __device__ __forceinline__ void norm_row(float (&v)[PER][2], int D, const half_t
   const float rstd = 1.f / sqrtf(wave_sum(q) / static_cast<float>(D) + eps);
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const int c = 2 * (lane + 64 * k);
-    if (c < D) {
-      const half2_t gk = *reinterpret_cast<const half2_t*>(g + c), bk = *reinterpret_cast<const half2_t*>(b + c);
+    if (2 * (lane + 64 * k) < D) {
 #pragma unroll
       for (int e = 0; e < 2; ++e)
-        v[k][e] = (v[k][e] - mean) * rstd * static_cast<float>(gk[e]) + static_cast<float>(bk[e]);
+        v[k][e] = (v[k][e] - mean) * rstd * static_cast<float>(g[k][e]) + static_cast<float>(b[k][e]);
     }
-  }
-}
-template <int PER>
-__device__ __forceinline__ void load_row2(float (&v)[PER][2], const half_t* row, int D, bool add) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const int c = 2 * (lane + 64 * k);
-    const half2_t x = c < D ? *reinterpret_cast<const half2_t*>(row + c) : half2_t{};
-#pragma unroll
-    for (int e = 0; e < 2; ++e) v[k][e] = (add ? v[k][e] : 0.f) + static_cast<float>(x[e]);
   }
 }
 template <int PER>
@@ -231,10 +250,6 @@ __device__ __forceinline__ void store_row2(const float (&v)[PER][2], half_t* row
   }
 }
 
-struct Norm {
-  const half_t *g, *b;
-};
-
 // One wave per (batch, leaf q): its parent is coarse query m = q C / Q. parent[b, m] = LN(z[b, m]; trunk), qleaf[b, q] =
 // LN(parent + child[q]; childn), cq[b, h Q + q] = sum over head h's columns of qleaf bk (the keys' bias term).
 template <int PER>
@@ -245,29 +260,46 @@ __global__ __launch_bounds__(64) void pool_queries_kernel(const half_t* __restri
                                                           float* __restrict__ cq) {
   __shared__ float prod[128 * PER];
   const int q = blockIdx.x, b = blockIdx.y, lane = threadIdx.x, m = q / (Q / C), hd = D / G;
-  float v[PER][2];
-  load_row2(v, z + (static_cast<int64_t>(b) * C + m) * D, D, false);
-  norm_row(v, D, trunk.g, trunk.b, eps);
+  half2_t x[PER], ch[PER], tg[PER], tb[PER], cg[PER], cb[PER];
+  load_pairs(x, z + (static_cast<int64_t>(b) * C + m) * D, D);
+  load_pairs(tg, trunk.g, D);
+  load_pairs(tb, trunk.b, D);
+  load_pairs(ch, child + static_cast<int64_t>(q) * D, D);
+  load_pairs(cg, childn.g, D);
+  load_pairs(cb, childn.b, D);
+  float v[PER][2], kb[PER][2];
 #pragma unroll
   for (int k = 0; k < PER; ++k)
 #pragma unroll
-    for (int e = 0; e < 2; ++e) v[k][e] = static_cast<float>(static_cast<half_t>(v[k][e]));  // as the stored parent
+    for (int e = 0; e < 2; ++e) {
+      v[k][e] = static_cast<float>(x[k][e]);
+      kb[k][e] = 2 * (lane + 64 * k) < D ? bk[2 * (lane + 64 * k) + e] : 0.f;
+    }
+  norm_row(v, D, tg, tb, eps);
   if (q % (Q / C) == 0) store_row2(v, parent + (static_cast<int64_t>(b) * C + m) * D, D);
-  load_row2(v, child + static_cast<int64_t>(q) * D, D, true);
-  norm_row(v, D, childn.g, childn.b, eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+#pragma unroll
+    for (int e = 0; e < 2; ++e)  // the parent as stored
+      v[k][e] = static_cast<float>(static_cast<half_t>(v[k][e])) + static_cast<float>(ch[k][e]);
+  norm_row(v, D, cg, cb, eps);
   store_row2(v, qleaf + (static_cast<int64_t>(b) * Q + q) * D, D);
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int c = 2 * (lane + 64 * k);
 #pragma unroll
     for (int e = 0; e < 2; ++e)
-      if (c < D) prod[c + e] = static_cast<float>(static_cast<half_t>(v[k][e])) * bk[c + e];
+      if (c < D) prod[c + e] = static_cast<float>(static_cast<half_t>(v[k][e])) * kb[k][e];
   }
   __syncthreads();
-  for (int h = lane; h < G; h += 64) {
+  for (int h0 = 0; h0 < G; h0 += 16) {  // four lanes per head
+    const int h = h0 + (lane >> 2);
     float s = 0.f;
-    for (int e = 0; e < hd; ++e) s += prod[h * hd + e];
-    cq[(static_cast<int64_t>(b) * G + h) * Q + q] = s;
+    if (h < G)
+      for (int e = lane & 3; e < hd; e += 4) s += prod[h * hd + e];
+    s = s + dpp<DPP_XOR3>(s);
+    s = s + dpp<DPP_XOR1>(s);
+    if (h < G && (lane & 3) == 0) cq[(static_cast<int64_t>(b) * G + h) * Q + q] = s;
   }
 }
 
@@ -282,6 +314,7 @@ __global__ __launch_bounds__(256) void pool_keys_kernel(const half_t* __restrict
   const int r = min(r0 + i16, R - 1);
   const half_t* pq = qleaf + static_cast<int64_t>(r) * D + h * hd + 4 * kq;
   float4_t acc[4] = {};
+#pragma unroll 3
   for (int k = 0; k < hd; k += 16) {
     const half4_t x = *reinterpret_cast<const half4_t*>(pq + k);
 #pragma unroll
@@ -310,13 +343,21 @@ __global__ __launch_bounds__(64) void pool_tree_kernel(const half_t* __restrict_
                                                        Norm leafn, const float* __restrict__ partial, int nblk, float eps,
                                                        int C, int Q, int G, int D, half_t* __restrict__ tree) {
   const int q = blockIdx.x, b = blockIdx.y, B = gridDim.y, lane = threadIdx.x;
+  half2_t x[PER], y[PER], g[PER], be[PER];
+  load_pairs(x, parent + (static_cast<int64_t>(b) * C + q / (Q / C)) * D, D);
+  load_pairs(y, zc + (static_cast<int64_t>(b) * Q + q) * D, D);
+  load_pairs(g, leafn.g, D);
+  load_pairs(be, leafn.b, D);
   float s = 0.f;
+#pragma unroll 5
   for (int i = lane; i < nblk * G; i += 64) s += partial[(static_cast<int64_t>(b) * nblk * G + i) * Q + q];
   const float mass = wave_sum(s) / static_cast<float>(G);
   float v[PER][2];
-  load_row2(v, parent + (static_cast<int64_t>(b) * C + q / (Q / C)) * D, D, false);
-  load_row2(v, zc + (static_cast<int64_t>(b) * Q + q) * D, D, true);
-  norm_row(v, D, leafn.g, leafn.b, eps);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[k][e] = static_cast<float>(x[k][e]) + static_cast<float>(y[k][e]);
+  norm_row(v, D, g, be, eps);
   const float gate = mass / (mass + 4.f);
 #pragma unroll
   for (int k = 0; k < PER; ++k)
@@ -374,21 +415,24 @@ extern "C" int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, 
   if (B == 0) return FF_OK;
   if (!xn || !u || !c || !bias || !a_t || !partial) return fail(FF_EINVAL, "pool_weights: null pointer");
   if (!al(xn, 16) || !al(u, 16) || !al(a_t, 4)) return fail(FF_EINVAL, "pool_weights: misaligned pointer");
-  const dim3 grid(static_cast<unsigned>(ff_pool_weights_blocks(N)), static_cast<unsigned>(B));
+  const int64_t blocks = ff_pool_weights_blocks(N) * B;
+  if (blocks > 0x7fffffff) return fail(FF_EINVAL, "pool_weights: too many token blocks");
+  const dim3 grid(static_cast<unsigned>(blocks));
   const hipStream_t st = as_stream(stream);
   const auto *px = static_cast<const half_t*>(xn), *pu = static_cast<const half_t*>(u);
   auto* pa = static_cast<half_t*>(a_t);
   const int Ni = static_cast<int>(N), Gi = static_cast<int>(G), Di = static_cast<int>(D), li = static_cast<int>(ldt);
-#define FF_PW(MM, GMAX) \
-  pool_weights_kernel<MM, GMAX><<<grid, 512, 0, st>>>(px, pu, u_stride, c, c_stride, bias, Ni, Gi, Di, li, pa, partial)
+#define FF_PW(MM, GMAX, NT)                                                                                           \
+  pool_weights_kernel<MM, GMAX, NT><<<grid, 64 * (pw_waves<GMAX, NT>()), 0, st>>>(px, pu, u_stride, c, c_stride, bias, \
+                                                                                  Ni, Gi, Di, li, pa, partial)
   if (M == 6 && G * M <= 96)
-    FF_PW(6, 96);
+    FF_PW(6, 96, 1);
   else if (M == 6)
-    FF_PW(6, 512);
+    FF_PW(6, 512, 2);
   else if (G * M <= 288)
-    FF_PW(18, 288);
+    FF_PW(18, 288, 2);
   else
-    FF_PW(18, 512);
+    FF_PW(18, 512, 2);
 #undef FF_PW
   return check_launch("pool_weights");
 }
