@@ -75,8 +75,16 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+def _run(name: str, dev: int, *args) -> None:
+    """Calls a launching function of the library on device `dev`'s current stream, with that device current. A call is
+    made of a few us of host work in all, so nothing is switched or built that is not needed: the device is entered only
+    if it is not the current one already, and the stream comes as its raw handle."""
+    fn = getattr(lib(), name)
+    if torch.cuda.current_device() == dev:
+        _check(fn(*args, torch._C._cuda_getCurrentRawStream(dev)))
+        return
+    with torch.cuda.device(dev):
+        _check(fn(*args, torch._C._cuda_getCurrentRawStream(dev)))
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -84,15 +92,22 @@ def _require(cond: bool, msg: str) -> None:
         raise RuntimeError(msg)
 
 
-def _on_gpu(*ts: torch.Tensor | None) -> None:
-    dev = None
+def _on_gpu(*ts: torch.Tensor | None) -> int:
+    """The device index of contiguous tensors that are all on one GPU."""
+    dev = -1
     for t in ts:
         if t is None:
             continue
-        _require(t.is_cuda, "foidfinder_rocm ops take GPU tensors")
-        _require(t.is_contiguous(), "foidfinder_rocm ops take contiguous tensors")
-        dev = dev or t.device
-        _require(t.device == dev, "all tensors must be on one device")
+        if not t.is_cuda:
+            raise RuntimeError("foidfinder_rocm ops take GPU tensors")
+        if not t.is_contiguous():
+            raise RuntimeError("foidfinder_rocm ops take contiguous tensors")
+        d = t.get_device()
+        if dev < 0:
+            dev = d
+        elif d != dev:
+            raise RuntimeError("all tensors must be on one device")
+    return dev
 
 
 # ---- op implementations (raw; also callable directly, bypassing the dispatcher) ----
@@ -107,7 +122,7 @@ def rot_q8_1024(
     eps: float = 1e-5,
 ) -> None:
     """x fp16 [T, 1024] -> out int8 [T, 1024], row_scale fp32 [T]; LayerNorm(gamma, beta, eps) first if given."""
-    _on_gpu(x, gamma, beta, out, row_scale)
+    dev = _on_gpu(x, gamma, beta, out, row_scale)
     _require(x.dim() == 2 and x.size(1) == 1024 and x.dtype == torch.float16, "x must be fp16 [T, 1024]")
     _require(out.dtype == torch.int8 and out.shape == x.shape, "out must be int8 [T, 1024]")
     _require(row_scale.dtype == torch.float32 and row_scale.numel() == x.size(0), "row_scale must be fp32 [T]")
@@ -115,9 +130,7 @@ def rot_q8_1024(
         _require(beta is not None, "gamma and beta go together")
         _require(gamma.dtype == beta.dtype == torch.float32 and gamma.numel() == beta.numel() == 1024,
                  "gamma/beta must be fp32 [1024]")
-    with torch.cuda.device(x.device):
-        _check(lib().ff_rot_q8_1024(_ptr(x), _ptr(gamma), _ptr(beta), eps, x.size(0), _ptr(out), _ptr(row_scale),
-                                    _stream(x)))
+    _run("ff_rot_q8_1024", dev, _ptr(x), _ptr(gamma), _ptr(beta), eps, x.size(0), _ptr(out), _ptr(row_scale))
 
 
 def rot_q8_h128(
@@ -132,7 +145,7 @@ def rot_q8_h128(
     """x fp16 [T, C] (C % 128 == 0) -> out int8 [T, C], row_scale fp32 [T]; LayerNorm over the first c_real columns
     (default: all) first if gamma is given. gamma/beta are fp32 [C] with zeros in columns >= c_real
     (`pad_norm` builds them)."""
-    _on_gpu(x, out, row_scale, gamma, beta)
+    dev = _on_gpu(x, out, row_scale, gamma, beta)
     _require(x.dim() == 2 and x.dtype == torch.float16, "x must be fp16 [T, C]")
     _require(out.dtype == torch.int8 and out.shape == x.shape, "out must be int8 [T, C]")
     _require(row_scale.dtype == torch.float32 and row_scale.numel() == x.size(0), "row_scale must be fp32 [T]")
@@ -142,9 +155,7 @@ def rot_q8_h128(
         _require(beta is not None, "gamma and beta go together")
         _require(gamma.dtype == beta.dtype == torch.float32 and gamma.numel() == beta.numel() == C,
                  "gamma/beta must be fp32 [C], zero past c_real")
-    with torch.cuda.device(x.device):
-        _check(lib().ff_rot_q8_h128(_ptr(x), x.size(0), C, cr, _ptr(gamma), _ptr(beta), eps, _ptr(out),
-                                    _ptr(row_scale), _stream(x)))
+    _run("ff_rot_q8_h128", dev, _ptr(x), x.size(0), C, cr, _ptr(gamma), _ptr(beta), eps, _ptr(out), _ptr(row_scale))
 
 
 def pad_norm(weight: torch.Tensor, bias: torch.Tensor, C: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -175,13 +186,15 @@ def gemm_s8(
 ) -> None:
     """A int8 [M, K] x W int8 [N, K] -> epilogue into out. `stages` selects the tile variant (0 = default), the
     knob the engine autotunes (the reference's pipeline depth)."""
-    _on_gpu(A, W, row_scale, col_scale, bias, out, rope_cos, rope_sin)
+    dev = _on_gpu(A, W, row_scale, col_scale, bias, out, rope_cos, rope_sin)
     _require(A.dtype == W.dtype == torch.int8 and A.dim() == W.dim() == 2, "A and W must be int8 matrices")
     M, K = A.shape
     N = W.size(0)
     _require(W.size(1) == K, "A and W must share K")
     want = torch.int32 if epi == EPI_I32 else torch.float16
-    _require(out.dtype == want and tuple(out.shape) == out_shape(M, N, epi), f"out must be {want} {out_shape(M, N, epi)}")
+    shape = out_shape(M, N, epi)
+    if out.dtype != want or tuple(out.shape) != shape:
+        raise RuntimeError(f"out must be {want} {shape}")
     if epi != EPI_I32:
         _require(row_scale.dtype == col_scale.dtype == bias.dtype == torch.float32, "scales and bias must be fp32")
         _require(row_scale.numel() == M and col_scale.numel() == N and bias.numel() == N, "scale/bias sizes")
@@ -191,27 +204,25 @@ def gemm_s8(
         _require(rope_cos.dtype == rope_sin.dtype == torch.float32 and rope_cos.shape == rope_sin.shape
                  and rope_cos.dim() == 2 and rope_cos.size(1) == 32, "RoPE tables must be fp32 [L, 32]")
         rope_len = rope_cos.size(0)
-    with torch.cuda.device(A.device):
-        _check(lib().ff_gemm_s8(_ptr(A), _ptr(W), M, N, K, _ptr(row_scale), _ptr(col_scale), _ptr(bias), _ptr(out),
-                                epi, stages, _ptr(rope_cos), _ptr(rope_sin), rope_len, q_scale, _stream(A)))
+    _run("ff_gemm_s8", dev, _ptr(A), _ptr(W), M, N, K, _ptr(row_scale), _ptr(col_scale), _ptr(bias), _ptr(out), epi,
+         stages, _ptr(rope_cos), _ptr(rope_sin), rope_len, q_scale)
 
 
 def attention(qkv: torch.Tensor, out: torch.Tensor, seq_len: int) -> None:
     """qkv fp16 [T, 3C] (q rotated and pre-scaled, k rotated) -> out fp16 [T, C]; heads of 64, any seq_len."""
-    _on_gpu(qkv, out)
+    dev = _on_gpu(qkv, out)
     _require(qkv.dtype == out.dtype == torch.float16, "qkv and out must be fp16")
     _require(qkv.dim() == 2 and qkv.size(1) % 192 == 0, "qkv must be [T, 3 * heads * 64]")
     C = qkv.size(1) // 3
     _require(out.shape == (qkv.size(0), C), "out must be [T, C]")
-    with torch.cuda.device(qkv.device):
-        _check(lib().ff_attention(_ptr(qkv), _ptr(out), qkv.size(0), C // 64, seq_len, _stream(qkv)))
+    _run("ff_attention", dev, _ptr(qkv), _ptr(out), qkv.size(0), C // 64, seq_len)
 
 
 def resample_u8(src: torch.Tensor, axis: int, kk: torch.Tensor, bounds: torch.Tensor, row0: int, out: torch.Tensor,
                 region: tuple[int, int, int, int]) -> None:
     """One Pillow resampling pass (include/foidfinder_rocm.h, ff_resample_u8): src uint8 [H, W, 3] -> out uint8
     [out_h, out_w, 3], `region` = (top, left, h, w) resampled along axis 0 (width) or 1 (height), the rest white."""
-    _on_gpu(src, kk, bounds, out)
+    dev = _on_gpu(src, kk, bounds, out)
     _require(src.dtype == out.dtype == torch.uint8 and src.dim() == out.dim() == 3 and src.size(2) == out.size(2) == 3,
              "src and out must be uint8 [rows, cols, 3]")
     _require(src.is_contiguous() and out.is_contiguous(), "src and out must be contiguous")
@@ -220,36 +231,31 @@ def resample_u8(src: torch.Tensor, axis: int, kk: torch.Tensor, bounds: torch.Te
     top, left, h, w = region
     n = w if axis == 0 else h
     _require(kk.size(0) >= n and bounds.size(0) >= n, "kk/bounds need a row per output index of the region")
-    with torch.cuda.device(src.device):
-        _check(lib().ff_resample_u8(_ptr(src), src.size(0), src.size(1), axis, _ptr(kk), _ptr(bounds), kk.size(1),
-                                    row0, _ptr(out), out.size(0), out.size(1), top, left, h, w, _stream(src)))
+    _run("ff_resample_u8", dev, _ptr(src), src.size(0), src.size(1), axis, _ptr(kk), _ptr(bounds), kk.size(1), row0,
+         _ptr(out), out.size(0), out.size(1), top, left, h, w)
 
 
 def bicubic_taps(width: tuple[int, int, int], height: tuple[int, int, int], kk_w: torch.Tensor, bounds_w: torch.Tensor,
                  kk_h: torch.Tensor, bounds_h: torch.Tensor) -> None:
     """Pillow's bicubic taps of both axes (include/foidfinder_rocm.h, ff_bicubic_taps): `width` and `height` are (input
     size, output size, shift); kk int32 [output size, ksize], bounds int32 [output size, 2]."""
-    _on_gpu(kk_w, bounds_w, kk_h, bounds_h)
+    dev = _on_gpu(kk_w, bounds_w, kk_h, bounds_h)
     for (_, n, _), kk, bounds in ((width, kk_w, bounds_w), (height, kk_h, bounds_h)):
         _require(kk.dtype == bounds.dtype == torch.int32 and kk.dim() == 2 and kk.size(0) == n
                  and tuple(bounds.shape) == (n, 2), "kk int32 [n, ksize], bounds int32 [n, 2]")
-    with torch.cuda.device(kk_w.device):
-        _check(lib().ff_bicubic_taps(width[0], width[1], kk_w.size(1), _ptr(kk_w), _ptr(bounds_w), width[2],
-                                     height[0], height[1], kk_h.size(1), _ptr(kk_h), _ptr(bounds_h), height[2],
-                                     _stream(kk_w)))
+    _run("ff_bicubic_taps", dev, width[0], width[1], kk_w.size(1), _ptr(kk_w), _ptr(bounds_w), width[2], height[0],
+         height[1], kk_h.size(1), _ptr(kk_h), _ptr(bounds_h), height[2])
 
 
 def layer_norm2(x: torch.Tensor, g1: torch.Tensor, b1: torch.Tensor, g2: torch.Tensor, b2: torch.Tensor, eps: float,
                 out: torch.Tensor) -> None:
     """out = LN(fp16(LN(x; g1, b1)); g2, b2) over the last dimension of fp16 x [..., C] (fp16 params [C])."""
-    _on_gpu(x, g1, b1, g2, b2, out)
+    dev = _on_gpu(x, g1, b1, g2, b2, out)
     C = x.size(-1)
     _require(x.dtype == out.dtype == torch.float16 and x.is_contiguous() and out.is_contiguous()
              and out.shape == x.shape, "x and out must be contiguous fp16 of one shape")
     _require(all(t.dtype == torch.float16 and t.numel() == C for t in (g1, b1, g2, b2)), "params must be fp16 [C]")
-    with torch.cuda.device(x.device):
-        _check(lib().ff_layer_norm2(_ptr(x), x.numel() // C, C, _ptr(g1), _ptr(b1), _ptr(g2), _ptr(b2), eps, _ptr(out),
-                                    _stream(x)))
+    _run("ff_layer_norm2", dev, _ptr(x), x.numel() // C, C, _ptr(g1), _ptr(b1), _ptr(g2), _ptr(b2), eps, _ptr(out))
 
 
 def slot_weights_blocks(N: int) -> int:
@@ -260,7 +266,7 @@ def slot_weights(logits: torch.Tensor, c: torch.Tensor, bias: torch.Tensor, head
                  partial: torch.Tensor) -> None:
     """Tree-pool weights (include/foidfinder_rocm.h, ff_slot_weights): logits fp16 [B, N, heads*M] + c fp32 ([heads*M]
     shared or [B, heads*M]) -> a_t fp16 [B, heads*M, N], partial fp32 [B, blocks, heads*M]."""
-    _on_gpu(logits, c, bias, a_t, partial)
+    dev = _on_gpu(logits, c, bias, a_t, partial)
     B, N, GM = logits.shape
     M = bias.numel()
     _require(logits.dtype == torch.float16 and logits.is_contiguous() and GM == heads * M, "logits fp16 [B, N, heads*M]")
@@ -269,9 +275,8 @@ def slot_weights(logits: torch.Tensor, c: torch.Tensor, bias: torch.Tensor, head
     _require(a_t.dtype == torch.float16 and a_t.is_contiguous() and a_t.shape == (B, GM, N), "a_t fp16 [B, heads*M, N]")
     _require(partial.dtype == torch.float32 and partial.is_contiguous()
              and partial.shape == (B, slot_weights_blocks(N), GM), "partial fp32 [B, blocks, heads*M]")
-    with torch.cuda.device(logits.device):
-        _check(lib().ff_slot_weights(_ptr(logits), _ptr(c), 0 if c.numel() == GM else GM, _ptr(bias), B, N, heads, M,
-                                     _ptr(a_t), _ptr(partial), _stream(logits)))
+    _run("ff_slot_weights", dev, _ptr(logits), _ptr(c), 0 if c.numel() == GM else GM, _ptr(bias), B, N, heads, M,
+         _ptr(a_t), _ptr(partial))
 
 
 def pool_weights_blocks(N: int) -> int:
@@ -280,12 +285,14 @@ def pool_weights_blocks(N: int) -> int:
 
 def _half(shape: tuple, *ts: torch.Tensor) -> None:
     for t in ts:
-        _require(t.dtype == torch.float16 and tuple(t.shape) == tuple(shape), f"need fp16 {tuple(shape)}")
+        if t.dtype != torch.float16 or tuple(t.shape) != shape:
+            raise RuntimeError(f"need fp16 {shape}")
 
 
 def _float(numel: int, *ts: torch.Tensor) -> None:
     for t in ts:
-        _require(t.dtype == torch.float32 and t.numel() == numel, f"need fp32 of {numel} elements")
+        if t.dtype != torch.float32 or t.numel() != numel:
+            raise RuntimeError(f"need fp32 of {numel} elements")
 
 
 def pool_weights(xn: torch.Tensor, u: torch.Tensor, c: torch.Tensor, bias: torch.Tensor, heads: int, a_t: torch.Tensor,
@@ -293,7 +300,7 @@ def pool_weights(xn: torch.Tensor, u: torch.Tensor, c: torch.Tensor, bias: torch
     """Tree-pool weights from the tokens and the queries' u (include/foidfinder_rocm.h, ff_pool_weights): xn fp16
     [B, N, D], u fp16 [heads*M, D] (shared) or [B, heads*M, D], c fp32 [heads*M] or [B, heads*M], bias fp32 [M] -> a_t
     fp16 [B, heads*M, ldt], partial fp32 [B, blocks, heads*M]."""
-    _on_gpu(xn, u, c, bias, a_t, partial)
+    dev = _on_gpu(xn, u, c, bias, a_t, partial)
     B, N, D = xn.shape
     M = bias.numel()
     GM = heads * M
@@ -302,31 +309,29 @@ def pool_weights(xn: torch.Tensor, u: torch.Tensor, c: torch.Tensor, bias: torch
     _require(c.dtype == bias.dtype == torch.float32 and c.numel() in (GM, B * GM), "c must be fp32 [heads*M] or [B, heads*M]")
     _half((B, GM, a_t.size(-1)), a_t)
     _float(B * pool_weights_blocks(N) * GM, partial)
-    with torch.cuda.device(xn.device):
-        _check(lib().ff_pool_weights(_ptr(xn), _ptr(u), 0 if u.dim() == 2 else GM * D, _ptr(c), 0 if c.numel() == GM else GM,
-                                     _ptr(bias), B, N, heads, M, D, a_t.size(-1), _ptr(a_t), _ptr(partial), _stream(xn)))
+    _run("ff_pool_weights", dev, _ptr(xn), _ptr(u), 0 if u.dim() == 2 else GM * D, _ptr(c), 0 if c.numel() == GM else
+         GM, _ptr(bias), B, N, heads, M, D, a_t.size(-1), _ptr(a_t), _ptr(partial))
 
 
 def pool_values(pooled: torch.Tensor, wv: torch.Tensor, bv: torch.Tensor, partial: torch.Tensor, heads: int,
                 z: torch.Tensor) -> None:
     """z fp16 [B, M, D] from pooled fp16 [B, heads*M, D], wv fp16 [D, D], bv fp32 [D] and the weights' partial sums."""
-    _on_gpu(pooled, wv, bv, partial, z)
+    dev = _on_gpu(pooled, wv, bv, partial, z)
     B, M, D = z.shape
     _half((B, M, D), z)
     _half((B, heads * M, D), pooled)
     _half((D, D), wv)
     _float(D, bv)
     _float(B * partial.size(1) * heads * M, partial)
-    with torch.cuda.device(z.device):
-        _check(lib().ff_pool_values(_ptr(pooled), _ptr(wv), _ptr(bv), _ptr(partial), partial.size(1), B, heads, M, D,
-                                    _ptr(z), _stream(z)))
+    _run("ff_pool_values", dev, _ptr(pooled), _ptr(wv), _ptr(bv), _ptr(partial), partial.size(1), B, heads, M, D,
+         _ptr(z))
 
 
 def pool_queries(z: torch.Tensor, trunk_g: torch.Tensor, trunk_b: torch.Tensor, child: torch.Tensor,
                  child_g: torch.Tensor, child_b: torch.Tensor, bk: torch.Tensor, heads: int, eps: float,
                  parent: torch.Tensor, qleaf: torch.Tensor, cq: torch.Tensor) -> None:
     """z fp16 [B, C, D] -> parent fp16 [B, C, D], qleaf fp16 [B, Q, D], cq fp32 [B, heads*Q] (ff_pool_queries)."""
-    _on_gpu(z, trunk_g, trunk_b, child, child_g, child_b, bk, parent, qleaf, cq)
+    dev = _on_gpu(z, trunk_g, trunk_b, child, child_g, child_b, bk, parent, qleaf, cq)
     B, C, D = z.shape
     Q = child.size(0)
     _half((B, C, D), z, parent)
@@ -335,49 +340,45 @@ def pool_queries(z: torch.Tensor, trunk_g: torch.Tensor, trunk_b: torch.Tensor, 
     _half((D,), trunk_g, trunk_b, child_g, child_b)
     _float(D, bk)
     _float(B * heads * Q, cq)
-    with torch.cuda.device(z.device):
-        _check(lib().ff_pool_queries(_ptr(z), _ptr(trunk_g), _ptr(trunk_b), _ptr(child), _ptr(child_g), _ptr(child_b),
-                                     _ptr(bk), eps, B, C, Q, heads, D, _ptr(parent), _ptr(qleaf), _ptr(cq), _stream(z)))
+    _run("ff_pool_queries", dev, _ptr(z), _ptr(trunk_g), _ptr(trunk_b), _ptr(child), _ptr(child_g), _ptr(child_b),
+         _ptr(bk), eps, B, C, Q, heads, D, _ptr(parent), _ptr(qleaf), _ptr(cq))
 
 
 def pool_keys(qleaf: torch.Tensor, kT: torch.Tensor, u: torch.Tensor) -> None:
     """u fp16 [B, heads*Q, D] from qleaf fp16 [B, Q, D] and kT fp16 [heads, D, D / heads] (ff_pool_keys)."""
-    _on_gpu(qleaf, kT, u)
+    dev = _on_gpu(qleaf, kT, u)
     B, Q, D = qleaf.shape
     heads = kT.size(0)
     _half((B, Q, D), qleaf)
     _half((heads, D, D // heads), kT)
     _half((B, heads * Q, D), u)
-    with torch.cuda.device(u.device):
-        _check(lib().ff_pool_keys(_ptr(qleaf), _ptr(kT), B, Q, heads, D, _ptr(u), _stream(u)))
+    _run("ff_pool_keys", dev, _ptr(qleaf), _ptr(kT), B, Q, heads, D, _ptr(u))
 
 
 def pool_tree(parent: torch.Tensor, zc: torch.Tensor, g: torch.Tensor, b: torch.Tensor, partial: torch.Tensor,
               heads: int, eps: float, tree: torch.Tensor) -> None:
     """tree fp16 [Q, B, D] from parent fp16 [B, C, D], zc fp16 [B, Q, D] and the weights' partial sums (ff_pool_tree)."""
-    _on_gpu(parent, zc, g, b, partial, tree)
+    dev = _on_gpu(parent, zc, g, b, partial, tree)
     B, Q, D = zc.shape
     _half((B, parent.size(1), D), parent)
     _half((B, Q, D), zc)
     _half((D,), g, b)
     _half((Q, B, D), tree)
     _float(B * partial.size(1) * heads * Q, partial)
-    with torch.cuda.device(zc.device):
-        _check(lib().ff_pool_tree(_ptr(parent), _ptr(zc), _ptr(g), _ptr(b), _ptr(partial), partial.size(1), eps, B,
-                                  parent.size(1), Q, heads, D, _ptr(tree), _stream(zc)))
+    _run("ff_pool_tree", dev, _ptr(parent), _ptr(zc), _ptr(g), _ptr(b), _ptr(partial), partial.size(1), eps, B,
+         parent.size(1), Q, heads, D, _ptr(tree))
 
 
 def pool_leaf(tree: torch.Tensor, wl: torch.Tensor, bl: torch.Tensor, leaf: torch.Tensor) -> None:
     """leaf fp16 [B, Q*F] from tree fp16 [Q, B, D], wl fp16 [Q, F, D], bl fp16 [Q, F] (ff_pool_leaf)."""
-    _on_gpu(tree, wl, bl, leaf)
+    dev = _on_gpu(tree, wl, bl, leaf)
     Q, B, D = tree.shape
     F = wl.size(1)
     _half((Q, B, D), tree)
     _half((Q, F, D), wl)
     _half((Q, F), bl)
     _half((B, Q * F), leaf)
-    with torch.cuda.device(tree.device):
-        _check(lib().ff_pool_leaf(_ptr(tree), _ptr(wl), _ptr(bl), B, Q, F, D, _ptr(leaf), _stream(tree)))
+    _run("ff_pool_leaf", dev, _ptr(tree), _ptr(wl), _ptr(bl), B, Q, F, D, _ptr(leaf))
 
 
 def head_fits(rows: int, W: torch.Tensor) -> bool:
@@ -389,7 +390,7 @@ def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor
          beta: torch.Tensor | None = None, eps: float = 1e-6) -> None:
     """Tag head: out fp32 [B, N] = LN(x) W^T + bias, x fp16 [B, K] with contiguous rows (any row stride that is a
     multiple of 8), W fp16 [N, K], bias fp16 [N]; the norm (fp32 gamma, beta [K]) only if given (ff_head)."""
-    _on_gpu(W, bias, out, gamma, beta)
+    dev = _on_gpu(W, bias, out, gamma, beta)
     B, K = x.shape
     N = W.size(0)
     _require(x.device == W.device and x.dtype == torch.float16 and x.stride(1) == 1, "x must be fp16 rows on W's device")
@@ -399,9 +400,8 @@ def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor
     if gamma is not None:
         _require(beta is not None, "gamma and beta go together")
         _float(K, gamma, beta)
-    with torch.cuda.device(W.device):
-        _check(lib().ff_head(_ptr(x), max(x.stride(0), K), _ptr(gamma), _ptr(beta), eps, _ptr(W), _ptr(bias), B, N, K,
-                             _ptr(out), _stream(W)))
+    _run("ff_head", dev, _ptr(x), max(x.stride(0), K), _ptr(gamma), _ptr(beta), eps, _ptr(W), _ptr(bias), B, N, K,
+         _ptr(out))
 
 
 # ---- torch.ops.foidfinder_rocm registration (schemas as kernels.cu:268-273, plus eps / the fused norm) ----
