@@ -19,7 +19,7 @@ CSRC = PKG / "csrc"
 INCLUDE = PKG.parent / "include"
 LIB = PKG / "libfoidfinder_rocm.so"
 SOURCES = ["capi.hip", "rotq8.hip", "gemm_s8.hip", "attention.hip", "resample.hip", "pool.hip", "tree_pool.hip",
-           "head.hip"]
+           "head.hip", "stem.hip"]
 ARCH = "gfx950"
 
 FLAGS = [

@@ -25,7 +25,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 
-from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, lib, pad_norm
+from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, lib, pad_norm, pad_patch_weight
 
 Q_SCALE = 0.125 * math.log2(math.e)  # softmax scale x log2(e), folded into q by the QKV epilogue (engine.py:26)
 FORMAT = "foidfinder-eva02-int8-v1"
@@ -332,7 +332,12 @@ class Eva02Int8(Int8Engine):
             return t[p + ".weight"].float().contiguous(), t[p + ".bias"].float().contiguous()
 
         d = cfg.dim
-        self.patch_w_t = t["patch_embed.weight"].half().t().contiguous()  # [p*p*3, d]
+        self.fused_stem = cfg.patch == 14  # ff_patch_embed's patch size; other sizes take the library product
+        w = t["patch_embed.weight"].half()
+        if self.fused_stem:
+            self.patch_w = pad_patch_weight(w)
+        else:
+            self.patch_w_t = w.t().contiguous()  # [p*p*3, d]
         pos = t["pos_embed"].float().reshape(cfg.tokens, d)
         self.patch_bias_pos = (t["patch_embed.bias"].float() + pos[1:]).half().contiguous()  # [g*g, d]
         self.cls_pos = (t["cls_token"].float().reshape(d) + pos[0]).half().contiguous()
@@ -362,7 +367,8 @@ class Eva02Int8(Int8Engine):
         T, d, hp = B * cfg.tokens, cfg.dim, cfg.hidden_pad
         return {
             "x": torch.empty(T, d, device=dev, dtype=torch.half),
-            "patch": torch.empty(B * cfg.grid * cfg.grid, d, device=dev, dtype=torch.half),
+            **({} if self.fused_stem else
+               {"patch": torch.empty(B * cfg.grid * cfg.grid, d, device=dev, dtype=torch.half)}),
             "a8": torch.empty(T, d, device=dev, dtype=torch.int8),
             "rs": torch.empty(T, device=dev),
             "qkv": torch.empty(T, 3 * d, device=dev, dtype=torch.half),
@@ -393,10 +399,13 @@ class Eva02Int8(Int8Engine):
         k, cfg = self.k, self.cfg
         B, L, d = img.shape[0], cfg.tokens, cfg.dim
         x, a8, rs = buf["x"], buf["a8"], buf["rs"]
-        torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
         xv = x.view(B, L, d)
-        torch.add(buf["patch"].view(B, L - 1, d), self.patch_bias_pos, out=xv[:, 1:])
-        xv[:, 0] = self.cls_pos
+        if self.fused_stem:
+            k.patch_embed(img.to(torch.half).contiguous(), self.patch_w, self.patch_bias_pos, self.cls_pos, xv)
+        else:
+            torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
+            torch.add(buf["patch"].view(B, L - 1, d), self.patch_bias_pos, out=xv[:, 1:])
+            xv[:, 0] = self.cls_pos
         v = {name: self.variants.get((name, B), 0) for name in GEMMS}
         eps = cfg.eps
         if trace is not None:

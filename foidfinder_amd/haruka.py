@@ -31,7 +31,7 @@ import torch
 import torch.nn.functional as F
 
 from .engine import Int8Engine, eva02_rope_tables, rotate_quantize
-from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, pad_norm, pool_weights_blocks, slot_weights_blocks
+from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, pad_norm, pad_patch_weight, pool_weights_blocks, slot_weights_blocks
 
 ARCHITECTURE = "haruka-eva02-tree"  # foidfinder/haruka.py:14
 QUANTIZED = ("qkv", "proj", "fc1", "fc2")  # the backbone linears that run as W8A8
@@ -224,7 +224,11 @@ class HarukaInt8(Int8Engine):
             return x.half().contiguous()
 
         # stem (mlx/haruka.py:77-80): patch weights over (kh, kw, c) with the pixel normalization folded in
-        self.patch_w_t = half(t["patch_w"].reshape(d, -1).t())
+        self.fused_stem = cfg.patch == 14  # ff_patch_embed's patch size; other sizes take the library product
+        if self.fused_stem:
+            self.patch_w = pad_patch_weight(half(t["patch_w"].reshape(d, -1)))
+        else:
+            self.patch_w_t = half(t["patch_w"].reshape(d, -1).t())
         self.patch_b = half(t["patch_b"].reshape(cfg.grid * cfg.grid, d))
         self.cls = half(t["cls"].reshape(d))
         self.norm = (half(t["norm.weight"]), half(t["norm.bias"]))  # fp16, as the reference's weights
@@ -279,7 +283,8 @@ class HarukaInt8(Int8Engine):
         T, d, h = B * cfg.tokens, cfg.dim, cfg.hidden
         return {
             "x": torch.empty(T, d, device=dev, dtype=torch.half),
-            "patch": torch.empty(B * cfg.grid * cfg.grid, d, device=dev, dtype=torch.half),
+            **({} if self.fused_stem else
+               {"patch": torch.empty(B * cfg.grid * cfg.grid, d, device=dev, dtype=torch.half)}),
             "a8": torch.empty(T, d, device=dev, dtype=torch.int8),
             "rs": torch.empty(T, device=dev),
             "qkv": torch.empty(T, 3 * d, device=dev, dtype=torch.half),
@@ -399,10 +404,13 @@ class HarukaInt8(Int8Engine):
         k, cfg = self.k, self.cfg
         B, L, d = img.shape[0], cfg.tokens, cfg.dim
         x, a8, rs = buf["x"], buf["a8"], buf["rs"]
-        torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
         xv = x.view(B, L, d)
-        torch.add(buf["patch"].view(B, L - 1, d), self.patch_b, out=xv[:, 1:])
-        xv[:, 0] = self.cls
+        if self.fused_stem:
+            k.patch_embed(img.to(torch.half).contiguous(), self.patch_w, self.patch_b, self.cls, xv)
+        else:
+            torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
+            torch.add(buf["patch"].view(B, L - 1, d), self.patch_b, out=xv[:, 1:])
+            xv[:, 0] = self.cls
         v = {name: self.variants.get((name, B), 0) for name in QUANTIZED}
         eps = cfg.eps
         if trace is not None:

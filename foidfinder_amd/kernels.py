@@ -46,6 +46,7 @@ SIGNATURES = {
     "ff_pool_keys": ([_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp], _int),
     "ff_pool_tree": ([*[_vp] * 5, _i64, _f32, *[_i64] * 5, _vp, _vp], _int),
     "ff_pool_leaf": ([_vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp], _int),
+    "ff_patch_embed": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp], _int),
     "ff_head": ([_vp, _i64, _vp, _vp, _f32, _vp, _vp, _i64, _i64, _i64, _vp, _vp], _int),
 }
 ABI_VERSION = 3
@@ -381,6 +382,30 @@ def pool_leaf(tree: torch.Tensor, wl: torch.Tensor, bl: torch.Tensor, leaf: torc
     _run("ff_pool_leaf", dev, _ptr(tree), _ptr(wl), _ptr(bl), B, Q, F, D, _ptr(leaf))
 
 
+PATCH_COLS, PATCH_PAD = 588, 608  # 14 x 14 x 3, and the row length of patch_embed's weights
+
+
+def pad_patch_weight(w: torch.Tensor) -> torch.Tensor:
+    """Patch weights [N, 588] -> fp16 [N, 608] with zeros past column 588, as patch_embed takes them."""
+    out = torch.zeros(w.size(0), PATCH_PAD, dtype=torch.half, device=w.device)
+    out[:, :PATCH_COLS] = w
+    return out
+
+
+def patch_embed(img: torch.Tensor, w: torch.Tensor, bias_pos: torch.Tensor, cls: torch.Tensor, x: torch.Tensor) -> None:
+    """x fp16 [B, 1 + grid^2, N]: the class row, then each 14 x 14 patch of img fp16 [B, S, S, 3] times w fp16 [N, 608]
+    (pad_patch_weight) plus bias_pos fp16 [grid^2, N] (ff_patch_embed)."""
+    dev = _on_gpu(img, w, bias_pos, cls, x)
+    B, S = img.shape[:2]
+    grid, N = S // 14, w.size(0)
+    _half((B, grid * 14, grid * 14, 3), img)
+    _half((N, PATCH_PAD), w)
+    _half((grid * grid, N), bias_pos)
+    _half((N,), cls)
+    _half((B, 1 + grid * grid, N), x)
+    _run("ff_patch_embed", dev, _ptr(img), _ptr(w), _ptr(bias_pos), _ptr(cls), B, grid, N, _ptr(x))
+
+
 def head_fits(rows: int, W: torch.Tensor) -> bool:
     """Whether `head` takes this many rows of x with W [N, K] (others go to the library's GEMM)."""
     return rows <= 64 and W.size(1) % 32 == 0 and W.size(1) <= 1280
@@ -432,9 +457,10 @@ _LIB.define("pool_keys(Tensor qleaf, Tensor kT, Tensor(a!) u) -> ()")
 _LIB.define("pool_tree(Tensor parent, Tensor zc, Tensor g, Tensor b, Tensor partial, int heads, float eps, "
             "Tensor(a!) tree) -> ()")
 _LIB.define("pool_leaf(Tensor tree, Tensor wl, Tensor bl, Tensor(a!) leaf) -> ()")
+_LIB.define("patch_embed(Tensor img, Tensor w, Tensor bias_pos, Tensor cls, Tensor(a!) x) -> ()")
 _LIB.define("head(Tensor x, Tensor W, Tensor bias, Tensor(a!) out, Tensor? gamma=None, Tensor? beta=None, "
             "float eps=1e-06) -> ()")
-for _fn in (pool_weights, pool_values, pool_queries, pool_keys, pool_tree, pool_leaf, head):
+for _fn in (pool_weights, pool_values, pool_queries, pool_keys, pool_tree, pool_leaf, patch_embed, head):
     _LIB.impl(_fn.__name__, _fn, "CUDA")
 _LIB.impl("layer_norm2", layer_norm2, "CUDA")
 _LIB.impl("slot_weights", slot_weights, "CUDA")

@@ -143,6 +143,12 @@ int ff_pool_tree(const void* parent, const void* zc, const void* g, const void* 
 int ff_pool_leaf(const void* tree, const void* wl, const void* bl, int64_t B, int64_t Q, int64_t F, int64_t D,
                  void* leaf, void* stream);
 
+/* ViT stem over 14 x 14 patches: x fp16 [B, 1 + grid^2, N], x[b, 1 + p] = patch p . w[n] + bias_pos[p, n], x[b, 0] = cls.
+ * img fp16 [B, 14 grid, 14 grid, 3], patch columns in (row, column, channel) order, w fp16 [N, 608] (588 columns, zeros
+ * past them), bias_pos fp16 [grid^2, N], cls fp16 [N], N % 128 == 0. */
+int ff_patch_embed(const void* img, const void* w, const void* bias_pos, const void* cls, int64_t B, int64_t grid,
+                   int64_t N, void* x, void* stream);
+
 /* Tag head: out fp32 [B, N] = LN(x) W^T + bias (the norm only with gamma and beta, fp32 [K]); x fp16, B <= 64 rows
  * x_stride elements apart (% 8 == 0), W fp16 [N, K], bias fp16 [N], K % 32 == 0, K <= 1280. */
 int ff_head(const void* x, int64_t x_stride, const float* gamma, const float* beta, float eps, const void* W,

@@ -146,3 +146,21 @@ def test_pool_head_matches_library_chain(dev, batch, pool_heads, leaf_dim):
     # the library chain rounds its logits, products and masses to fp16 at a dozen points: 4e-3 of the result's size
     rel = ((got - want).double().norm() / want.double().norm()).item()
     assert rel < 4e-3, f"fused and library pools differ by {rel:.2e}"
+
+
+@pytest.mark.parametrize(("B", "grid", "N"), [(1, 1, 128), (2, 9, 128), (3, 8, 768), (1, 17, 384), (40, 8, 1024)])
+def test_patch_embed(dev, B, grid, N):
+    """One patch, patch counts that end inside a workgroup's 64, both column splits (the last is past 1024 workgroups of
+    64 columns), and raw pixel values: the class row is copied, the others are float64's within one fp16 rounding (fp32
+    sums of 588 products)."""
+    S = 14 * grid
+    img = (torch.rand(B, S, S, 3, device=dev, generator=torch.Generator(device=dev).manual_seed(B)) * 255).round().half()
+    w, bias = randn(dev, N, 588, std=1e-3, seed=1).half(), randn(dev, grid * grid, N, seed=2).half()
+    cls = randn(dev, N, seed=3).half()
+    x = torch.full((B, 1 + grid * grid, N), float("nan"), device=dev, dtype=torch.half)
+    K.patch_embed(img, K.pad_patch_weight(w), bias, cls, x)
+    p = img.double().view(B, grid, 14, grid, 14, 3).permute(0, 1, 3, 2, 4, 5).reshape(B, grid * grid, 588)
+    want = p @ w.double().t() + bias.double()
+    assert torch.equal(x[:, 0], cls.expand(B, N))
+    bound = FP16 * want.abs() + 588 * 2.0**-24 * (p @ w.double().abs().t() + bias.double().abs()) + 2.0**-25
+    assert ((x[:, 1:].double() - want).abs() <= bound).all()
