@@ -2,7 +2,7 @@
 // never formed (logits = xn . u, u = Wk_h^T q; pooled = w^T xn, then Wv_h), the two attention levels each take:
 //
 //  * pool_weights: logits xn u^T on MFMA and from them the slot-sigmoid weights, transposed, in one kernel;
-//  * (the pooling product w^T xn, a library GEMM)
+//  * pool_sum: the pooling product w^T xn;
 //  * pool_values: the value projection of the pooled tokens plus the value bias times each query's mass;
 //
 // and between and after them: pool_queries (parent norm, leaf queries), pool_keys (the leaf queries' u), pool_tree (leaf
@@ -22,17 +22,20 @@ __device__ __forceinline__ void to_lds(const void* base, int nbytes, void* lds_d
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds_dst, 16, voff, 0, 0, 0);
 }
 
-constexpr int PW_TOK = 64;  // tokens per workgroup of pool_weights
+constexpr int PW_TOK = 96;   // tokens per workgroup of pool_weights
+constexpr int PW_SLOTS = 5;  // its LDS ring's depth
 
-// A workgroup per (batch, block of 64 tokens). Logits of the block's tokens against all GM = G M query columns: u [GM, D] and xn
-// stream through three LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
-// conflict-free fragment reads) filled by buffer->LDS loads, two slots ahead; rows past GM or the sequence read as
-// zeros. A wave takes one 32-query tile (MFMA rows) and NT of the block's two 32-token tiles (MFMA columns): nine waves
-// of two at Haruka's 288 leaf columns, six of one at its 96 coarse columns. The fp32 logits go to LDS as [GM][64 + 1]; a
-// thread then turns the M logits of a (token, head) pair into weights in place: softmax over the queries times
-// sigmoid(logit + bias), from the hardware exp2 and reciprocal (each about 1 ulp). Tokens past the sequence get weight 0.
-// partial[b, block, j] is column j's sum over the block's tokens, a_t[b, j, n] the weight in fp16 (rows of ldt; a row's
-// pad column may be written with 0). GMAX bounds GM: at 288, 75 KB of LDS let two workgroups share a CU.
+// A workgroup per (batch, block of 96 tokens). Logits of the block's tokens against all GM = G M query columns: u [GM, D] and xn
+// stream through five LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
+// conflict-free fragment reads) filled by buffer->LDS loads, four slots ahead: both were written by the launches before,
+// through other L2s, and a load takes ~0.8 us (two slots ahead ran 33 us at 288 columns and 16 x 1025 tokens). Rows past
+// GM or the sequence read as zeros. A wave takes one 32-query tile (MFMA rows) and NT of the block's three 32-token tiles
+// (MFMA columns): nine waves of three at Haruka's 288 leaf columns, nine of one at its 96 coarse columns. The fp32 logits
+// go to LDS as [GM][96 + 1]; a thread then turns the M logits of a (token, head) pair into weights in place: softmax over
+// the queries times sigmoid(logit + bias), from the hardware exp2 and reciprocal (each about 1 ulp). Tokens past the
+// sequence get weight 0. partial[b, block, j] is column j's sum over the block's tokens, a_t[b, j, n] the weight in fp16
+// (rows of ldt, their pad columns 0). GMAX bounds GM. 96 tokens, not 64: 1025 are 11 blocks then, 176 workgroups at 16
+// images, one per CU, where 17 blocks would be 272, the last ones with a token each.
 template <int GMAX, int NT>
 constexpr int pw_waves() {
   return GMAX / 32 * (PW_TOK / 32 / NT);
@@ -45,7 +48,7 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
   constexpr int WV = pw_waves<GMAX, NT>(), THREADS = 64 * WV;
   constexpr int LOADS = (GMAX + PW_TOK) / 16;     // 1 KB loads per slot: 16 rows each, queries, then tokens
   constexpr int PER = (LOADS + WV - 1) / WV;      // per wave, the last only in waves below LOADS % WV (0: all)
-  constexpr int SLOT = LOADS * 1024, SLOTS = 3;
+  constexpr int SLOT = LOADS * 1024, SLOTS = PW_SLOTS;
   constexpr int LDT = PW_TOK + 1;
   constexpr int BYTES = SLOTS * SLOT > GMAX * LDT * 4 ? SLOTS * SLOT : GMAX * LDT * 4;
   constexpr float LOG2E = 1.4426950408889634f;
@@ -75,20 +78,22 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
   auto frag = [&](const uint8_t* base, int row, int chunk) __attribute__((always_inline)) {
     return *reinterpret_cast<const half8_t*>(base + row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4));
   };
-  const int qt = NT == 2 ? wave : wave >> 1, t0 = NT == 2 ? 0 : wave & 1, fr = lane & 31, fh = lane >> 5;
+  constexpr int TS = PW_TOK / 32 / NT;  // waves per query tile
+  const int qt = wave / TS, t0 = wave % TS * NT, fr = lane & 31, fh = lane >> 5;
   float16_t acc[NT] = {};
   const int chunks = D / 32;  // at least four (D % 128 == 0)
-  issue(0);
-  issue(1);
+#pragma unroll
+  for (int i = 0; i < SLOTS - 1; ++i)
+    if (i < chunks) issue(i);
   for (int kc = 0; kc < chunks; ++kc) {
-    // slot kc has landed once only slot kc + 1's loads are outstanding
-    if (kc + 1 == chunks)
+    // slot kc has landed once only the SLOTS - 2 slots after it have loads outstanding
+    if (kc + SLOTS - 2 >= chunks)
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     else if (full)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SLOTS - 2) * PER) : "memory");
     else
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER - 1) : "memory");
-    __builtin_amdgcn_s_barrier();  // and every wave has read slot kc - 1, which slot kc + 2 takes over
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SLOTS - 2) * (PER - 1)) : "memory");
+    __builtin_amdgcn_s_barrier();  // and every wave has read slot kc - 1, which slot kc + SLOTS - 1 takes over
     asm volatile("" ::: "memory");
     const uint8_t* su = lds + kc % SLOTS * SLOT;
     const uint8_t* sx = su + GMAX * 64;
@@ -99,7 +104,7 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
 #pragma unroll
       for (int i = 0; i < NT; ++i) xf[ks][i] = frag(sx, 32 * (t0 + i) + fr, 2 * ks + fh);
     }
-    if (kc + 2 < chunks) issue(kc + 2);
+    if (kc + SLOTS - 1 < chunks) issue(kc + SLOTS - 1);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -116,8 +121,8 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
     }
   const float* cb = c + b * c_stride;
   __syncthreads();
-  for (int p = threadIdx.x; p < PW_TOK * G; p += THREADS) {  // a wave's 64 lanes are the block's tokens, its head is uniform
-    const int t = p % PW_TOK, h = __builtin_amdgcn_readfirstlane(p / PW_TOK);
+  for (int p = threadIdx.x; p < PW_TOK * G; p += THREADS) {
+    const int t = p % PW_TOK, h = p / PW_TOK;
     float l[M], w[M], mx = -INFINITY, s = 0.f;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
@@ -143,12 +148,125 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
     for (int t = 0; t < PW_TOK; ++t) s += tile[j * LDT + t];
     partial[(static_cast<int64_t>(b) * blocks + blk) * GM + j] = s;
   }
-  // two query rows per wave and pass, two tokens (4 bytes) per lane; ldt is even, so a pair past an odd end is pad
-  const int t2 = 2 * (lane & 31);
-  if (t2 < ntok)
-    for (int j = 2 * wave + (lane >> 5); j < GM; j += 2 * WV)
+  // a query row per wave and pass, two tokens (4 bytes) per lane, up to the row's (even) pitch: past the sequence the
+  // tile holds zeros
+  const int t2 = 2 * lane;
+  if (t2 < PW_TOK && t2 < ldt - n0)
+    for (int j = wave; j < GM; j += WV)
       *reinterpret_cast<half2_t*>(a_t + (static_cast<int64_t>(b) * GM + j) * ldt + n0 + t2) =
           half2_t{static_cast<half_t>(tile[j * LDT + t2]), static_cast<half_t>(tile[j * LDT + t2 + 1])};
+}
+
+// pooled[b, j, d] = sum_n a_t[b, j, n] xn[b, n, d]: a workgroup per (batch, 96 queries j, 64 SUB columns d), wave w the 32
+// columns 32 w against the three 32-query tiles (columns as MFMA rows, queries as columns), the tokens in chunks of 64
+// through four LDS slots, three ahead (a load takes ~0.8 us: its rows come from other L2s). xn's rows are the product's k:
+// its fragments come through the transposing ds_read_b64_tr_b16, which hands a lane 4 consecutive tokens of one column
+// (slot u of lane half f: token 8 f + u of 16, so that a_t's fragments are 16-byte reads; 8-byte ones, which conflict
+// two ways, made LDS the bound at 21 and 23 us a launch). Tokens past the sequence
+// read as zero rows of xn against finite weights (a_t's zero pad, or the next row); queries past GM read as zeros and are
+// not stored. SUB = 3 where 192 divides D (Haruka's 768: 64 and 192 workgroups at 16 images for the 96 coarse and 288 leaf
+// queries, one per CU), else 2.
+// 16 images, per launch: as a library product 15.9 and 28.2 us; two slots of 128 columns 16.0 and 21.3.
+constexpr int PS_J = 96, PS_N = 64, PS_SLOTS = 4;
+
+template <int OFF>
+__device__ __forceinline__ void tr_read(half4_t& v, uint32_t lds_addr) {
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "n"(OFF) : "memory");
+}
+
+template <int SUB>
+__global__ __launch_bounds__(128 * SUB) void pool_sum_kernel(const half_t* __restrict__ a_t, const half_t* __restrict__ xn,
+                                                             int N, int GM, int D, int ldt,
+                                                             half_t* __restrict__ pooled) {
+  constexpr int WV = 2 * SUB, XB = PS_N * 128;             // waves; bytes of 64 columns of a chunk (rows of 128)
+  constexpr int LOADS = SUB * 8 + PS_J * PS_N * 2 / 1024;  // 1 KB loads per slot, 8 rows each: xn by 64 columns, then a_t
+  constexpr int PER = LOADS / WV, SLOT = LOADS * 1024;
+  static_assert(LOADS % WV == 0, "every wave issues as many loads");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[PS_SLOTS * SLOT];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fr = lane & 31, fh = lane >> 5;
+  // 1-D grid over (batch, query tile, column tile), a batch's workgroups on one XCD
+  const int td = D / (64 * SUB), tj = (GM + PS_J - 1) / PS_J, t = xcd_remap(blockIdx.x, gridDim.x);
+  const int b = t / (td * tj), j0 = t / td % tj * PS_J, d0 = t % td * 64 * SUB;
+  const half_t* xb = xn + static_cast<int64_t>(b) * N * D + d0;
+  const half_t* ab = a_t + (static_cast<int64_t>(b) * GM + j0) * ldt;
+  const int a_bytes = (GM - j0) * ldt * 2;
+
+  // 16-byte chunk c of row r sits at slot c ^ 2 (r & 2) of xn's rows (the four rows of a transposing read on distinct
+  // banks) and at c ^ ((r >> 1) & 7) of a_t's
+  auto issue = [&](int chunk) __attribute__((always_inline)) {
+    uint8_t* dst = lds + chunk % PS_SLOTS * SLOT;
+    const int n0 = chunk * PS_N;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int q = wave + WV * p;  // wave-uniform
+      if (q < 8 * SUB) {
+        const int r = 8 * (q & 7) + (lane >> 3), c = (lane & 7) ^ ((r & 2) << 1);
+        to_lds(xb + static_cast<int64_t>(n0) * D, (N - n0) * D * 2 - d0 * 2, dst + q * 1024,
+               static_cast<uint32_t>(r * D * 2 + (q >> 3) * 128 + c * 16));
+      } else {
+        const int r = 8 * (q - 8 * SUB) + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        to_lds(ab, a_bytes, dst + q * 1024, static_cast<uint32_t>(r * ldt * 2 + n0 * 2 + c * 16));
+      }
+    }
+  };
+  const int row = 8 * fh + ((lane & 15) >> 2), col = 32 * (wave & 1) + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const uint32_t xoff =
+      static_cast<uint32_t>((wave >> 1) * XB + row * 128 + (((col >> 3) ^ ((row & 2) << 1)) << 4) + (col & 7) * 2);
+  float16_t acc[3] = {};
+  const int chunks = (N + PS_N - 1) / PS_N;
+#pragma unroll
+  for (int i = 0; i < PS_SLOTS - 1; ++i)
+    if (i < chunks) issue(i);
+  for (int k = 0; k < chunks; ++k) {
+    // chunk k has landed once only the PS_SLOTS - 2 chunks after it have loads outstanding
+    if (k + PS_SLOTS - 2 >= chunks)
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((PS_SLOTS - 2) * PER) : "memory");
+    __builtin_amdgcn_s_barrier();  // and every wave has read chunk k - 1
+    asm volatile("" ::: "memory");
+    if (k + PS_SLOTS - 1 < chunks) issue(k + PS_SLOTS - 1);
+    const uint8_t* sl = lds + k % PS_SLOTS * SLOT;
+    const uint32_t xa = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)sl)) + xoff;
+    half4_t x[4][2];
+    tr_read<0 * 128>(x[0][0], xa), tr_read<4 * 128>(x[0][1], xa);
+    tr_read<16 * 128>(x[1][0], xa), tr_read<20 * 128>(x[1][1], xa);
+    tr_read<32 * 128>(x[2][0], xa), tr_read<36 * 128>(x[2][1], xa);
+    tr_read<48 * 128>(x[3][0], xa), tr_read<52 * 128>(x[3][1], xa);
+    half8_t w[4][3];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int r = 32 * i + fr;
+        w[tt][i] = *reinterpret_cast<const half8_t*>(sl + SUB * XB + r * 128 + (((2 * tt + fh) ^ ((r >> 1) & 7)) << 4));
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[2][0]), "+v"(x[2][1]),
+                   "+v"(x[3][0]), "+v"(x[3][1])::"memory");
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt) {
+      const half4_t lo = x[tt][0], hi = x[tt][1];
+      const half8_t xf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+#pragma unroll
+      for (int i = 0; i < 3; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf, w[tt][i], acc[i], 0, 0, 0);
+    }
+  }
+  // acc[i][4 q + e]: column d0 + 32 wave + 8 q + 4 (lane / 32) + e of query j0 + 32 i + lane % 32
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int j = j0 + 32 * i + fr;
+    if (j >= GM) continue;
+    half_t* o = pooled + (static_cast<int64_t>(b) * GM + j) * D + d0 + 32 * wave + 4 * fh;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      half4_t v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = static_cast<half_t>(acc[i][4 * q + e]);
+      *reinterpret_cast<half4_t*>(o + 8 * q) = v;
+    }
+  }
 }
 
 // One 16 x 16 product tile over K (K % 32 == 0, columns contiguous) by 4 waves: wave w takes the 32-column steps w,
@@ -406,12 +524,13 @@ extern "C" int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, 
                                void* a_t, float* partial, void* stream) {
   clear_error();
   FF_POOL_CHECK("pool_weights", B, G, D);
-  if (N <= 0 || N > (1 << 24)) return fail(FF_EINVAL, "pool_weights: bad N");
+  if (N <= 0 || N > (1 << 18)) return fail(FF_EINVAL, "pool_weights: bad N");
   if (M != 6 && M != 18) return fail(FF_EINVAL, "pool_weights: M must be 6 or 18 (the tree pool's query counts)");
-  if (G * M > 512) return fail(FF_EINVAL, "pool_weights: G*M above 512");
+  if (G * M > 384) return fail(FF_EINVAL, "pool_weights: G*M above 384");
   if ((u_stride != 0 && u_stride < G * M * D) || u_stride % 8 != 0 || (c_stride != 0 && c_stride < G * M))
     return fail(FF_EINVAL, "pool_weights: u_stride must be 0 or >= G*M*D, c_stride 0 or >= G*M");
-  if (ldt < N || ldt % 2 != 0) return fail(FF_EINVAL, "pool_weights: need ldt >= N, even");
+  if (ldt < N || ldt % 2 != 0 || ldt > (N + 7) / 8 * 8)
+    return fail(FF_EINVAL, "pool_weights: need ldt even and N <= ldt <= the next multiple of 8");
   if (B == 0) return FF_OK;
   if (!xn || !u || !c || !bias || !a_t || !partial) return fail(FF_EINVAL, "pool_weights: null pointer");
   if (!al(xn, 16) || !al(u, 16) || !al(a_t, 4)) return fail(FF_EINVAL, "pool_weights: misaligned pointer");
@@ -428,13 +547,37 @@ extern "C" int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, 
   if (M == 6 && G * M <= 96)
     FF_PW(6, 96, 1);
   else if (M == 6)
-    FF_PW(6, 512, 2);
+    FF_PW(6, 384, 3);
   else if (G * M <= 288)
-    FF_PW(18, 288, 2);
+    FF_PW(18, 288, 3);
   else
-    FF_PW(18, 512, 2);
+    FF_PW(18, 384, 3);
 #undef FF_PW
   return check_launch("pool_weights");
+}
+
+extern "C" int ff_pool_sum(const void* a_t, const void* xn, int64_t B, int64_t N, int64_t GM, int64_t D, int64_t ldt,
+                           void* pooled, void* stream) {
+  clear_error();
+  FF_POOL_CHECK("pool_sum", B, 1, D);
+  if (N <= 0 || N > (1 << 18)) return fail(FF_EINVAL, "pool_sum: bad N");
+  if (GM <= 0 || GM > 512) return fail(FF_EINVAL, "pool_sum: need 0 < GM <= 512");
+  if (ldt != (N + 7) / 8 * 8) return fail(FF_EINVAL, "pool_sum: ldt must be N rounded up to a multiple of 8");
+  if (B == 0) return FF_OK;
+  if (!a_t || !xn || !pooled) return fail(FF_EINVAL, "pool_sum: null pointer");
+  if (!al(a_t, 16) || !al(xn, 16) || !al(pooled, 8)) return fail(FF_EINVAL, "pool_sum: misaligned pointer");
+  const int sub = D % 192 == 0 ? 3 : 2;
+  const int64_t blocks = B * ((GM + PS_J - 1) / PS_J) * (D / (64 * sub));
+  if (blocks > 0x7fffffff) return fail(FF_EINVAL, "pool_sum: too many tiles");
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const auto *pa = static_cast<const half_t*>(a_t), *px = static_cast<const half_t*>(xn);
+  auto* po = static_cast<half_t*>(pooled);
+  const int Ni = static_cast<int>(N), Gi = static_cast<int>(GM), Di = static_cast<int>(D), li = static_cast<int>(ldt);
+  if (sub == 3)
+    pool_sum_kernel<3><<<grid, 384, 0, as_stream(stream)>>>(pa, px, Ni, Gi, Di, li, po);
+  else
+    pool_sum_kernel<2><<<grid, 256, 0, as_stream(stream)>>>(pa, px, Ni, Gi, Di, li, po);
+  return check_launch("pool_sum");
 }
 
 extern "C" int ff_pool_values(const void* pooled, const void* wv, const float* bv, const float* partial, int64_t nblk,

@@ -262,7 +262,7 @@ class HarukaInt8(Int8Engine):
         leaf_w = half(t["pool.leaf.weight"].reshape(cfg.leaves, d, cfg.leaf_dim))
         # The pool's own kernels take heads and leaves of whole 16-column tiles (Haruka: 48 and 64); other shapes run
         # on library products, with those products' weight layouts.
-        self.fused_pool = hd % 16 == 0 and cfg.leaf_dim % 16 == 0 and d <= 2048 and Hp * cfg.leaves <= 512
+        self.fused_pool = hd % 16 == 0 and cfg.leaf_dim % 16 == 0 and d <= 2048 and Hp * cfg.leaves <= 384
         if self.fused_pool:
             self.coarse_u = coarse_u
             self.pool_v = half(kv_w[d:])  # [d, d]: Wv
@@ -341,11 +341,12 @@ class HarukaInt8(Int8Engine):
             return torch.empty(*shape, device=xn.device, dtype=dtype)
 
         def attend(u, c, bias, M):
-            a_t = new(B, Hp * M, (N + 7) // 8 * 8)  # whole 16-byte rows; the product reads the first N columns
+            a_t = new(B, Hp * M, (N + 7) // 8 * 8)  # whole 16-byte rows
             partial = new(B, pool_weights_blocks(N), Hp * M, dtype=torch.float32)
             k.pool_weights(xn, u, c, bias, Hp, a_t, partial)
-            z = new(B, M, d)
-            k.pool_values(torch.bmm(a_t[:, :, :N], xn), self.pool_v, self.pool_bv.view(-1), partial, Hp, z)
+            pooled, z = new(B, Hp * M, d), new(B, M, d)
+            k.pool_sum(a_t, xn, pooled)
+            k.pool_values(pooled, self.pool_v, self.pool_bv.view(-1), partial, Hp, z)
             return z, partial
 
         z, _ = attend(self.coarse_u, self.coarse_c, self.q_coarse_bias, C)

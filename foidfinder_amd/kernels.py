@@ -41,6 +41,7 @@ SIGNATURES = {
     "ff_slot_weights": ([_vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp], _int),
     "ff_pool_weights_blocks": ([_i64], _i64),
     "ff_pool_weights": ([_vp, _vp, _i64, _vp, _i64, _vp, *[_i64] * 6, _vp, _vp, _vp], _int),
+    "ff_pool_sum": ([_vp, _vp, *[_i64] * 5, _vp, _vp], _int),
     "ff_pool_values": ([_vp, _vp, _vp, _vp, *[_i64] * 5, _vp, _vp], _int),
     "ff_pool_queries": ([*[_vp] * 7, _f32, *[_i64] * 5, _vp, _vp, _vp, _vp], _int),
     "ff_pool_keys": ([_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp], _int),
@@ -314,6 +315,18 @@ def pool_weights(xn: torch.Tensor, u: torch.Tensor, c: torch.Tensor, bias: torch
          GM, _ptr(bias), B, N, heads, M, D, a_t.size(-1), _ptr(a_t), _ptr(partial))
 
 
+def pool_sum(a_t: torch.Tensor, xn: torch.Tensor, pooled: torch.Tensor) -> None:
+    """pooled fp16 [B, GM, D] = a_t xn over the N tokens of xn fp16 [B, N, D], a_t fp16 [B, GM, ldt] as pool_weights leaves
+    it (ff_pool_sum)."""
+    dev = _on_gpu(a_t, xn, pooled)
+    B, N, D = xn.shape
+    GM = a_t.size(1)
+    _half((B, N, D), xn)
+    _half((B, GM, a_t.size(-1)), a_t)
+    _half((B, GM, D), pooled)
+    _run("ff_pool_sum", dev, _ptr(a_t), _ptr(xn), B, N, GM, D, a_t.size(-1), _ptr(pooled))
+
+
 def pool_values(pooled: torch.Tensor, wv: torch.Tensor, bv: torch.Tensor, partial: torch.Tensor, heads: int,
                 z: torch.Tensor) -> None:
     """z fp16 [B, M, D] from pooled fp16 [B, heads*M, D], wv fp16 [D, D], bv fp32 [D] and the weights' partial sums."""
@@ -450,6 +463,7 @@ _LIB.define("layer_norm2(Tensor x, Tensor g1, Tensor b1, Tensor g2, Tensor b2, f
 _LIB.define("slot_weights(Tensor logits, Tensor c, Tensor bias, int heads, Tensor(a!) a_t, Tensor(b!) partial) -> ()")
 _LIB.define("pool_weights(Tensor xn, Tensor u, Tensor c, Tensor bias, int heads, Tensor(a!) a_t, Tensor(b!) partial) "
             "-> ()")
+_LIB.define("pool_sum(Tensor a_t, Tensor xn, Tensor(a!) pooled) -> ()")
 _LIB.define("pool_values(Tensor pooled, Tensor wv, Tensor bv, Tensor partial, int heads, Tensor(a!) z) -> ()")
 _LIB.define("pool_queries(Tensor z, Tensor trunk_g, Tensor trunk_b, Tensor child, Tensor child_g, Tensor child_b, "
             "Tensor bk, int heads, float eps, Tensor(a!) parent, Tensor(b!) qleaf, Tensor(c!) cq) -> ()")
@@ -460,7 +474,7 @@ _LIB.define("pool_leaf(Tensor tree, Tensor wl, Tensor bl, Tensor(a!) leaf) -> ()
 _LIB.define("patch_embed(Tensor img, Tensor w, Tensor bias_pos, Tensor cls, Tensor(a!) x) -> ()")
 _LIB.define("head(Tensor x, Tensor W, Tensor bias, Tensor(a!) out, Tensor? gamma=None, Tensor? beta=None, "
             "float eps=1e-06) -> ()")
-for _fn in (pool_weights, pool_values, pool_queries, pool_keys, pool_tree, pool_leaf, patch_embed, head):
+for _fn in (pool_weights, pool_sum, pool_values, pool_queries, pool_keys, pool_tree, pool_leaf, patch_embed, head):
     _LIB.impl(_fn.__name__, _fn, "CUDA")
 _LIB.impl("layer_norm2", layer_norm2, "CUDA")
 _LIB.impl("slot_weights", slot_weights, "CUDA")

@@ -118,12 +118,17 @@ int ff_slot_weights(const void* logits, const float* c, int64_t c_stride, const 
  * and weights fp16, sums, biases and masses fp32.
  *
  * ff_pool_weights: ff_slot_weights with the logits' product in it: l[m] = xn[b, n] . u[b, h*M + m] + c[...], u fp16
- * [B, G*M, D] (u_stride elements between batches, 0: shared), M = 6 or 18, G*M <= 512. a_t fp16 [B, G*M, ldt] (ldt >= N,
- * even; pad columns undefined), partial fp32 [B, ff_pool_weights_blocks(N), G*M]. */
+ * [B, G*M, D] (u_stride elements between batches, 0: shared), M = 6 or 18, G*M <= 384, N <= 2^18. a_t fp16
+ * [B, G*M, ldt] (ldt even, from N to the next multiple of 8; pad columns 0), partial fp32
+ * [B, ff_pool_weights_blocks(N), G*M]. */
 int64_t ff_pool_weights_blocks(int64_t N);
 int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, const float* c, int64_t c_stride,
                     const float* bias, int64_t B, int64_t N, int64_t G, int64_t M, int64_t D, int64_t ldt, void* a_t,
                     float* partial, void* stream);
+/* pooled fp16 [B, GM, D]: pooled[b, j] = sum_n a_t[b, j, n] xn[b, n]; a_t as ff_pool_weights leaves it, ldt = N
+ * rounded up to a multiple of 8, GM <= 512. */
+int ff_pool_sum(const void* a_t, const void* xn, int64_t B, int64_t N, int64_t GM, int64_t D, int64_t ldt, void* pooled,
+                void* stream);
 /* z[b, m, h*hd + e] = pooled[b, h*M + m] . wv[h*hd + e] + bv[h*hd + e] * sum_k partial[b, k, h*M + m]; pooled
  * [B, G*M, D], wv [D, D], z [B, M, D]. */
 int ff_pool_values(const void* pooled, const void* wv, const float* bv, const float* partial, int64_t nblk, int64_t B,

@@ -54,8 +54,8 @@ def test_head(dev, B, N, K_, norm):
     assert ((out.double() - want).abs() <= bound).all()
 
 
-@pytest.mark.parametrize(("B", "N", "G", "M", "D"), [(1, 1, 16, 6, 768), (2, 64, 16, 18, 768), (3, 65, 4, 18, 128),
-                                                     (1, 129, 20, 18, 640), (2, 63, 64, 6, 1024)])
+@pytest.mark.parametrize(("B", "N", "G", "M", "D"), [(1, 1, 16, 6, 768), (2, 96, 16, 18, 768), (3, 97, 4, 18, 128),
+                                                     (1, 193, 20, 18, 640), (2, 95, 64, 6, 1024)])
 @pytest.mark.parametrize("shared", [True, False])
 def test_pool_weights(dev, B, N, G, M, D, shared):
     xn = randn(dev, B, N, D, seed=1).half()
@@ -74,6 +74,20 @@ def test_pool_weights(dev, B, N, G, M, D, shared):
     assert ((got - want).abs() <= (FP16 + 2e-5) * want + 2.0**-24).all()
     mass = w.sum(1)
     assert ((partial.double().sum(1) - mass).abs() <= 3e-5 * mass).all()
+    assert (a_t[:, :, N:] == 0).all()
+
+
+@pytest.mark.parametrize(("B", "N", "GM", "D"), [(1, 1, 96, 128), (2, 64, 288, 768), (3, 65, 24, 256), (2, 127, 120, 384),
+                                                 (1, 1025, 512, 128), (1, 333, 97, 192 * 2)])
+def test_pool_sum(dev, B, N, GM, D):
+    """One token, token counts around a chunk of 64, queries that end inside a tile of 96 and past five tiles; whatever
+    follows a row's N weights (zero pad, the next row) must not count."""
+    xn = randn(dev, B, N, D, seed=1).half()
+    a_t = torch.zeros(B, GM, (N + 7) // 8 * 8, device=dev, dtype=torch.half)
+    a_t[:, :, :N] = torch.rand(B, GM, N, device=dev, generator=torch.Generator(device=dev).manual_seed(N)).half()
+    pooled = torch.full((B, GM, D), float("nan"), device=dev, dtype=torch.half)
+    K.pool_sum(a_t, xn, pooled)
+    close(pooled, torch.matmul(a_t[:, :, :N].double().contiguous(), xn.double()), "pooled")
 
 
 @pytest.mark.parametrize(("B", "C", "Q", "G", "D", "F"), [(1, 6, 18, 16, 768, 64), (3, 6, 18, 8, 128, 16),
