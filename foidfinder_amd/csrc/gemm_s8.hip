@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 
@@ -803,7 +804,7 @@ constexpr int KS_CHUNK = 128 * 64;     // one staged chunk: 64 A rows + 64 W row
 constexpr int KS_PART = 64 * 64 * 4;   // one wave's 64 x 64 int32 partial tile
 
 template <int EPI>
-__global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs args) {
+__global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs args, int panel) {
   constexpr int WV = 4;          // waves per block
   constexpr int SLOTS = WV / 2;  // partial slots in the chunk buffers
   static_assert(stage_bytes<EPI, 1>() <= KS_CHUNK, "a quadrant's staging fits its wave's chunk buffer");
@@ -814,7 +815,12 @@ __global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs a
   const int M = args.M, N = args.N, K = args.K, nch = K / 64;
   const int tiles_n = (N + 63) / 64;
   const int t = xcd_remap(blockIdx.x, gridDim.x);
-  const int m0 = (t / tiles_n) * 64, n0 = (t % tiles_n) * 64;
+  // Tiles run through panels of `panel` columns, row by row inside a panel: an XCD's contiguous run of them is then close
+  // to a square, the shape that reads the fewest rows of A and W into its L2 (row by row over all columns, each XCD read
+  // nearly all of W: fc1 of one image took 20.4 us instead of 16.5, a 577-row fc2 10.9 instead of 9.2).
+  const int tiles_m = (M + 63) / 64, p = t / (panel * tiles_m), in_p = t - p * panel * tiles_m;
+  const int width = min(panel, tiles_n - p * panel);
+  const int m0 = in_p / width * 64, n0 = (p * panel + in_p % width) * 64;
   const int a_bytes = buf_bytes(static_cast<int64_t>(M - m0) * K), w_bytes = buf_bytes(static_cast<int64_t>(N - n0) * K);
   const int8_t* abase = args.A + static_cast<int64_t>(m0) * K;
   const int8_t* wbase = args.W + static_cast<int64_t>(n0) * K;
@@ -908,13 +914,22 @@ static int launch_ksplit(const GemmArgs& a, int epi, hipStream_t st) {
   const int64_t blocks = static_cast<int64_t>((a.M + 63) / 64) * ((a.N + 63) / 64);
   if (blocks > 0x7fffffff) return fail(FF_EINVAL, "gemm_s8: too many tiles");
   const dim3 grid(static_cast<unsigned>(blocks));
+  // 1, 2, 4 or 8 panels (so that the eight XCDs' runs do not straddle them more than they must), as close as these come
+  // to the side of a square of an eighth of the tiles
+  const int tiles_n = (a.N + 63) / 64;
+  const double side = std::sqrt(static_cast<double>(blocks) / 8.0);
+  int panel = tiles_n;
+  for (int np = 2; np <= 8; np *= 2) {
+    const int w = (tiles_n + np - 1) / np;
+    if (std::abs(std::log(w / side)) < std::abs(std::log(panel / side))) panel = w;
+  }
   switch (epi) {
-    case FF_EPI_QKV_ROPE: gemm_s8_ksplit_kernel<FF_EPI_QKV_ROPE><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_RESIDUAL: gemm_s8_ksplit_kernel<FF_EPI_RESIDUAL><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_GELU_F16: gemm_s8_ksplit_kernel<FF_EPI_GELU_F16><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_SWIGLU: gemm_s8_ksplit_kernel<FF_EPI_SWIGLU><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_BIAS_F16: gemm_s8_ksplit_kernel<FF_EPI_BIAS_F16><<<grid, 256, 0, st>>>(a); break;
-    case FF_EPI_I32: gemm_s8_ksplit_kernel<FF_EPI_I32><<<grid, 256, 0, st>>>(a); break;
+    case FF_EPI_QKV_ROPE: gemm_s8_ksplit_kernel<FF_EPI_QKV_ROPE><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_RESIDUAL: gemm_s8_ksplit_kernel<FF_EPI_RESIDUAL><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_GELU_F16: gemm_s8_ksplit_kernel<FF_EPI_GELU_F16><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_SWIGLU: gemm_s8_ksplit_kernel<FF_EPI_SWIGLU><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_BIAS_F16: gemm_s8_ksplit_kernel<FF_EPI_BIAS_F16><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_I32: gemm_s8_ksplit_kernel<FF_EPI_I32><<<grid, 256, 0, st>>>(a, panel); break;
     default: return fail(FF_EINVAL, "gemm_s8: bad epilogue");
   }
   return check_launch("gemm_s8");
