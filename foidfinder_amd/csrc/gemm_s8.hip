@@ -1354,8 +1354,8 @@ constexpr VariantCost kCost[kVariants] = {
 };
 
 // A variant by M alone (6 below 4096 rows, 3 below 16384, then 4), unless another's estimate is lower by more than the
-// fit's error. Against the fastest variant of each timed product the pick is 1 % slower on average; by M alone it was
-// 14 %, and 138 % at worst: qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. (The lowest
+// fit's error. Against the fastest variant of each timed product the pick is 0.3 % slower on average and 15 % at worst; by
+// M alone it was 14 and 138 %: qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. (The lowest
 // estimate as it stands took variant 2 for Haruka's qkv at 16 images, 3 % slower than 4 there.) Every variant's results
 // are the same bits.
 static int pick_variant(int64_t M, int64_t N, int64_t K) {
