@@ -5,7 +5,8 @@
 // kernel is a weight stream: a persistent grid whose waves each take a 16-tag tile, load 12 of its 16 x 32 fragments
 // straight from global memory into registers (12 KB in flight per wave) and multiply them with v_mfma_f32_16x16x32_f16
 // by x's fragments, which every workgroup keeps in LDS in fragment order. x's rows are padded to 16, 32 or 64. Sums,
-// bias and result stay fp32.
+// bias and result stay fp32. Haruka's head at 16 images: 44.7-48 us (5.1-4.7 TB/s; the library product 89 us); EVA02-L's at
+// one image 13.3 us with its norm (library 13.0, and five launches of 4-5 us for the norm and the casts).
 #include <algorithm>
 
 #include "common.h"

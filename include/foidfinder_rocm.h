@@ -118,7 +118,7 @@ int ff_slot_weights(const void* logits, const float* c, int64_t c_stride, const 
  * and weights fp16, sums, biases and masses fp32.
  *
  * ff_pool_weights: ff_slot_weights with the logits' product in it: l[m] = xn[b, n] . u[b, h*M + m] + c[...], u fp16
- * [B, G*M, D] (u_stride elements between batches, 0: shared), M = 6 or 18, G*M <= 384, N <= 2^18. a_t fp16
+ * [B, G*M, D] (u_stride elements between batches, 0: shared), M = 6 or 18, G*M <= 384, N*D <= 2^30. a_t fp16
  * [B, G*M, ldt] (ldt even, from N to the next multiple of 8; pad columns 0), partial fp32
  * [B, ff_pool_weights_blocks(N), G*M]. */
 int64_t ff_pool_weights_blocks(int64_t N);

@@ -137,7 +137,7 @@ def test_pool_chain(dev, B, C, Q, G, D, F):
 
 
 @pytest.mark.parametrize(("batch", "pool_heads", "leaf_dim"), [(1, 16, 64), (5, 8, 16), (3, 6, 64), (2, 16, 20)])
-def test_pool_head_matches_library_chain(dev, batch, pool_heads, leaf_dim):
+def test_pool_head_matches_library_chain(dev, monkeypatch, batch, pool_heads, leaf_dim):
     """A whole pool head on its own kernels against the library chain, which also serves the shapes that are not whole
     16-column tiles (leaves of 20 here: refused by the rule)."""
     dim = 384 if pool_heads == 6 else 768
@@ -151,11 +151,7 @@ def test_pool_head_matches_library_chain(dev, batch, pool_heads, leaf_dim):
     assert got.shape == (batch, 100) and torch.isfinite(got).all()
     if not eng.fused_pool:
         return
-    eng.fused_pool = False
-    d, hd, Q = dim, dim // pool_heads, cfg.leaves
-    eng.coarse_uT = eng.coarse_u.t().contiguous()
-    eng.pool_vT = eng.pool_v.view(pool_heads, hd, d).transpose(1, 2).contiguous()
-    eng.leaf_w = eng.leaf_wT.transpose(1, 2).contiguous()
+    monkeypatch.setattr(eng, "_pool_leaves", eng._pool_leaves_library)
     want = eng.pool_head(x)
     # the library chain rounds its logits, products and masses to fp16 at a dozen points: 4e-3 of the result's size
     rel = ((got - want).double().norm() / want.double().norm()).item()
