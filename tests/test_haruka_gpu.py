@@ -234,6 +234,36 @@ def test_gpu_bicubic_taps_are_the_host_taps(dev, width, height):
         assert np.array_equal(g.cpu().numpy(), a)
 
 
+def test_uploads_from_threads_and_streams(dev):
+    """The letterbox's pinned uploads: six threads on streams of their own, more than the buffers kept, sizes that grow a
+    buffer and one past its limit, the host array overwritten right after each call; every copy is the array it was given,
+    and no more than BUFFERS buffers stay."""
+    import threading
+
+    from foidfinder_amd.backends.rocm.preprocess import _Uploads
+
+    up, bad = _Uploads(), []
+
+    def work(seed):
+        r = np.random.default_rng(seed)
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for n in [1, 1000, 300_000, 7, 5_000_000, 64, up.LIMIT + 3 if seed == 0 else 4096]:
+                a = r.integers(0, 256, n, dtype=np.uint8)
+                want = a.copy()
+                t = up.put(torch.from_numpy(a), dev)
+                a[:] = 0
+                if not np.array_equal(t.cpu().numpy(), want):
+                    bad.append((seed, n))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad and 0 < len(up.free) <= up.BUFFERS
+
+
 @pytest.mark.parametrize(("w", "h"), RESIZE_CASES)
 def test_gpu_letterbox_is_bit_exact_with_pillow(dev, w, h):
     """The Haruka letterbox on the GPU (ff_resample_u8, two passes) against the oracle's letterbox in the pass order of
