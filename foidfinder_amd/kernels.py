@@ -426,8 +426,9 @@ def head_fits(rows: int, W: torch.Tensor) -> bool:
 
 def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor, gamma: torch.Tensor | None = None,
          beta: torch.Tensor | None = None, eps: float = 1e-6) -> None:
-    """Tag head: out fp32 [B, N] = LN(x) W^T + bias, x fp16 [B, K] with contiguous rows (any row stride that is a
-    multiple of 8), W fp16 [N, K], bias fp16 [N]; the norm (fp32 gamma, beta [K]) only if given (ff_head)."""
+    """Tag head: out fp32 [B, N] = LN(x) W^T + bias, x fp16 [B, K] with contiguous rows (any row stride from K up that is
+    a multiple of 8; rows that overlap are refused), W fp16 [N, K], bias fp16 [N]; the norm (fp32 gamma, beta [K]) only if
+    given (ff_head)."""
     dev = _on_gpu(W, bias, out, gamma, beta)
     B, K = x.shape
     N = W.size(0)
@@ -438,7 +439,8 @@ def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor
     if gamma is not None:
         _require(beta is not None, "gamma and beta go together")
         _float(K, gamma, beta)
-    _run("ff_head", dev, _ptr(x), max(x.stride(0), K), _ptr(gamma), _ptr(beta), eps, _ptr(W), _ptr(bias), B, N, K,
+    stride = x.stride(0) if B > 1 else K  # a single row's stride says nothing
+    _run("ff_head", dev, _ptr(x), stride, _ptr(gamma), _ptr(beta), eps, _ptr(W), _ptr(bias), B, N, K,
          _ptr(out))
 
 

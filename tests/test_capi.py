@@ -142,3 +142,20 @@ def test_pool_kernels_reject_bad_arguments():
     assert "LDS" in sw(G=64)[1]
     assert "null" in sw(ptrs=None)[1]
     assert sw(B=0) == (FF_OK, "")
+
+
+def test_head_hands_the_row_stride_of_several_rows_to_the_library(monkeypatch):
+    """Rows closer than K (an expanded or overlapping view) must reach ff_head's own check as they are: with any larger
+    stride the kernel would read rows that the tensor does not hold. One row's stride is never used."""
+    strides = []
+    monkeypatch.setattr(K, "_on_gpu", lambda *ts: 0)
+    monkeypatch.setattr(K, "_run", lambda name, dev, x, x_stride, *rest: strides.append(x_stride))
+    w, b = torch.zeros(48, 64, dtype=torch.half), torch.zeros(48, dtype=torch.half)
+    flat = torch.zeros(1000, dtype=torch.half)
+    for x in (flat[:64].expand(16, 64), flat.as_strided((3, 64), (8, 1)), flat.as_strided((3, 64), (72, 1)),
+              flat.as_strided((3, 64), (67, 1)), flat.as_strided((1, 64), (3, 1)), flat[:0].view(0, 64)):
+        K.head(x, w, b, torch.zeros(x.size(0), 48))
+    assert strides == [0, 8, 72, 67, 64, 64]
+    for s in (0, 8, 67):
+        status, msg = err(K.lib().ff_head(256, s, None, None, 1e-6, 256, 256, 3, 48, 64, 256, None))
+        assert status == FF_EINVAL and "x_stride" in msg

@@ -54,6 +54,18 @@ def test_head(dev, B, N, K_, norm):
     assert ((out.double() - want).abs() <= bound).all()
 
 
+def test_head_refuses_overlapping_rows(dev):
+    """Refused on the host before any launch; one row is taken whatever its stride is."""
+    w, b, flat = randn(dev, 48, 64, std=0.05).half(), randn(dev, 48).half(), randn(dev, 256, seed=1).half()
+    for x in (flat[:64].expand(16, 64), flat.as_strided((3, 64), (8, 1)), flat.as_strided((3, 64), (65, 1))):
+        with pytest.raises(RuntimeError, match="x_stride"):
+            K.head(x, w, b, torch.empty(x.size(0), 48, device=dev))
+    one, two = torch.empty(1, 48, device=dev), torch.empty(1, 48, device=dev)
+    K.head(flat.as_strided((1, 64), (3, 1)), w, b, one)
+    K.head(flat[:64].view(1, 64), w, b, two)
+    assert torch.equal(one, two)
+
+
 @pytest.mark.parametrize(("B", "N", "G", "M", "D"), [(1, 1, 16, 6, 768), (2, 96, 16, 18, 768), (3, 97, 4, 18, 128),
                                                      (1, 193, 20, 18, 640), (2, 95, 64, 6, 1024)])
 @pytest.mark.parametrize("shared", [True, False])
