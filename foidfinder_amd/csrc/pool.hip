@@ -59,11 +59,14 @@ __global__ __launch_bounds__(256) void layer_norm2_kernel(const half_t* __restri
     if (64 * k + lane < C) orow[64 * k + lane] = static_cast<half_t>(v[k]);
 }
 
+// Eight fp16 values at any multiple of 8 bytes: one 16-byte global load or store (they need no more than 4-byte alignment).
+typedef half8_t half8_a8 __attribute__((aligned(8)));
+
 // The same two norms for C = 256 CH (Haruka's 768): a row per 32-lane half-wave, lane l the 8 columns 8 (l + 32 k) .. of
 // each 256, so a load or store moves 16 bytes per lane, the reductions need no step across the halves, and each serves
-// two rows. Half-waves stream rows with the four affine vectors in registers and the next row's loads in flight. Same
-// arithmetic as layer_norm2_kernel; only the order of the sums differs. 16 400 x 768: 12.6 us (4.0 TB/s); a wave per row with
-// 8-byte pieces took 17.8.
+// two rows. Half-waves stream rows with the four affine vectors in registers and the next row's loads in flight. The sums
+// run in another order than layer_norm2_kernel's, and the squares and the affine step are fused multiply-adds (one
+// rounding less each). 16 400 x 768: 12.6 us (4.0 TB/s); a wave per row with 8-byte pieces took 17.8.
 template <int CH>
 __global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __restrict__ x, int64_t T,
                                                               const half_t* __restrict__ g1,
@@ -77,17 +80,17 @@ __global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __re
   half8_t ga[CH], ba[CH], gb[CH], bb[CH], nxt[CH];
   auto load = [&](int64_t r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < CH; ++k) nxt[k] = *reinterpret_cast<const half8_t*>(x + r * C + 8 * (lane + 32 * k));
+    for (int k = 0; k < CH; ++k) nxt[k] = *reinterpret_cast<const half8_a8*>(x + r * C + 8 * (lane + 32 * k));
   };
   int64_t row = static_cast<int64_t>(blockIdx.x) * 8 + (threadIdx.x >> 5);
   if (row < T) load(row);
 #pragma unroll
   for (int k = 0; k < CH; ++k) {
     const int c = 8 * (lane + 32 * k);
-    ga[k] = *reinterpret_cast<const half8_t*>(g1 + c);
-    ba[k] = *reinterpret_cast<const half8_t*>(b1 + c);
-    gb[k] = *reinterpret_cast<const half8_t*>(g2 + c);
-    bb[k] = *reinterpret_cast<const half8_t*>(b2 + c);
+    ga[k] = *reinterpret_cast<const half8_a8*>(g1 + c);
+    ba[k] = *reinterpret_cast<const half8_a8*>(b1 + c);
+    gb[k] = *reinterpret_cast<const half8_a8*>(g2 + c);
+    bb[k] = *reinterpret_cast<const half8_a8*>(b2 + c);
   }
   constexpr float inv_c = 1.f / static_cast<float>(C);
   auto half_sum = [](float v) __attribute__((always_inline)) {
@@ -135,7 +138,7 @@ __global__ __launch_bounds__(256) void layer_norm2_vec_kernel(const half_t* __re
       half8_t h;
 #pragma unroll
       for (int t = 0; t < 8; ++t) h[t] = static_cast<half_t>(v[k][t]);
-      *reinterpret_cast<half8_t*>(out + row * C + 8 * (lane + 32 * k)) = h;
+      *reinterpret_cast<half8_a8*>(out + row * C + 8 * (lane + 32 * k)) = h;
     }
   }
 }
@@ -245,9 +248,9 @@ extern "C" int ff_layer_norm2(const void* x, int64_t T, int64_t C, const void* g
   const auto *pg2 = static_cast<const half_t*>(g2), *pb2 = static_cast<const half_t*>(b2);
   auto* po = static_cast<half_t*>(out);
   const int Ci = static_cast<int>(C);
-  const auto aligned16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const bool vec = C % 256 == 0 && C <= 1024 && aligned16(x) && aligned16(g1) && aligned16(b1) && aligned16(g2) &&
-                   aligned16(b2) && aligned16(out);
+  const auto aligned8 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 8 == 0; };
+  const bool vec = C % 256 == 0 && C <= 1024 && aligned8(x) && aligned8(g1) && aligned8(b1) && aligned8(g2) &&
+                   aligned8(b2) && aligned8(out);
   if (vec) {
     const dim3 vgrid(static_cast<unsigned>(std::min<int64_t>((T + 7) / 8, 1024)));  // rows past that are streamed
     switch (C / 256) {

@@ -463,13 +463,14 @@ def test_attention_identical_keys_give_mean_of_values(dev, rng):
 
 
 def test_layer_norm2_matches_two_float_layer_norms(dev, rng):
-    """ff_layer_norm2 against two float64 LayerNorms with the fp16 rounding between them: the 8-byte-vector kernel
-    (C % 256 == 0 up to 1024, also with more rows than its grid has waves) and the per-column kernel (2048, 64, and
-    768 on a tensor that starts 2 bytes past an 8-byte boundary)."""
+    """ff_layer_norm2 against two float64 LayerNorms with the fp16 rounding between them: the half-wave kernel (C % 256
+    == 0 up to 1024, each of its four widths, an odd row in a wave, more rows than its grid has half-waves, and tensors
+    that start 8 bytes past a 16-byte boundary) and the per-column kernel (2048, 64, and 768 on a tensor that starts 2
+    bytes past an 8-byte boundary)."""
     from foidfinder_amd import kernels as K
 
     for T, C, shift in ((300, 768, 0), (8300, 768, 0), (7, 1024, 0), (3, 256, 0), (5, 2048, 0), (1, 64, 0),
-                        (9, 768, 1)):
+                        (9, 768, 1), (41, 512, 0), (11, 512, 4), (8301, 768, 4), (6, 1024, 4), (5, 256, 4)):
         x = (rng.standard_normal((T, C)) * 3 + 0.5).astype(np.float16)
         g1, b1, g2, b2 = ((1 + 0.1 * rng.standard_normal(C)).astype(np.float16), (0.1 * rng.standard_normal(C)).astype(np.float16),
                           (1 + 0.1 * rng.standard_normal(C)).astype(np.float16), (0.1 * rng.standard_normal(C)).astype(np.float16))
