@@ -232,6 +232,22 @@ class Int8Engine:
     def _forward(self, img: torch.Tensor, buf: dict[str, torch.Tensor], trace: dict | None = None) -> torch.Tensor:
         raise NotImplementedError
 
+    def _pixels(self, img: torch.Tensor) -> torch.Tensor:
+        """The images as ff_patch_embed reads them: fp16 [B, S, S, 3], contiguous, from a multiple of 4 bytes. Takes the
+        dtypes, shapes, strides and storage offsets that patchify takes, and refuses what its library product would: a
+        tensor that autograd follows."""
+        if img.requires_grad and torch.is_grad_enabled():
+            raise RuntimeError("the int8 engines have no backward: call them under torch.no_grad() or detach the images")
+        B, g, p = img.shape[0], self.cfg.grid, self.cfg.patch
+        x = img.to(torch.half).view(B, g, p, g, p, 3).reshape(B, g * p, g * p, 3).contiguous()
+        return x if x.data_ptr() % 4 == 0 else x.clone()
+
+    def _patch_embed(self, img: torch.Tensor, bias_pos: torch.Tensor, cls: torch.Tensor, x: torch.Tensor) -> None:
+        """x [B, tokens, d] = class row and patch embeddings, on the stem kernel (at most 65535 images a launch)."""
+        px, most = self._pixels(img), 65535
+        for b in range(0, px.size(0), most):
+            self.k.patch_embed(px[b : b + most], self.patch_w, bias_pos, cls, x[b : b + most])
+
     def _gemm(self, a, lw, rs, epi, variant, out, rope=None):
         w, ws, b = lw
         cos, sin = rope if rope is not None else (None, None)
@@ -401,7 +417,7 @@ class Eva02Int8(Int8Engine):
         x, a8, rs = buf["x"], buf["a8"], buf["rs"]
         xv = x.view(B, L, d)
         if self.fused_stem:
-            k.patch_embed(img.to(torch.half).contiguous(), self.patch_w, self.patch_bias_pos, self.cls_pos, xv)
+            self._patch_embed(img, self.patch_bias_pos, self.cls_pos, xv)
         else:
             torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
             torch.add(buf["patch"].view(B, L - 1, d), self.patch_bias_pos, out=xv[:, 1:])

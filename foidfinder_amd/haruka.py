@@ -416,7 +416,7 @@ class HarukaInt8(Int8Engine):
         x, a8, rs = buf["x"], buf["a8"], buf["rs"]
         xv = x.view(B, L, d)
         if self.fused_stem:
-            k.patch_embed(img.to(torch.half).contiguous(), self.patch_w, self.patch_b, self.cls, xv)
+            self._patch_embed(img, self.patch_b, self.cls, xv)
         else:
             torch.matmul(self.patchify(img), self.patch_w_t, out=buf["patch"])
             torch.add(buf["patch"].view(B, L - 1, d), self.patch_b, out=xv[:, 1:])

@@ -323,3 +323,15 @@ def test_full_depth_eva02_l_end_to_end(dev):
         assert all(np.argmax(served[i]) == np.argmax(ref[i]) for i in range(n)), report
         checked, bad = gap_filtered_topk(served, ref)
         assert checked > 0 and not bad, report
+
+
+def test_eager_takes_the_images_that_patchify_takes(dev):
+    """An eager call on strided, flat or misaligned views gives the bits of the same pixels laid out plainly."""
+    from foidfinder_amd.engine import Eva02Int8
+    from test_host import image_forms
+
+    cfg = engine_cfg(depth=1, img=42, tags=32)
+    eng = Eva02Int8(raw_and_converted(cfg)[1], cfg, device=dev)
+    for what, img in image_forms(2, 42, dev):
+        plain = eng.patchify(img).view(2, 3, 3, 14, 14, 3).permute(0, 1, 3, 2, 4, 5).reshape(2, 42, 42, 3).contiguous()
+        assert torch.equal(eng.eager(img), eng.eager(plain)), what

@@ -112,3 +112,60 @@ def test_model_dir_round_trip(tmp_path):
 def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def image_forms(B, S, device="cpu"):
+    """(what, images) forms that the engines' patchify takes: dtypes, strides, storage offsets and shapes."""
+    g = torch.Generator().manual_seed(B)
+    base = (torch.rand(B, S, S, 3, generator=g) * 255).to(device)
+    half = base.half()
+    shifted = torch.zeros(half.numel() + 1, dtype=torch.half, device=device)[1:].view_as(half).copy_(half)
+    wide = torch.zeros(B, S + 3, S + 5, 4, dtype=torch.half, device=device)
+    wide[:, 1 : S + 1, 2 : S + 2, :3] = half
+    return [("fp16", half), ("fp32", base), ("float64", base.double()), ("uint8", base.byte()),
+            ("two bytes past a word", shifted), ("crop of a larger image", wide[:, 1 : S + 1, 2 : S + 2, :3]),
+            ("channels first in memory", half.permute(0, 3, 1, 2).contiguous().permute(0, 2, 3, 1)),
+            ("repeated image", half[:1].expand(B, S, S, 3)), ("rows of one axis", half.view(B, S, S * 3)),
+            ("flat", half.view(B, -1)), ("patch grid", wide[:, 1 : S + 1, 2 : S + 2, :3].view(B, S // 14, 14, S // 14, 14, 3))]
+
+
+def bare_engine(S):
+    eng = object.__new__(E.Eva02Int8)
+    eng.cfg = E.Eva02Config(img_size=S)
+    return eng
+
+
+@pytest.mark.parametrize(("B", "S"), [(1, 14), (3, 42)])
+def test_stem_takes_the_images_that_patchify_takes(B, S):
+    """What the stem kernel is handed is contiguous fp16 [B, S, S, 3] from a multiple of 4 bytes, and holds the pixels
+    that patchify reads; shapes that patchify refuses and images that autograd follows are refused."""
+    eng = bare_engine(S)
+    for what, img in image_forms(B, S):
+        px = eng._pixels(img)
+        assert px.shape == (B, S, S, 3) and px.dtype == torch.half and px.is_contiguous(), what
+        assert px.data_ptr() % 4 == 0, what
+        assert torch.equal(eng.patchify(px), eng.patchify(img)), what
+    for bad in (torch.zeros(B, S, S, 4), torch.zeros(B, S + 14, S, 3), torch.zeros(B, S, S)):
+        for f in (eng.patchify, eng._pixels):
+            with pytest.raises(RuntimeError):
+                f(bad)
+    followed = torch.zeros(B, S, S, 3, requires_grad=True)
+    with pytest.raises(RuntimeError, match="backward"):
+        eng._pixels(followed)
+    with torch.no_grad():
+        assert eng._pixels(followed).shape == (B, S, S, 3)
+
+
+def test_stem_splits_batches_past_a_launch():
+    """More images than one launch takes run in slices that cover every image once."""
+    eng, B = bare_engine(14), 65535 * 2 + 3
+    calls = []
+
+    class Ops:
+        @staticmethod
+        def patch_embed(px, w, bias_pos, cls, x):
+            calls.append((px.size(0), x.size(0), x.storage_offset()))
+
+    eng.k, eng.patch_w = Ops, None
+    eng._patch_embed(torch.zeros(1, 14, 14, 3, dtype=torch.half).expand(B, 14, 14, 3), None, None, torch.zeros(B, 2, 8))
+    assert calls == [(65535, 65535, 0), (65535, 65535, 65535 * 16), (3, 3, 2 * 65535 * 16)]
