@@ -106,6 +106,13 @@ class _Uploads:
         self.lock = threading.Lock()
         self.free: list[tuple[torch.Tensor, torch.cuda.Event]] = []  # oldest first
 
+    @staticmethod
+    def _buffer(n: int) -> torch.Tensor:
+        """A pinned buffer of at least n bytes that serves later calls too: on the host whatever torch's default device
+        is, and no inference tensor, which calls outside the inference mode could not write."""
+        with torch.inference_mode(False):
+            return torch.empty(1 << (n - 1).bit_length(), dtype=torch.uint8, device="cpu", pin_memory=True)
+
     def put(self, host: torch.Tensor, device: torch.device) -> torch.Tensor:
         n = host.numel()
         if device.type != "cuda" or not 0 < n <= self.LIMIT:
@@ -117,7 +124,7 @@ class _Uploads:
         if buf is not None:
             event.synchronize()
         if buf is None or buf.numel() < n:
-            buf = torch.empty(1 << (n - 1).bit_length(), dtype=torch.uint8, pin_memory=True)
+            buf = self._buffer(n)
         staged = buf[:n].view(host.shape)
         staged.copy_(host)
         with torch.cuda.device(device):

@@ -284,6 +284,21 @@ def test_taps_window_is_the_taps_bounds():
             assert taps_window(n_in, n_out, i) == (b[i, 0], b[i].sum())
 
 
+def test_staging_buffers_do_not_follow_the_callers_modes(monkeypatch):
+    """A staging buffer outlives the call that makes it: it must be writable outside an inference mode that it was made
+    in, and lie on the host under a default device."""
+    from foidfinder_amd.backends.rocm.preprocess import _Uploads
+
+    real = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: real(*a, **kw))  # no GPU, no pinned memory
+    with torch.inference_mode():
+        buf = _Uploads._buffer(100)
+    assert not buf.is_inference() and buf.numel() == 128
+    buf[:3].copy_(torch.arange(3, dtype=torch.uint8))
+    with torch.device("meta"):
+        assert _Uploads._buffer(1).device.type == "cpu"
+
+
 def test_bicubic_taps_match_the_pillow_known_answers():
     """The reference's own Pillow tap tables (web/src/engine/engine.test.ts:8-34), kept as a fixture."""
     from pathlib import Path

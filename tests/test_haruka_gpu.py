@@ -264,6 +264,28 @@ def test_uploads_from_threads_and_streams(dev):
     assert not bad and 0 < len(up.free) <= up.BUFFERS
 
 
+def test_letterbox_across_inference_mode_and_default_device(dev):
+    """The staging buffers that a call under inference_mode leaves serve later calls outside it, and a default device
+    changes nothing."""
+    from foidfinder_amd.backends.rocm.preprocess import _uploads, letterbox_gpu
+
+    image = np.random.default_rng(3).integers(0, 256, (60, 90, 3), dtype=np.uint8)
+
+    def run():
+        out = torch.empty(56, 56, 3, dtype=torch.uint8, device=dev)
+        letterbox_gpu(image, 56, out)
+        return out.cpu().numpy()
+
+    _uploads.free.clear()
+    with torch.inference_mode():
+        first = run()
+    torch.cuda.synchronize()
+    assert np.array_equal(run(), first)
+    _uploads.free.clear()
+    with torch.device(dev):
+        assert np.array_equal(run(), first)
+
+
 @pytest.mark.parametrize(("w", "h"), RESIZE_CASES)
 def test_gpu_letterbox_is_bit_exact_with_pillow(dev, w, h):
     """The Haruka letterbox on the GPU (ff_resample_u8, two passes) against the oracle's letterbox in the pass order of
