@@ -803,8 +803,57 @@ __device__ __forceinline__ void tail_block(const GemmArgs& args, int m_first, in
 constexpr int KS_CHUNK = 128 * 64;     // one staged chunk: 64 A rows + 64 W rows x 64 K bytes
 constexpr int KS_PART = 64 * 64 * 4;   // one wave's 64 x 64 int32 partial tile
 
+// The order of the 64 x 64 tiles: the columns are split into panels and tiles run row by row inside a panel, so that an
+// XCD's contiguous run of them is close to a square, the shape that reads the fewest rows of A and W into its L2 (row by
+// row over all columns, each XCD reads nearly all of W: fc1 of one image took 20.4 us instead of 16.5, a 577-row fc2 10.9
+// instead of 9.2).
+//
+// share >= 0: 8 >> share panels, the columns split as evenly as they go; 1 << share whole XCDs share a panel's tiles, the
+// grid is eight times the longest run, and blocks past their XCD's run leave at once. share < 0: panels of `width`
+// columns, one sequence over all of them cut into eighths. There a run that crosses into the next panel ends with tiles
+// whose rows nothing else on the XCD reads, and where some CUs get a second block, those late blocks decide the launch:
+// K = 2816, N = 768, M = 1455 (276 tiles, two panels) 13.7 us, whole XCDs 11.7, over all columns 11.9.
+struct KsOrder {
+  int share, width;
+  int64_t grid;
+};
+
+// Whole XCDs where the 1, 2, 4 or 8 panels closest to squares leave the longest run at one block per CU (32) or near an
+// even share. Columns that do not split that evenly (25 of them, say) run as one sequence where that is free of the late
+// blocks (at most a block per CU) or drowns them (half the CUs or more have two), else in the closest split that does.
+// Near is 6 % where the late blocks count, else 3 % (N = 1600, M = 2600, split 4 % unevenly, runs 4-5 % behind the
+// sequence). Over 980 products (N 768-4096, K 768-4736, M 64-4095) the mean time is 0.88 of the order over all columns and
+// the worst 1.05 (four above 1.03); one sequence of the same panels everywhere has 0.90, 1.20 and 23 above 1.05.
+static KsOrder ks_order(int64_t M, int64_t N) {
+  const int64_t tiles_m = (M + 63) / 64, tiles_n = (N + 63) / 64, blocks = tiles_m * tiles_n, even = (blocks + 7) / 8;
+  auto run = [&](int lg) {
+    int64_t r = 0;
+    for (int64_t p = 0; p < 1 << lg; ++p) {
+      const int64_t tiles = (((p + 1) * tiles_n >> lg) - (p * tiles_n >> lg)) * tiles_m;
+      r = std::max(r, (tiles + (8 >> lg) - 1) >> (3 - lg));
+    }
+    return r;
+  };
+  const bool late = blocks > 256 && blocks <= 384;
+  auto fits = [&](int lg) { return run(lg) <= 32 || run(lg) * 100 <= even * (late ? 106 : 103); };
+  const double side = std::sqrt(static_cast<double>(blocks) / 8.0);
+  int best[2] = {0, 0};  // closest to squares: of all splits, of those that fit
+  double off[2];
+  for (int lg = 0; lg < 4 && (1 << lg) <= tiles_n; ++lg) {
+    const double o = std::abs(std::log(static_cast<double>(tiles_n) / (1 << lg) / side));
+    for (int f = 0; f < 2; ++f) {
+      if (lg > 0 && (o >= off[f] || (f == 1 && !fits(lg)))) continue;
+      best[f] = lg;
+      off[f] = o;
+    }
+  }
+  if (best[0] != best[1] && !late)
+    return {-1, static_cast<int>((tiles_n + (1 << best[0]) - 1) >> best[0]), blocks};
+  return {3 - best[1], 0, 8 * run(best[1])};
+}
+
 template <int EPI>
-__global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs args, int panel) {
+__global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs args, int share, int panel) {
   constexpr int WV = 4;          // waves per block
   constexpr int SLOTS = WV / 2;  // partial slots in the chunk buffers
   static_assert(stage_bytes<EPI, 1>() <= KS_CHUNK, "a quadrant's staging fits its wave's chunk buffer");
@@ -814,13 +863,22 @@ __global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs a
   const int fr = lane & 31, fk = lane >> 5;
   const int M = args.M, N = args.N, K = args.K, nch = K / 64;
   const int tiles_n = (N + 63) / 64;
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
-  // Tiles run through panels of `panel` columns, row by row inside a panel: an XCD's contiguous run of them is then close
-  // to a square, the shape that reads the fewest rows of A and W into its L2 (row by row over all columns, each XCD read
-  // nearly all of W: fc1 of one image took 20.4 us instead of 16.5, a 577-row fc2 10.9 instead of 9.2).
-  const int tiles_m = (M + 63) / 64, p = t / (panel * tiles_m), in_p = t - p * panel * tiles_m;
-  const int width = min(panel, tiles_n - p * panel);
-  const int m0 = in_p / width * 64, n0 = (p * panel + in_p % width) * 64;
+  const int tiles_m = (M + 63) / 64;
+  int c0, width, in_p;  // the tile's panel and its place there (see KsOrder)
+  if (share >= 0) {
+    const int xcd = blockIdx.x & 7, p = xcd >> share, j = xcd & ((1 << share) - 1), k = blockIdx.x >> 3;
+    c0 = p * tiles_n >> (3 - share);
+    width = ((p + 1) * tiles_n >> (3 - share)) - c0;
+    const int tiles = width * tiles_m, q = tiles >> share, r = tiles & ((1 << share) - 1);
+    if (k >= q + (j < r)) return;
+    in_p = j * q + min(j, r) + k;
+  } else {
+    const int t = xcd_remap(blockIdx.x, gridDim.x), p = t / (panel * tiles_m);
+    c0 = p * panel;
+    width = min(panel, tiles_n - c0);
+    in_p = t - c0 * tiles_m;
+  }
+  const int m0 = in_p / width * 64, n0 = (c0 + in_p % width) * 64;
   const int a_bytes = buf_bytes(static_cast<int64_t>(M - m0) * K), w_bytes = buf_bytes(static_cast<int64_t>(N - n0) * K);
   const int8_t* abase = args.A + static_cast<int64_t>(m0) * K;
   const int8_t* wbase = args.W + static_cast<int64_t>(n0) * K;
@@ -913,23 +971,16 @@ __global__ __launch_bounds__(256, 4) void gemm_s8_ksplit_kernel(const GemmArgs a
 static int launch_ksplit(const GemmArgs& a, int epi, hipStream_t st) {
   const int64_t blocks = static_cast<int64_t>((a.M + 63) / 64) * ((a.N + 63) / 64);
   if (blocks > 0x7fffffff) return fail(FF_EINVAL, "gemm_s8: too many tiles");
-  const dim3 grid(static_cast<unsigned>(blocks));
-  // 1, 2, 4 or 8 panels (so that the eight XCDs' runs do not straddle them more than they must), as close as these come
-  // to the side of a square of an eighth of the tiles
-  const int tiles_n = (a.N + 63) / 64;
-  const double side = std::sqrt(static_cast<double>(blocks) / 8.0);
-  int panel = tiles_n;
-  for (int np = 2; np <= 8; np *= 2) {
-    const int w = (tiles_n + np - 1) / np;
-    if (std::abs(std::log(w / side)) < std::abs(std::log(panel / side))) panel = w;
-  }
+  const KsOrder o = ks_order(a.M, a.N);
+  if (o.grid > 0x7fffffff) return fail(FF_EINVAL, "gemm_s8: too many tiles");
+  const dim3 grid(static_cast<unsigned>(o.grid));
   switch (epi) {
-    case FF_EPI_QKV_ROPE: gemm_s8_ksplit_kernel<FF_EPI_QKV_ROPE><<<grid, 256, 0, st>>>(a, panel); break;
-    case FF_EPI_RESIDUAL: gemm_s8_ksplit_kernel<FF_EPI_RESIDUAL><<<grid, 256, 0, st>>>(a, panel); break;
-    case FF_EPI_GELU_F16: gemm_s8_ksplit_kernel<FF_EPI_GELU_F16><<<grid, 256, 0, st>>>(a, panel); break;
-    case FF_EPI_SWIGLU: gemm_s8_ksplit_kernel<FF_EPI_SWIGLU><<<grid, 256, 0, st>>>(a, panel); break;
-    case FF_EPI_BIAS_F16: gemm_s8_ksplit_kernel<FF_EPI_BIAS_F16><<<grid, 256, 0, st>>>(a, panel); break;
-    case FF_EPI_I32: gemm_s8_ksplit_kernel<FF_EPI_I32><<<grid, 256, 0, st>>>(a, panel); break;
+    case FF_EPI_QKV_ROPE: gemm_s8_ksplit_kernel<FF_EPI_QKV_ROPE><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
+    case FF_EPI_RESIDUAL: gemm_s8_ksplit_kernel<FF_EPI_RESIDUAL><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
+    case FF_EPI_GELU_F16: gemm_s8_ksplit_kernel<FF_EPI_GELU_F16><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
+    case FF_EPI_SWIGLU: gemm_s8_ksplit_kernel<FF_EPI_SWIGLU><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
+    case FF_EPI_BIAS_F16: gemm_s8_ksplit_kernel<FF_EPI_BIAS_F16><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
+    case FF_EPI_I32: gemm_s8_ksplit_kernel<FF_EPI_I32><<<grid, 256, 0, st>>>(a, o.share, o.width); break;
     default: return fail(FF_EINVAL, "gemm_s8: bad epilogue");
   }
   return check_launch("gemm_s8");

@@ -275,6 +275,22 @@ def test_gemm_s8_k_group_tiles_bit_exact(dev, rng, M, N, K, epi, variant):
     assert bad.size == 0, f"{len(bad)} mismatches, first at {bad[:4].tolist()}"
 
 
+@pytest.mark.parametrize(("M", "N"), [(1, 16), (65, 464), (257, 1600), (577, 1600), (700, 1600), (1455, 768), (1300, 1280),
+                                      (2401, 656), (3500, 1232)])
+def test_gemm_s8_block_orders_bit_exact(dev, rng, M, N):
+    """The 64 x 64 blocks' orders: one tile; panels that whole XCDs share, of unequal width (29 columns in four, 25 in
+    eight, 25 in two), where some CUs take a second block (275, 276 and 420 tiles) and where all do (1100); and one
+    sequence of unequal panels cut into eighths (25 columns in 250 tiles, 11 in 418). Every tile is written: the output
+    starts as another value."""
+    from foidfinder_amd import kernels as Kn
+
+    a, w, rs, cs, bias = gemm_inputs(rng, M, N, 64)
+    out = torch.full((M, N), -7, dtype=torch.int32, device=dev)
+    Kn.gemm_s8(to_gpu(a, dev), to_gpu(w, dev), None, None, None, out, OG.EPI_I32, 6, None, None, 1.0)
+    want = (a.astype(np.float32) @ w.astype(np.float32).T).astype(np.int32)  # exact: sums below 2^24
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
 @pytest.mark.parametrize("variant", GEMM_VARIANTS)
 @pytest.mark.parametrize("rope_len", [1, 5, 8, 65, 200])
 def test_gemm_s8_qkv_short_rope_tables(dev, rng, rope_len, variant):
