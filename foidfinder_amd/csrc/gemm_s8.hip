@@ -1387,11 +1387,12 @@ static int launch_pair(const GemmArgs& a, int epi, hipStream_t st) {
 constexpr int kVariants = 6;
 
 // Estimated time of a variant in us on 256 CUs: a launch, its rounds of tiles over the CUs (each a chain of K slices)
-// and the chip-wide throughput of all tiles. The constants are a non-negative least-squares fit to 2100 timed launches
-// (16 products of the taggers and linears, K 768-4736, N 768-5632, M 1-32800, all epilogues), within 5-9 % rms each.
+// and the chip-wide throughput of all tiles. The constants are non-negative least-squares fits to timed launches (16
+// products of the taggers and linears, K 768-4736, N 768-5632, M 1-32800, all epilogues: 2100 launches for variants 1-5,
+// and 1400 of variant 6 with its present tile order), within 6-10 % rms each on 200 products outside the fits.
 struct VariantCost {
   int bm, bn;         // tile
-  int per_round;      // tiles that run at once
+  int per_round;      // tiles a round, as fitted (variants 2 and 6 keep 512 and 1024 resident)
   double launch;      // us per launch
   double round;       // us per round
   double round_k;     // us per round and 1000 K
@@ -1401,14 +1402,15 @@ struct VariantCost {
 constexpr VariantCost kCost[kVariants] = {
     {128, 128, 256, 2.0, 3.5, 2.6, 0.65, 2.5},  {256, 128, 256, 5.2, 0.4, 6.1, 2.4, 2.3},
     {256, 256, 256, 2.1, 6.0, 7.5, 3.9, 4.75},  {256, 256, 256, 5.0, 2.7, 8.1, 3.6, 5.75},
-    {256, 128, 256, 1.7, 4.3, 4.4, 2.1, 2.8},   {64, 64, 512, 4.0, 0.0, 1.05, 0.245, 1.72},
+    {256, 128, 256, 1.7, 4.3, 4.4, 2.1, 2.8},   {64, 64, 512, 3.9, 0.17, 1.06, 0.37, 1.32},
 };
 
-// A variant by M alone (6 below 4096 rows, 3 below 16384, then 4), unless another's estimate is lower by more than the
-// fit's error. Against the fastest variant of each timed product the pick is 0.3 % slower on average and 15 % at worst; by
-// M alone it was 14 and 138 %: qkv of one image 13.9 -> 10.8 us, fc1 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. (The lowest
-// estimate as it stands took variant 2 for Haruka's qkv at 16 images, 3 % slower than 4 there.) Every variant's results
-// are the same bits.
+// A variant by M alone (6 below 4096 rows, 3 below 16384, then 4), unless another's estimate is lower by a margin: 3 %
+// against variant 6, whose constants are the closest where it is the pick, 6 % against the others (the lowest estimate as
+// it stands took variant 2 for Haruka's qkv at 16 images, 3 % slower than 4 there). On 200 products drawn from the same
+// ranges and not fitted to, the pick is 0.2 % slower than the fastest variant on average and 11 % at worst, and never
+// more than 1 % slower than the one by M; by M alone it would be 9.5 and 111 %: qkv of one image 13.9 -> 10.8 us, fc1
+// 20.2 -> 12.6, PixAI's fc2 48.4 -> 33.4. Every variant's results are the same bits.
 static int pick_variant(int64_t M, int64_t N, int64_t K) {
   auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const double k = static_cast<double>(K) * 1e-3;
@@ -1432,7 +1434,7 @@ static int pick_variant(int64_t M, int64_t N, int64_t K) {
       best_t = t;
     }
   }
-  return best_t < 0.94 * rows_t ? best : by_rows;
+  return best_t < (by_rows == 6 ? 0.97 : 0.94) * rows_t ? best : by_rows;
 }
 
 }  // namespace ff
