@@ -97,8 +97,8 @@ class _Uploads:
     """Host images to the GPU through pinned memory: a threaded copy into a staging buffer and a DMA from it take 13 + 66
     us for 1200 x 900, the runtime's pageable copy 125, and the call returns before the DMA ends. At most BUFFERS staging
     buffers of at most LIMIT bytes are kept, for all threads and streams: a buffer is taken under the lock and handed back
-    with an event recorded behind its DMA on the caller's stream, which its next user waits for; a larger image takes the
-    pageable copy."""
+    with an event recorded behind its DMA on the caller's stream, which its next user waits for. Larger images take the
+    pageable copy, as does a call under graph capture, whose copy would read the shared buffer again on every replay."""
 
     BUFFERS, LIMIT = 4, 16 << 20
 
@@ -114,10 +114,14 @@ class _Uploads:
             return torch.empty(1 << (n - 1).bit_length(), dtype=torch.uint8, device="cpu", pin_memory=True)
 
     def put(self, host: torch.Tensor, device: torch.device) -> torch.Tensor:
-        n = host.numel()
-        if device.type != "cuda" or not 0 < n <= self.LIMIT:
-            return host.to(device)
-        buf = None
+        if device.type == "cuda" and 0 < host.numel() <= self.LIMIT:
+            with torch.cuda.device(device):
+                if not torch.cuda.is_current_stream_capturing():
+                    return self._staged(host, device)
+        return host.to(device)
+
+    def _staged(self, host: torch.Tensor, device: torch.device) -> torch.Tensor:
+        n, buf = host.numel(), None
         with self.lock:
             if len(self.free) >= self.BUFFERS or self.free and self.free[0][1].query():
                 buf, event = self.free.pop(0)
@@ -127,10 +131,9 @@ class _Uploads:
             buf = self._buffer(n)
         staged = buf[:n].view(host.shape)
         staged.copy_(host)
-        with torch.cuda.device(device):
-            out = staged.to(device, non_blocking=True)
-            event = torch.cuda.Event()
-            event.record()
+        out = staged.to(device, non_blocking=True)
+        event = torch.cuda.Event()
+        event.record()
         with self.lock:
             if len(self.free) < self.BUFFERS:
                 self.free.append((buf, event))

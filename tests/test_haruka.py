@@ -299,6 +299,41 @@ def test_staging_buffers_do_not_follow_the_callers_modes(monkeypatch):
         assert _Uploads._buffer(1).device.type == "cpu"
 
 
+def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
+    """A call under graph capture must not touch a shared buffer: its replays would read what later calls put there. It
+    takes the plain copy, as larger images do, and images on the host alone."""
+    import contextlib
+
+    from foidfinder_amd.backends.rocm.preprocess import _Uploads
+
+    up, staged = _Uploads(), []
+    monkeypatch.setattr(up, "_staged", lambda host, device: staged.append(host.numel()) or host)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    capturing = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+
+    class Image:  # stands in for a tensor: no GPU to copy to
+        dtype = torch.uint8
+
+        def __init__(self, n):
+            self.n = n
+
+        def numel(self):
+            return self.n
+
+        def to(self, device):
+            return "plain"
+
+    cuda = torch.device("cuda", 0)
+    up.put(Image(100), cuda)
+    assert staged == [100]
+    capturing[0] = True
+    assert up.put(Image(100), cuda) == "plain"
+    capturing[0] = False
+    assert up.put(Image(0), cuda) == up.put(Image(up.LIMIT + 1), cuda) == up.put(Image(5), torch.device("cpu")) == "plain"
+    assert staged == [100]
+
+
 def test_bicubic_taps_match_the_pillow_known_answers():
     """The reference's own Pillow tap tables (web/src/engine/engine.test.ts:8-34), kept as a fixture."""
     from pathlib import Path
