@@ -301,7 +301,8 @@ def test_staging_buffers_do_not_follow_the_callers_modes(monkeypatch):
 
 def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
     """A call under graph capture must not touch a shared buffer: its replays would read what later calls put there. It
-    takes the plain copy, as larger images do, and images on the host alone."""
+    takes the plain copy, as larger images do, images for the host, and other dtypes, which must reach the resize's own
+    check as they are."""
     import contextlib
 
     from foidfinder_amd.backends.rocm.preprocess import _Uploads
@@ -313,10 +314,8 @@ def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
 
     class Image:  # stands in for a tensor: no GPU to copy to
-        dtype = torch.uint8
-
-        def __init__(self, n):
-            self.n = n
+        def __init__(self, n, dtype=torch.uint8):
+            self.n, self.dtype = n, dtype
 
         def numel(self):
             return self.n
@@ -331,6 +330,7 @@ def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
     assert up.put(Image(100), cuda) == "plain"
     capturing[0] = False
     assert up.put(Image(0), cuda) == up.put(Image(up.LIMIT + 1), cuda) == up.put(Image(5), torch.device("cpu")) == "plain"
+    assert up.put(Image(100, torch.float32), cuda) == up.put(Image(100, torch.int16), cuda) == "plain"
     assert staged == [100]
 
 
