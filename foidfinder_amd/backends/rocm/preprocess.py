@@ -14,6 +14,7 @@ is (foidfinder/backends/mlx/kernels.py:75-186).
 
 from __future__ import annotations
 
+import ctypes
 import math
 import threading
 
@@ -93,6 +94,18 @@ def taps_window(in_size: int, out_size: int, index: int) -> tuple[int, int]:
     return max(math.trunc(center - support + 0.5), 0), min(math.trunc(center + support + 0.5), in_size)
 
 
+def _as_tensor(image: np.ndarray) -> torch.Tensor:
+    """The array as a tensor over the same memory, for reading only; a copy only of an array whose elements are not in
+    order. PIL's arrays cannot be written, of which torch would warn, so such memory goes by its address; the tensor keeps
+    the array alive."""
+    image = np.require(image, requirements="C" if image.size else "CW")
+    if not image.flags.writeable:
+        memory = (ctypes.c_uint8 * image.nbytes).from_address(image.ctypes.data)
+        memory.owner = image
+        image = np.frombuffer(memory, image.dtype).reshape(image.shape)
+    return torch.from_numpy(image)
+
+
 class _Uploads:
     """Host images to the GPU through pinned memory: a threaded copy into a staging buffer and a DMA from it take 13 + 66
     us for 1200 x 900, the runtime's pageable copy 125, and the call returns before the DMA ends. At most BUFFERS staging
@@ -151,7 +164,7 @@ def letterbox_gpu(rgb: np.ndarray, size: int, out: torch.Tensor) -> None:
 
     h, w = rgb.shape[:2]
     dev = out.device
-    src = _uploads.put(torch.from_numpy(np.require(rgb, requirements=["C", "W"])), dev)  # PIL arrays are read-only
+    src = _uploads.put(_as_tensor(rgb), dev)
     if (w, h) == (size, size):
         out.copy_(src)
         return

@@ -284,6 +284,28 @@ def test_taps_window_is_the_taps_bounds():
             assert taps_window(n_in, n_out, i) == (b[i, 0], b[i].sum())
 
 
+@pytest.mark.parametrize("dtype", [np.uint8, np.float32, np.int16])
+def test_images_reach_the_upload_without_a_copy(dtype):
+    """A PIL image's array cannot be written; it is read where it lies, without a warning, and stays alive as long as the
+    tensor over it. Arrays whose elements are not in order are copied into order."""
+    import gc
+    import warnings
+
+    from foidfinder_amd.backends.rocm.preprocess import _as_tensor
+
+    want = np.random.default_rng(0).integers(0, 100, (5, 7, 3)).astype(dtype)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        fixed = np.frombuffer(want.tobytes(), dtype).reshape(want.shape)
+        assert not fixed.flags.writeable and _as_tensor(fixed).data_ptr() == fixed.ctypes.data
+        assert _as_tensor(want).data_ptr() == want.ctypes.data
+        for a in (fixed[:, ::-1], fixed[1:4, 2:5], fixed.transpose(1, 0, 2), want[::2], fixed[:0]):
+            assert np.array_equal(_as_tensor(a).numpy(), a)
+        tensors = [_as_tensor(np.frombuffer(want.tobytes(), dtype).reshape(want.shape)) for _ in range(50)]
+        gc.collect()
+        assert all(np.array_equal(t.numpy(), want) for t in tensors)
+
+
 def test_staging_buffers_do_not_follow_the_callers_modes(monkeypatch):
     """A staging buffer outlives the call that makes it: it must be writable outside an inference mode that it was made
     in, and lie on the host under a default device."""
