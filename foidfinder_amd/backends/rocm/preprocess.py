@@ -110,10 +110,12 @@ class _Uploads:
     """Host images to the GPU through pinned memory: a threaded copy into a staging buffer and a DMA from it take 13 + 66
     us for 1200 x 900, the runtime's pageable copy 125, and the call returns before the DMA ends. At most BUFFERS staging
     buffers of at most LIMIT bytes are kept, for all threads and streams: a buffer is taken under the lock and handed back
-    with an event recorded behind its DMA on the caller's stream, which its next user waits for. Larger images take the
-    pageable copy, as do other dtypes (which the resize refuses) and a call under graph capture, whose copy would read the shared buffer again on every replay."""
+    with an event recorded behind its DMA on the caller's stream, which its next user waits for. The pageable copy takes
+    larger images, images up to LEAST bytes (waking the copy's threads costs more than it saves: preprocess_haruka of 448 x
+    448 in 145 us staged, 127 pageable; at 600 x 448 both 190), other dtypes (which the resize refuses), and calls under
+    graph capture, whose copy would read the shared buffer again on every replay."""
 
-    BUFFERS, LIMIT = 4, 16 << 20
+    BUFFERS, LEAST, LIMIT = 4, 640 << 10, 16 << 20
 
     def __init__(self):
         self.lock = threading.Lock()
@@ -127,7 +129,7 @@ class _Uploads:
             return torch.empty(1 << (n - 1).bit_length(), dtype=torch.uint8, device="cpu", pin_memory=True)
 
     def put(self, host: torch.Tensor, device: torch.device) -> torch.Tensor:
-        if device.type == "cuda" and host.dtype == torch.uint8 and 0 < host.numel() <= self.LIMIT:
+        if device.type == "cuda" and host.dtype == torch.uint8 and self.LEAST < host.numel() <= self.LIMIT:
             with torch.cuda.device(device):
                 if not torch.cuda.is_current_stream_capturing():
                     return self._staged(host, device)

@@ -323,8 +323,8 @@ def test_staging_buffers_do_not_follow_the_callers_modes(monkeypatch):
 
 def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
     """A call under graph capture must not touch a shared buffer: its replays would read what later calls put there. It
-    takes the plain copy, as larger images do, images for the host, and other dtypes, which must reach the resize's own
-    check as they are."""
+    takes the plain copy, as small and larger images do, images for the host, and other dtypes, which must reach the
+    resize's own check as they are."""
     import contextlib
 
     from foidfinder_amd.backends.rocm.preprocess import _Uploads
@@ -345,15 +345,18 @@ def test_uploads_that_keep_clear_of_the_staging_buffers(monkeypatch):
         def to(self, device):
             return "plain"
 
-    cuda = torch.device("cuda", 0)
-    up.put(Image(100), cuda)
-    assert staged == [100]
+    cuda, n = torch.device("cuda", 0), up.LEAST + 1
+    up.put(Image(n), cuda)
+    up.put(Image(up.LIMIT), cuda)
+    assert staged == [n, up.LIMIT]
     capturing[0] = True
-    assert up.put(Image(100), cuda) == "plain"
+    assert up.put(Image(n), cuda) == "plain"
     capturing[0] = False
-    assert up.put(Image(0), cuda) == up.put(Image(up.LIMIT + 1), cuda) == up.put(Image(5), torch.device("cpu")) == "plain"
-    assert up.put(Image(100, torch.float32), cuda) == up.put(Image(100, torch.int16), cuda) == "plain"
-    assert staged == [100]
+    for m in (0, 1, up.LEAST, up.LIMIT + 1):
+        assert up.put(Image(m), cuda) == "plain"
+    assert up.put(Image(n), torch.device("cpu")) == "plain"
+    assert up.put(Image(n, torch.float32), cuda) == up.put(Image(n, torch.int16), cuda) == "plain"
+    assert len(staged) == 2
 
 
 def test_bicubic_taps_match_the_pillow_known_answers():

@@ -236,7 +236,7 @@ def test_gpu_bicubic_taps_are_the_host_taps(dev, width, height):
 
 def test_uploads_from_threads_and_streams(dev):
     """The letterbox's pinned uploads: six threads on streams of their own, more than the buffers kept, sizes that grow a
-    buffer and one past its limit, the host array overwritten right after each call; every copy is the array it was given,
+    buffer, some that pass the buffers by and one past their limit, the host array overwritten right after each call; every copy is the array it was given,
     and no more than BUFFERS buffers stay."""
     import threading
 
@@ -248,7 +248,7 @@ def test_uploads_from_threads_and_streams(dev):
         r = np.random.default_rng(seed)
         stream = torch.cuda.Stream()
         with torch.cuda.stream(stream):
-            for n in [1, 1000, 300_000, 7, 5_000_000, 64, up.LIMIT + 3 if seed == 0 else 4096]:
+            for n in [1, 700_000, 1_300_000, 4096, 5_000_000, up.LEAST + 1, up.LIMIT + 3 if seed == 0 else up.LEAST]:
                 a = r.integers(0, 256, n, dtype=np.uint8)
                 want = a.copy()
                 t = up.put(torch.from_numpy(a), dev)
@@ -269,7 +269,7 @@ def test_letterbox_across_inference_mode_and_default_device(dev):
     changes nothing."""
     from foidfinder_amd.backends.rocm.preprocess import _uploads, letterbox_gpu
 
-    image = np.random.default_rng(3).integers(0, 256, (60, 90, 3), dtype=np.uint8)
+    image = np.random.default_rng(3).integers(0, 256, (600, 900, 3), dtype=np.uint8)
 
     def run():
         out = torch.empty(56, 56, 3, dtype=torch.uint8, device=dev)
