@@ -564,10 +564,11 @@ extern "C" int ff_pool_sum(const void* a_t, const void* xn, int64_t B, int64_t N
                            void* pooled, void* stream) {
   clear_error();
   FF_POOL_CHECK("pool_sum", B, 1, D);
-  if (N <= 0 || N > (int64_t(1) << 30) / D) return fail(FF_EINVAL, "pool_sum: need 0 < N * D <= 2^30");
+  // a batch's tokens and weights span less than 2^31 bytes: their lengths are signed 32-bit numbers in the kernel
+  if (N <= 0 || N >= ((int64_t(1) << 30) + D - 1) / D) return fail(FF_EINVAL, "pool_sum: need 0 < N * D < 2^30");
   if (GM <= 0 || GM > 512) return fail(FF_EINVAL, "pool_sum: need 0 < GM <= 512");
-  if (GM * ldt > (int64_t(1) << 30)) return fail(FF_EINVAL, "pool_sum: GM * ldt above 2^30 is not supported");
   if (ldt != (N + 7) / 8 * 8) return fail(FF_EINVAL, "pool_sum: ldt must be N rounded up to a multiple of 8");
+  if (GM * ldt >= (int64_t(1) << 30)) return fail(FF_EINVAL, "pool_sum: need GM * ldt < 2^30");
   if (B == 0) return FF_OK;
   if (!a_t || !xn || !pooled) return fail(FF_EINVAL, "pool_sum: null pointer");
   if (!al(a_t, 16) || !al(xn, 16) || !al(pooled, 8)) return fail(FF_EINVAL, "pool_sum: misaligned pointer");
@@ -590,12 +591,12 @@ extern "C" int ff_pool_values(const void* pooled, const void* wv, const float* b
   clear_error();
   FF_POOL_CHECK("pool_values", B, G, D);
   if (M <= 0 || M > 64 || nblk <= 0 || nblk > (1 << 24)) return fail(FF_EINVAL, "pool_values: bad M or nblk");
+  const int64_t rows = (B * M + 15) / 16;
+  if (rows > 65535) return fail(FF_EINVAL, "pool_values: B*M too large");
   if (B == 0) return FF_OK;
   if (!pooled || !wv || !bv || !partial || !z) return fail(FF_EINVAL, "pool_values: null pointer");
   if (!al(pooled, 16) || !al(wv, 16) || !al(z, 8)) return fail(FF_EINVAL, "pool_values: misaligned pointer");
   const int hd = static_cast<int>(D / G);
-  const int64_t rows = (B * M + 15) / 16;
-  if (rows > 65535) return fail(FF_EINVAL, "pool_values: B*M too large");
   const dim3 grid(static_cast<unsigned>(hd / 16), static_cast<unsigned>(rows), static_cast<unsigned>(G));
   pool_values_kernel<<<grid, 256, 0, as_stream(stream)>>>(
       static_cast<const half_t*>(pooled), static_cast<const half_t*>(wv), bv, partial, static_cast<int>(nblk),
@@ -634,11 +635,11 @@ extern "C" int ff_pool_keys(const void* qleaf, const void* kT, int64_t B, int64_
   clear_error();
   FF_POOL_CHECK("pool_keys", B, G, D);
   if (Q <= 0 || Q > 65535) return fail(FF_EINVAL, "pool_keys: bad Q");
+  const int64_t rows = (B * Q + 15) / 16;
+  if (rows > 65535) return fail(FF_EINVAL, "pool_keys: B*Q too large");
   if (B == 0) return FF_OK;
   if (!qleaf || !kT || !u) return fail(FF_EINVAL, "pool_keys: null pointer");
   if (!al(qleaf, 8) || !al(kT, 8) || !al(u, 8)) return fail(FF_EINVAL, "pool_keys: misaligned pointer");
-  const int64_t rows = (B * Q + 15) / 16;
-  if (rows > 65535) return fail(FF_EINVAL, "pool_keys: B*Q too large");
   const dim3 grid(static_cast<unsigned>((D + 255) / 256), static_cast<unsigned>(rows), static_cast<unsigned>(G));
   pool_keys_kernel<<<grid, 256, 0, as_stream(stream)>>>(static_cast<const half_t*>(qleaf), static_cast<const half_t*>(kT),
                                                         static_cast<int>(B), static_cast<int>(Q), static_cast<int>(G),

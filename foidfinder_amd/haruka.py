@@ -31,7 +31,8 @@ import torch
 import torch.nn.functional as F
 
 from .engine import Int8Engine, eva02_rope_tables, rotate_quantize
-from .kernels import EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, pad_norm, pad_patch_weight, pool_weights_blocks, slot_weights_blocks
+from .kernels import (EPI_QKV_ROPE, EPI_RESIDUAL, EPI_SWIGLU, head_fits, kernels, pad_norm, pad_patch_weight, pool_fits,
+                      pool_weights_blocks, slot_weights_blocks)
 
 ARCHITECTURE = "haruka-eva02-tree"  # foidfinder/haruka.py:14
 QUANTIZED = ("qkv", "proj", "fc1", "fc2")  # the backbone linears that run as W8A8
@@ -322,9 +323,8 @@ class HarukaInt8(Int8Engine):
         cfg, k = self.cfg, self.k
         xn = torch.empty_like(x)
         k.layer_norm2(x, *self.norm, *self.pool["norm"], cfg.eps, xn)
-        # the pool's kernels address a batch's tokens and weights by 32-bit byte offsets
-        fits = x.shape[1] * max(cfg.dim, cfg.pool_heads * cfg.leaves) < 1 << 30
-        leaf = self._pool_leaves(xn) if self.fused_pool and fits else self._pool_leaves_library(xn)
+        fused = self.fused_pool and pool_fits(x.size(0), x.size(1), cfg.pool_heads, cfg.leaves, cfg.dim)
+        leaf = self._pool_leaves(xn) if fused else self._pool_leaves_library(xn)
         w, b = self.head
         if head_fits(leaf.size(0), w):
             out = torch.empty(leaf.size(0), cfg.tags, device=x.device, dtype=torch.float32)
@@ -364,8 +364,8 @@ class HarukaInt8(Int8Engine):
         return leaf
 
     def _pool_leaves_library(self, xn: torch.Tensor) -> torch.Tensor:
-        """_pool_leaves on library products, for heads or leaves that are not whole 16-column tiles (or batches past the
-        kernels' 32-bit offsets, which transpose the kernels' weights here)."""
+        """_pool_leaves on library products, for heads or leaves that are not whole 16-column tiles, and for pool_head calls
+        on more images or tokens than the kernels take (pool_fits), which transpose the kernels' weights here."""
         cfg, k = self.cfg, self.k
         B, N, d = xn.shape
         Hp, C, Q = cfg.pool_heads, cfg.coarse, cfg.leaves

@@ -285,6 +285,14 @@ def pool_weights_blocks(N: int) -> int:
     return lib().ff_pool_weights_blocks(N)
 
 
+def pool_fits(B: int, N: int, heads: int, leaves: int, dim: int) -> bool:
+    """Whether the tree pool's kernels take B images of N tokens (others go to the library's products): 32-bit byte
+    offsets within an image's tokens and weights (rows padded to 8 tokens), and at most 65535 launch rows of images and of
+    16 (image, leaf) pairs each."""
+    ldt = (N + 7) // 8 * 8
+    return N * dim < 1 << 30 and heads * leaves * ldt < 1 << 30 and B <= 65535 and B * leaves <= 16 * 65535
+
+
 def _half(shape: tuple, *ts: torch.Tensor) -> None:
     for t in ts:
         if t.dtype != torch.float16 or tuple(t.shape) != shape:

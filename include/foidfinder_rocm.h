@@ -126,7 +126,7 @@ int ff_pool_weights(const void* xn, const void* u, int64_t u_stride, const float
                     const float* bias, int64_t B, int64_t N, int64_t G, int64_t M, int64_t D, int64_t ldt, void* a_t,
                     float* partial, void* stream);
 /* pooled fp16 [B, GM, D]: pooled[b, j] = sum_n a_t[b, j, n] xn[b, n]; a_t as ff_pool_weights leaves it, ldt = N
- * rounded up to a multiple of 8, GM <= 512. */
+ * rounded up to a multiple of 8, GM <= 512, N*D < 2^30, GM*ldt < 2^30. */
 int ff_pool_sum(const void* a_t, const void* xn, int64_t B, int64_t N, int64_t GM, int64_t D, int64_t ldt, void* pooled,
                 void* stream);
 /* z[b, m, h*hd + e] = pooled[b, h*M + m] . wv[h*hd + e] + bv[h*hd + e] * sum_k partial[b, k, h*M + m]; pooled
