@@ -168,13 +168,21 @@ def test_pool_head_matches_library_chain(dev, monkeypatch, batch, pool_heads, le
     # the library chain rounds its logits, products and masses to fp16 at a dozen points: 4e-3 of the result's size
     rel = ((got - want).double().norm() / want.double().norm()).item()
     assert rel < 4e-3, f"fused and library pools differ by {rel:.2e}"
+    monkeypatch.undo()
+    monkeypatch.setattr("foidfinder_amd.haruka.pool_fits", lambda *sizes: False)  # more images or tokens than the kernels take
+    assert torch.equal(eng.pool_head(x), want)
 
 
-@pytest.mark.parametrize(("B", "grid", "N"), [(1, 1, 128), (2, 9, 128), (3, 8, 768), (1, 17, 384), (40, 8, 1024)])
-def test_patch_embed(dev, B, grid, N):
-    """One patch, patch counts that end inside a workgroup's 64, both column splits (the last is past 1024 workgroups of
-    64 columns), and raw pixel values: the class row is copied, the others are float64's within one fp16 rounding (fp32
-    sums of 588 products)."""
+@pytest.mark.parametrize(("B", "grid", "N", "cols"),
+                         [(1, 1, 128, 64), (2, 9, 128, 64), (3, 8, 768, 64), (1, 17, 384, 64), (40, 8, 1024, 64),
+                          (45, 9, 768, 256), (90, 9, 384, 128), (100, 8, 1024, 512), (12, 33, 768, 256)])
+def test_patch_embed(dev, B, grid, N, cols):
+    """One patch, patch counts that end inside a workgroup's 64, raw pixel values, and each split of the columns: 64 a
+    workgroup up to 1024 such workgroups (the fifth case has 640), past that 128, 256 or 512 in turns of 128, with a
+    partial last patch block (81 and 1089 patches). The class row is copied, the others are float64's within one fp16
+    rounding (fp32 sums of 588 products)."""
+    workgroups = -(-grid * grid // 64) * B * (N // 64)
+    assert cols == (64 if workgroups <= 1024 else next(c for c in (512, 256, 128) if N % c == 0))
     S = 14 * grid
     img = (torch.rand(B, S, S, 3, device=dev, generator=torch.Generator(device=dev).manual_seed(B)) * 255).round().half()
     w, bias = randn(dev, N, 588, std=1e-3, seed=1).half(), randn(dev, grid * grid, N, seed=2).half()
