@@ -173,9 +173,24 @@ __global__ __launch_bounds__(64 * (pw_waves<GMAX, NT>())) void pool_weights_kern
 // columns 16.0 and 21.3.
 constexpr int PS_J = 96, PS_N = 64, PS_SLOTS = 4;
 
-template <int OFF>
-__device__ __forceinline__ void tr_read(half4_t& v, uint32_t lds_addr) {
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "n"(OFF) : "memory");
+// The eight transposing reads of a chunk's 64 tokens, four columns' 16 tokens in x[tt][0] (tokens 0-3 of each lane half's 8)
+// and x[tt][1] (4-7), and the wait for them. One block: the results are the compiler's only once they have arrived, and
+// (as inline asm) its wait-insertion pass does not drain the buffer->LDS loads in flight before them.
+__device__ __forceinline__ void tr_read_chunk(half4_t (&x)[4][2], uint32_t lds_addr) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:512\n\t"
+      "ds_read_b64_tr_b16 %2, %8 offset:2048\n\t"
+      "ds_read_b64_tr_b16 %3, %8 offset:2560\n\t"
+      "ds_read_b64_tr_b16 %4, %8 offset:4096\n\t"
+      "ds_read_b64_tr_b16 %5, %8 offset:4608\n\t"
+      "ds_read_b64_tr_b16 %6, %8 offset:6144\n\t"
+      "ds_read_b64_tr_b16 %7, %8 offset:6656\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[2][0]), "=&v"(x[2][1]), "=&v"(x[3][0]),
+        "=&v"(x[3][1])
+      : "v"(lds_addr)
+      : "memory");
 }
 
 template <int SUB>
@@ -233,11 +248,6 @@ __global__ __launch_bounds__(128 * SUB) void pool_sum_kernel(const half_t* __res
     if (k + PS_SLOTS - 1 < chunks) issue(k + PS_SLOTS - 1);
     const uint8_t* sl = lds + k % PS_SLOTS * SLOT;
     const uint32_t xa = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void*)sl)) + xoff;
-    half4_t x[4][2];
-    tr_read<0 * 128>(x[0][0], xa), tr_read<4 * 128>(x[0][1], xa);
-    tr_read<16 * 128>(x[1][0], xa), tr_read<20 * 128>(x[1][1], xa);
-    tr_read<32 * 128>(x[2][0], xa), tr_read<36 * 128>(x[2][1], xa);
-    tr_read<48 * 128>(x[3][0], xa), tr_read<52 * 128>(x[3][1], xa);
     half8_t w[4][3];
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt)
@@ -246,9 +256,8 @@ __global__ __launch_bounds__(128 * SUB) void pool_sum_kernel(const half_t* __res
         const int r = 32 * i + fr;
         w[tt][i] = *reinterpret_cast<const half8_t*>(sl + SUB * XB + r * 128 + (((2 * tt + fh) ^ ((r >> 1) & 7)) << 4));
       }
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[2][0]), "+v"(x[2][1]),
-                   "+v"(x[3][0]), "+v"(x[3][1])::"memory");
+    half4_t x[4][2];
+    tr_read_chunk(x, xa);
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
       const half4_t lo = x[tt][0], hi = x[tt][1];
