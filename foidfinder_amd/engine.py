@@ -442,7 +442,7 @@ class Eva02Int8(Int8Engine):
             self._gemm(buf["h8"], lw["fc2"], rs, EPI_RESIDUAL, v["fc2"], x)
             if trace is not None:
                 trace[f"x{i}"] = x.clone()
-        if head_fits(B, self.head_w):
+        if head_fits(xv[:, 0], self.head_w):
             out = torch.empty(B, self.head_w.size(0), device=x.device, dtype=torch.float32)
             k.head(xv[:, 0], self.head_w, self.head_b, out, *self.norm, eps)
             return out

@@ -326,7 +326,7 @@ class HarukaInt8(Int8Engine):
         fused = self.fused_pool and pool_fits(x.size(0), x.size(1), cfg.pool_heads, cfg.leaves, cfg.dim)
         leaf = self._pool_leaves(xn) if fused else self._pool_leaves_library(xn)
         w, b = self.head
-        if head_fits(leaf.size(0), w):
+        if head_fits(leaf, w):
             out = torch.empty(leaf.size(0), cfg.tags, device=x.device, dtype=torch.float32)
             k.head(leaf, w, b, out)
             return out

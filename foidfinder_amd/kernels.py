@@ -427,9 +427,19 @@ def patch_embed(img: torch.Tensor, w: torch.Tensor, bias_pos: torch.Tensor, cls:
     _run("ff_patch_embed", dev, _ptr(img), _ptr(w), _ptr(bias_pos), _ptr(cls), B, grid, N, _ptr(x))
 
 
-def head_fits(rows: int, W: torch.Tensor) -> bool:
-    """Whether `head` takes this many rows of x with W [N, K] (others go to the library's GEMM)."""
-    return rows <= 64 and W.size(1) % 32 == 0 and W.size(1) <= 1280
+def head_fits(x: torch.Tensor, W: torch.Tensor) -> bool:
+    """Whether `head` takes the rows x with W [N, K] (others go to the library's GEMM): up to 64 rows, and fp16, which a
+    library product under autocast need not have left."""
+    return x.size(0) <= 64 and x.dtype == torch.float16 and W.size(1) % 32 == 0 and W.size(1) <= 1280
+
+
+def unfollowed(x: torch.Tensor) -> bool:
+    """Whether x is a plain GPU tensor that nothing follows, so that an op here can take the place of a torch product: these
+    ops go by addresses, past autograd (backward and forward), functorch's transforms, tracing and dispatch modes."""
+    return (type(x) is torch.Tensor and x.is_cuda and not (x.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad._current_level < 0 and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0)
 
 
 def head(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, out: torch.Tensor, gamma: torch.Tensor | None = None,

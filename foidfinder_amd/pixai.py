@@ -19,7 +19,7 @@ import torch
 import torch.nn.functional as F
 
 from .engine import Int8Engine, rotate_quantize
-from .kernels import EPI_GELU_F16, EPI_QKV_ROPE, EPI_RESIDUAL, head_fits, kernels
+from .kernels import EPI_GELU_F16, EPI_QKV_ROPE, EPI_RESIDUAL, head_fits, kernels, unfollowed
 
 FORMAT = "foidfinder-pixai-int8-v1"  # the reference's converted-checkpoint format name (engine.py:46)
 # Quantized block linears -> Hadamard block size of their input rotation (engine.py:45).
@@ -273,7 +273,7 @@ class PixAIInt8(Int8Engine):
         o = (p.unsqueeze(-1) * kv[1]).sum(2).reshape(B, d).half()  # [B, H, 64] -> [B, d]
         o = F.linear(o, *self.pool_proj)
         w, b = self.head
-        if head_fits(B, w):
+        if head_fits(o, w) and unfollowed(o):
             out = torch.empty(B, w.size(0), device=x.device, dtype=torch.float32)
             self.k.head(o, w, b, out)
             return out

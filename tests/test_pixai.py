@@ -204,3 +204,40 @@ def test_write_int8_dir_format(tmp_path):
             assert np.array_equal(f.get_tensor(k), want[k]), k
     with pytest.raises(RuntimeError, match="already in the int8 format"):
         write_int8_dir(out, tmp_path / "again", device="cpu")
+
+
+def test_pool_head_runs_where_torch_products_do():
+    """The pool head is torch products but for the tags' product: it takes tokens on the CPU, and autograd, forward-mode
+    derivatives and vmap go through it."""
+    from foidfinder_amd.pixai import PixAIInt8, convert_checkpoint, synthetic_checkpoint
+
+    cfg, ocfg = small_cfgs()
+    state = convert_checkpoint(synthetic_checkpoint(cfg, seed=0), cfg)
+    eng = PixAIInt8(state, cfg, device="cpu")
+    x = torch.randn(2, cfg.tokens, cfg.dim, generator=torch.Generator().manual_seed(1)).half()
+    got = eng.pool_head(x)
+    want = OP.pool_head(x.numpy().reshape(-1, cfg.dim), {k: v.numpy() for k, v in state.items()}, ocfg)
+    assert got.dtype == torch.float32 and np.abs(got.numpy() - want).max() < 1e-2
+    g, grad = check_followed_pool_head(eng, x)
+    t = torch.randn(x.shape, generator=torch.Generator().manual_seed(3)).to(x)
+    value, tangent = torch.func.jvp(eng.pool_head, (x,), (t,))
+    assert (value - got).norm() <= 2e-2 * got.norm()
+    back, fwd = (grad.double() * t.double()).sum(), (tangent.double() * g.double()).sum()
+    scale = tangent.double().norm() * g.double().norm()
+    assert scale > 0 and (back - fwd).abs() <= 2e-2 * scale
+
+
+def check_followed_pool_head(eng, x):
+    """Gradient and vmap of eng.pool_head at x agree with its plain result (fp16 products: 2e-2 of its size); returns the
+    outputs' gradient and the tokens'."""
+    plain = eng.pool_head(x).double()
+    leaf = x.clone().requires_grad_()
+    out = eng.pool_head(leaf)
+    assert out.requires_grad
+    g = torch.randn(out.shape, generator=torch.Generator().manual_seed(2)).to(out)
+    (out * g).sum().backward()
+    each = torch.func.vmap(lambda a: eng.pool_head(a[None])[0])(x)
+    for v in (out.detach(), each):
+        assert (v.double() - plain).norm() <= 2e-2 * plain.norm()
+    assert torch.isfinite(leaf.grad).all() and leaf.grad.abs().max() > 0
+    return g, leaf.grad

@@ -213,3 +213,32 @@ def test_preprocess_constant_and_transparent_images(dev):
     assert (out[1] == 1.0).all()
     comp = np.asarray(Image.alpha_composite(Image.new("RGBA", (40, 40), (255,) * 4), Image.fromarray(half, "RGBA")))
     assert np.abs(out[2] - np.float16(comp[0, 0, 0] / 255 * 2 - 1)).max() <= 1e-3
+
+
+def test_pool_head_followed_by_autograd_transforms_and_autocast(dev, monkeypatch):
+    """Tokens that autograd, vmap or a dispatch mode follows, and a bf16 autocast, take the library's tag product, which
+    they can follow; plain tokens take the kernel, under a no_grad too. (Forward-mode derivatives: torch's own LayerNorm
+    has none in fp16 on the GPU.)"""
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from foidfinder_amd.pixai import PixAIInt8
+    from test_pixai import check_followed_pool_head
+
+    cfg, _ = cfgs()
+    eng = PixAIInt8(model(cfg)[1], cfg, device=dev)
+    x = torch.randn(2, cfg.tokens, cfg.dim, generator=torch.Generator().manual_seed(1)).half().to(dev)
+    plain = eng.pool_head(x)
+    check_followed_pool_head(eng, x)
+    with torch.autocast("cuda", torch.bfloat16):
+        cast = eng.pool_head(x)
+    with FlopCounterMode(display=False) as flops:
+        counted = eng.pool_head(x)
+    assert flops.get_total_flops() > 2 * 2 * cfg.dim * (2 * cfg.tokens * cfg.dim + cfg.dim + cfg.tags) - 1
+    for v, rel in ((cast, 4e-2), (counted, 2e-2)):
+        assert (v - plain).norm() <= rel * plain.norm()
+    calls = []
+    monkeypatch.setattr(eng, "k", type("Ops", (), {"head": staticmethod(lambda *a: calls.append(a))}))
+    with torch.no_grad():
+        eng.pool_head(x.clone().requires_grad_())
+    eng.pool_head(x)
+    assert len(calls) == 2
