@@ -9,9 +9,10 @@ EVA02 SwiGLU MLP of foidfinder/backends/mlx/haruka.py:196-209):
   LN2 -> H1024 rotation -> int8                    -> fc1 GEMM + bias + SwiGLU -> fp16 [T, 2816]
   mlp LayerNorm -> block-H128 rotation -> int8     -> fc2 GEMM + bias + residual
 
-Weights carry the same rotations (W' = W H) and are quantized per output channel. Stem (patch GEMM) and head
-(final LayerNorm, tag GEMM) run in fp16 through PyTorch (hipBLASLt), as the reference's stem and head run through
-cuBLAS.
+Weights carry the same rotations (W' = W H) and are quantized per output channel. Stem (patch product, position and
+class row: ff_patch_embed) and head (final LayerNorm and tag product: ff_head) run on fp16 weights in one launch each;
+patch sizes other than 14 and the tags of more than 64 images run through PyTorch (hipBLASLt), as the reference's stem
+and head run through cuBLAS.
 """
 
 from __future__ import annotations

@@ -14,8 +14,9 @@ Input checkpoints are the reference's folded Haruka format (foidfinder/haruka.py
 in the patch embedding, 1/sqrt(head_dim) in the q rows and the pool's key rows, QKV and SwiGLU as single matrices)
 or its compressed download format (foidfinder/haruka_quant.py: per-row step x integer codes in gzipped zigzag byte
 planes). The folded q rows already carry the softmax scale, so the QKV epilogue multiplies q by log2(e) only.
-Stem (patch GEMM on raw 0..255 pixels) and the tree-pool head run in fp16 through PyTorch, as the reference runs
-them through MLX.
+Stem (raw 0..255 pixels, ff_patch_embed), tree pool (ff_layer_norm2, ff_pool_*) and tag product (ff_head) run on fp16
+weights in kernels of their own; shapes that those do not take, and the tags of more than 64 images, run on library
+products through PyTorch. The reference runs both through MLX.
 """
 
 from __future__ import annotations
@@ -333,7 +334,7 @@ class HarukaInt8(Int8Engine):
         return F.linear(leaf, w, b).float()
 
     def _pool_leaves(self, xn: torch.Tensor) -> torch.Tensor:
-        """Normed tokens [B, N, d] -> leaf features [B, Q * leaf_dim] fp16, on the pool's own kernels: twelve launches
+        """Normed tokens [B, N, d] -> leaf features [B, Q * leaf_dim] fp16, on the pool's own kernels: ten launches
         a call, where the library products with their element-wise steps take some forty."""
         cfg, k = self.cfg, self.k
         B, N, d = xn.shape
